@@ -29,7 +29,7 @@ HIPCC_FLAGS = [
 
 # Per-file additions.  The attention kernels take finite inputs (as the reference's): without
 # NaN semantics the compiler drops the canonicalising moves of every row-max step.
-FILE_FLAGS = {"attn_fwd.hip": ["-fno-honor-nans"]}
+FILE_FLAGS = {f: ["-fno-honor-nans"] for f in ("attn_fwd.hip", "attn_split.hip")}
 
 
 def hipcc() -> str:

@@ -5,6 +5,7 @@
 #include <mutex>
 
 #include "attn_kernels.h"
+#include "attn_split.h"
 
 namespace fa4cp {
 namespace {
@@ -240,8 +241,10 @@ extern "C" int fa4cp_attn_fwd(const fa4cp_attn_args* a, void* stream) {
 }
 
 
-// fa4cp_ring_sweep_fwd (kp == NULL) and fa4cp_ring_sweep_fwd_paged.
-static int ring_sweep_launch(const fa4cp_sweep_args* a, const fa4cp_sweep_kpages* kp, void* stream) {
+// fa4cp_ring_sweep_fwd (kp == NULL) and fa4cp_ring_sweep_fwd_paged; with a workspace the split
+// form where split_plan chooses it.
+static int ring_sweep_launch(const fa4cp_sweep_args* a, const fa4cp_sweep_kpages* kp, void* ws, int64_t ws_bytes,
+                             void* stream) {
   clear_error();
   if (a == nullptr) return set_error(FA4CP_EINVAL, "ring_sweep_fwd: null args");
   const bool empty = a->total == 0;  // no rows: every pointer may be NULL
@@ -325,6 +328,16 @@ static int ring_sweep_launch(const fa4cp_sweep_args* a, const fa4cp_sweep_kpages
   if (blocks == 0 || empty) return FA4CP_OK;
   if (blocks > 0x7fffffffLL) return set_error(FA4CP_EINVAL, "ring_sweep_fwd: grid too large");
   p.n_blocks = (int)blocks;
+  if (ws != nullptr) {
+    const SplitPlan pl = split_plan(a);
+    if (pl.split()) {
+      const int64_t need = split_bytes(pl, p.n_hg, d);
+      if (ws_bytes < need || ((uintptr_t)ws % 16) != 0)
+        return set_error(FA4CP_EINVAL, "ring_sweep_fwd_ws: workspace of %lld bytes at %p; %lld bytes, 16-byte aligned, "
+                         "needed", (long long)ws_bytes, ws, (long long)need);
+      return launch_split(p, pl, ws, a->dtype, d, hp, paged, (hipStream_t)stream);
+    }
+  }
   void (*fn)(SweepParams) = nullptr;
   const bool pack = nseq > 1;  // several sequences: the gap-free row tile order
 #define FA4CP_PICK_PK(KERNEL, H, ...)                                                       \
@@ -368,7 +381,7 @@ static int ring_sweep_launch(const fa4cp_sweep_args* a, const fa4cp_sweep_kpages
 }
 
 extern "C" int fa4cp_ring_sweep_fwd(const fa4cp_sweep_args* a, void* stream) {
-  return ring_sweep_launch(a, nullptr, stream);
+  return ring_sweep_launch(a, nullptr, nullptr, 0, stream);
 }
 
 extern "C" int fa4cp_ring_sweep_fwd_paged(const fa4cp_sweep_args* a, const fa4cp_sweep_kpages* kp, void* stream) {
@@ -376,5 +389,10 @@ extern "C" int fa4cp_ring_sweep_fwd_paged(const fa4cp_sweep_args* a, const fa4cp
     clear_error();
     return set_error(FA4CP_EINVAL, "ring_sweep_fwd_paged: null k_pages");
   }
-  return ring_sweep_launch(a, kp, stream);
+  return ring_sweep_launch(a, kp, nullptr, 0, stream);
+}
+
+extern "C" int fa4cp_ring_sweep_fwd_ws(const fa4cp_sweep_args* a, const fa4cp_sweep_kpages* kp, void* workspace,
+                                       int64_t workspace_bytes, void* stream) {
+  return ring_sweep_launch(a, kp, workspace, workspace_bytes, stream);
 }

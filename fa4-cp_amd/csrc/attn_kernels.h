@@ -303,31 +303,13 @@ __device__ __forceinline__ void decode_block(const Params& p, int& hg, int& seq,
   decode_block_at(p, (int)blockIdx.x, hg, seq, rt);
 }
 
-// decode_block for the sweep kernels over packed sequences: the grid counts n_rt row tiles for
-// every sequence (the longest one's), so most of a short sequence's workgroups have no rows.
-// Here the row tiles of a head group are numbered across the sequences without those gaps
-// (sequence j has ceil(L_j / rows) of them, still longest first within a sequence), and the
-// workgroups past the last real tile, all empty, come last in each XCD's dispatch order
-// instead of ahead of every sequence's tiles.  Returns false for those.  The sequences'
-// tile counts are summed 64 at a time across the wavefront's lanes.  The sweep kernels take
-// it as a template variant (PACK) used for more than one sequence only: with one sequence
-// there are no gaps, and the headline kernel built with the plain decode ran 0.2 % faster
-// (code placement), while C4 (8 sequences) gains 0.8 % from the packed order.
+// Row tile r of the packed sequences' real row tiles (sequence j has ceil(L_j / rows) of them,
+// longest first within a sequence): its sequence, index, rows and V^T start.  Returns false
+// past the last one.  The sequences' tile counts are summed 64 at a time across the wavefront's
+// lanes.
 template <typename Params>
-__device__ __forceinline__ bool decode_sweep_block(const Params& p, int rows, int& hg, int& seq, int& rt,
-                                                   int& qs, int& len, int64_t& vt_pos) {
-  const int per_hg = p.nseq * p.n_rt;
-  const int k = p.n_hg < 8 ? 8 / p.n_hg : 1;
-  int r;
-  if (k > 1 && p.n_hg * k == 8 && p.n_blocks % 8 == 0 && per_hg % k == 0) {
-    const int x = (int)blockIdx.x & 7;
-    hg = x / k;
-    r = x % k + k * (int)(blockIdx.x >> 3);
-  } else {
-    const int b = xcd_remap((int)blockIdx.x, p.n_blocks);
-    hg = b / per_hg;
-    r = b - hg * per_hg;
-  }
+__device__ __forceinline__ bool packed_row_tile(const Params& p, int rows, int r, int& seq, int& rt, int& qs, int& len,
+                                                int64_t& vt_pos) {
   const int lane = (int)(threadIdx.x & 63);
   int base = 0;       // real row tiles of the sequences before j0
   int64_t vbase = 0;  // their V^T columns (lengths padded to kVtPad, as vt_seq_start sums them)
@@ -366,6 +348,33 @@ __device__ __forceinline__ bool decode_sweep_block(const Params& p, int rows, in
     vbase += __builtin_amdgcn_readlane(vincl, 63);
   }
   return false;
+}
+
+// decode_block for the sweep kernels over packed sequences: the grid counts n_rt row tiles for
+// every sequence (the longest one's), so most of a short sequence's workgroups have no rows.
+// Here the row tiles of a head group are numbered across the sequences without those gaps
+// (sequence j has ceil(L_j / rows) of them, still longest first within a sequence), and the
+// workgroups past the last real tile, all empty, come last in each XCD's dispatch order
+// instead of ahead of every sequence's tiles.  Returns false for those.  The sweep kernels take
+// it as a template variant (PACK) used for more than one sequence only: with one sequence
+// there are no gaps, and the headline kernel built with the plain decode ran 0.2 % faster
+// (code placement), while C4 (8 sequences) gains 0.8 % from the packed order.
+template <typename Params>
+__device__ __forceinline__ bool decode_sweep_block(const Params& p, int rows, int& hg, int& seq, int& rt,
+                                                   int& qs, int& len, int64_t& vt_pos) {
+  const int per_hg = p.nseq * p.n_rt;
+  const int k = p.n_hg < 8 ? 8 / p.n_hg : 1;
+  int r;
+  if (k > 1 && p.n_hg * k == 8 && p.n_blocks % 8 == 0 && per_hg % k == 0) {
+    const int x = (int)blockIdx.x & 7;
+    hg = x / k;
+    r = x % k + k * (int)(blockIdx.x >> 3);
+  } else {
+    const int b = xcd_remap((int)blockIdx.x, p.n_blocks);
+    hg = b / per_hg;
+    r = b - hg * per_hg;
+  }
+  return packed_row_tile(p, rows, r, seq, rt, qs, len, vt_pos);
 }
 
 // Dynamic hand-out of the row tiles.  The hardware sends workgroup i to XCD i % 8, so a fixed
@@ -1064,9 +1073,10 @@ constexpr int kWaitLgkm = 0xC07F;
 // The load cursors' walk over a Geo's segment list in tiles of BN keys: K tiles are BN rows
 // of k_rsb bytes, V^T tiles BN positions of esz bytes further on.  Geo provides nseg(),
 // seg(s) -> StepSeg and base(src, is_k) -> the byte address of the segment's first K row
-// (this kv head) or V^T position (this kv head and sequence).  Each step is an increment, a
-// pointer bump and one compare against the cursor's next event tile; everything else (the
-// next segment, the partial last tile, a page) happens at events.  The phases of the
+// (this kv head) or V^T position (this kv head and sequence), n_tiles(), and first(), the tile
+// of segment 0 at which the walk starts (0 unless the list is a share of one, kSplit).  Each
+// step is an increment, a pointer bump and one compare against the cursor's next event tile;
+// everything else (the next segment, the partial last tile, a page) happens at events.  The phases of the
 // pipelines are issue-bound, so the walk keeps its per-tile instructions to that minimum.
 //
 // Paged K (Geo::kPagedK): base(src, true) is then page 0 of source src's cache (this kv
@@ -1103,7 +1113,8 @@ struct TileWalk {
     return pidx < pt_n ? sload_i32(c.prow + pidx) : -1;
   }
   // A paged K cursor at the first tile of page pidx: its address from the page's entry;
-  // returns whether the entry names a page of the cache.
+  // returns whether the entry names a page of the cache.  (enter and start may begin inside a
+  // page: they add the tiles of it that come before the cursor's.)
   __device__ __forceinline__ bool kpage_at(LoadCursor& c, int entry) const {
     c.ptr = c.pbase + (int64_t)(uint32_t)entry * page_bytes;
     c.pnext = c.prow + min(c.pidx + 1, pt_n - 1);
@@ -1135,10 +1146,12 @@ struct TileWalk {
       if (isk) {
         c.pbase = c.ptr;
         c.prow = geo.kpt_row(g.src);
-        c.pidx = 0;
-        live = kpage_at(c, kentry(c, 0));
+        c.pidx = Geo::kSplit ? c.t / tpp : 0;
+        live = kpage_at(c, kentry(c, c.pidx));
       }
     }
+    if constexpr (Geo::kSplit) c.ptr += (int64_t)(isk ? c.t - (Geo::kPagedK ? c.pidx * tpp : 0) : c.t) *
+                                        (isk ? BN * k_rsb : v_step);
     settle(c, isk, live);
   }
   __device__ __forceinline__ void fix(LoadCursor& c, bool isk) const {
@@ -1169,6 +1182,7 @@ struct TileWalk {
   }
   __device__ __forceinline__ LoadCursor start(bool isk) const {
     LoadCursor c{};
+    c.t = geo.first();
     if constexpr (Geo::kPagedK) {
       enter(c, geo.seg(0), isk);
       fix(c, isk);
@@ -1177,6 +1191,7 @@ struct TileWalk {
       c.tiles = g.tiles;
       c.keys = g.keys;
       c.ptr = geo.base(g.src, isk);
+      if constexpr (Geo::kSplit) c.ptr += (int64_t)c.t * (isk ? BN * k_rsb : v_step);
       fix_flat(c, isk);
     }
     return c;
@@ -1283,8 +1298,7 @@ __device__ __forceinline__ void vt_pipeline(const Geo& geo, const T* q, int64_t 
   const int lh = lane >> 5;
   const int nseg = geo.nseg();
 
-  int n_tiles = 0;
-  for (int s = 0; s < nseg; ++s) n_tiles += geo.seg(s).tiles;
+  const int n_tiles = geo.n_tiles();
 
   frag qf[NKS];
   {
@@ -1391,7 +1405,7 @@ __device__ __forceinline__ void vt_pipeline(const Geo& geo, const T* q, int64_t 
       }
   };
   // mask cursor (the tile in the MFMA phase)
-  MaskCursor mc{0, 0, geo.seg(0)};
+  MaskCursor mc{0, geo.first(), geo.seg(0)};
   auto mfix = [&]() __attribute__((always_inline)) {
     while (mc.t >= mc.g.tiles && mc.s < nseg) {
       ++mc.s;
@@ -1504,7 +1518,11 @@ __device__ __forceinline__ void vt_pipeline(const Geo& geo, const T* q, int64_t 
   if (grp == 0) __syncthreads();  // both groups pass the same number of barriers
 
   const float ltot = pair_sum(lsum);
-  const float inv = ltot > 0.f ? 1.0f / ltot : 0.f;
+  float inv = ltot > 0.f ? 1.0f / ltot : 0.f;
+  float row_lse = ltot > 0.f ? m * scale + logf(ltot) : -INFINITY;
+  if constexpr (Geo::kSplit) {
+    if (!geo.merge(o, inv, row_lse)) return;
+  }
   if (r0 + lq < Lq) {
     T* og = out + (int64_t)lq * o_rs;
 #pragma unroll
@@ -1516,14 +1534,16 @@ __device__ __forceinline__ void vt_pipeline(const Geo& geo, const T* q, int64_t 
                 (T)(o[dt][4 * g + 2] * inv), (T)(o[dt][4 * g + 3] * inv)};
         *reinterpret_cast<t4*>(og + 32 * dt + 8 * g + 4 * lh) = w;
       }
-    if (lh == 0) lse[(int64_t)lq * lse_rs] = ltot > 0.f ? m * scale + logf(ltot) : -INFINITY;
+    if (lh == 0) lse[(int64_t)lq * lse_rs] = row_lse;
   }
 }
 
 // One attention call: a single segment.
 struct OneSegment {
-  static constexpr bool kPagedK = false;
+  static constexpr bool kPagedK = false, kSplit = false;
+  static constexpr int first() { return 0; }
   StepSeg g;
+  __device__ __forceinline__ int n_tiles() const { return g.tiles; }
   const char* kb;
   const char* vb;
   __device__ __forceinline__ int nseg() const { return 1; }
@@ -1583,6 +1603,7 @@ __global__ __launch_bounds__(kPPThreads, 2) void attn_fwd_16bit_vt(AttnParams p)
 // s > rank: all keys of that source, back-half rows only) with one online softmax, and
 // writes the final out / lse: vt_pipeline over one segment per step.
 //--------------------------------------------------------------------------------------
+}  // namespace
 struct SweepParams {
   const void* q;
   void* out;
@@ -1608,18 +1629,25 @@ struct SweepParams {
   // dynamic row tile hand-out (claim_block): the launch's counters, or NULL for the fixed order
   unsigned* claim;
 };
+namespace {
 
 // The ring steps of one row tile (rows [row_tile0, row_tile0 + rows) of a sequence of L),
 // in tiles of BN keys.  PAGED: the K of every source is a paged cache (SweepParams::kpt).
 template <int BN, bool PAGED = false>
 struct RingSegments {
-  static constexpr bool kPagedK = PAGED;
+  static constexpr bool kPagedK = PAGED, kSplit = false;
+  static constexpr int first() { return 0; }
   const SweepParams* p;
   int L, row_tile0, rows, kvh, seq;
   // bytes from a source's K / V^T to this sequence and kv head (paged K: to this kv head
   // of the cache's first row)
   int64_t k_off, v_off;
   __device__ __forceinline__ int nseg() const { return p->S; }
+  __device__ __forceinline__ int n_tiles() const {
+    int n = 0;
+    for (int s = 0; s < p->S; ++s) n += seg(s).tiles;
+    return n;
+  }
   __device__ __forceinline__ StepSeg seg(int s) const {
     StepSeg g;
     g.src = p->rank - s < 0 ? p->rank - s + p->S : p->rank - s;
@@ -2445,8 +2473,7 @@ __device__ __forceinline__ void e8_pipeline(E8Lds<D>& lds, const Geo& geo,
   const int lh = lane >> 5;
   const int nseg = geo.nseg();
 
-  int n_tiles = 0;
-  for (int s = 0; s < nseg; ++s) n_tiles += geo.seg(s).tiles;
+  const int n_tiles = geo.n_tiles();
 
   // Q^T fragments: lane (query lq, half lh) holds d = 64 t + 32 lh + 0..31 of k-step t
   {
@@ -2583,7 +2610,7 @@ __device__ __forceinline__ void e8_pipeline(E8Lds<D>& lds, const Geo& geo,
   };
 
   // mask cursor (the tile in the MFMA phase) and the scale of its segment
-  MaskCursor mc{0, 0, geo.seg(0)};
+  MaskCursor mc{0, geo.first(), geo.seg(0)};
   bool seg_new = false;  // the tile in the MFMA phase starts a segment after the first
   float v_ratio = 1.f;   // vd of the previous segment / vd of this one
   auto mfix = [&]() __attribute__((always_inline)) {
@@ -2749,7 +2776,7 @@ __device__ __forceinline__ void e8_pipeline(E8Lds<D>& lds, const Geo& geo,
   using T = std::true_type;
   if constexpr (SP == 1) {
     // one segment: mask-free tiles with one e4m3 term, then masked tiles with two
-    const int n_free = mc.g.first_mask;
+    const int n_free = max(mc.g.first_mask - mc.t, 0);
     int j = 0;
     if (n_free > 0) {
       tile(0, P0{}, F{});
@@ -2782,7 +2809,11 @@ __device__ __forceinline__ void e8_pipeline(E8Lds<D>& lds, const Geo& geo,
   if (grp == 0) __syncthreads();  // both groups pass the same number of barriers
 
   const float ltot = pair_sum(lsum);
-  const float inv = ltot > 0.f ? mc.g.vd / ltot : 0.f;
+  float inv = ltot > 0.f ? mc.g.vd / ltot : 0.f;
+  float row_lse = ltot > 0.f ? m2 * kLn2 + logf(ltot) : -INFINITY;
+  if constexpr (Geo::kSplit) {
+    if (!geo.merge(o, inv, row_lse)) return;
+  }
   if (r0 + lq < Lq) {
     __bf16* og = out + (int64_t)lq * o_rs;
 #pragma unroll
@@ -2793,7 +2824,7 @@ __device__ __forceinline__ void e8_pipeline(E8Lds<D>& lds, const Geo& geo,
                     (__bf16)(o[dt][4 * g + 2] * inv), (__bf16)(o[dt][4 * g + 3] * inv)};
         *reinterpret_cast<bf16x4*>(og + 32 * dt + 8 * g + 4 * lh) = w;
       }
-    if (lh == 0) lse[(int64_t)lq * lse_rs] = ltot > 0.f ? m2 * kLn2 + logf(ltot) : -INFINITY;
+    if (lh == 0) lse[(int64_t)lq * lse_rs] = row_lse;
   }
 }
 

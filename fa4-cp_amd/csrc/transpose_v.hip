@@ -25,7 +25,19 @@ struct TransposeSet {
   const void* v[FA4CP_MAX_CP];
   void* vt[FA4CP_MAX_CP];
   const int32_t* pt[FA4CP_MAX_CP];
+  // A ring sweep's launch: of the first n_front tensors only the keys that the sweep's tiles
+  // reach, the front half of every sequence rounded up to kVtPad; and the words of `clear`
+  // (the sweep's counters) set to zero.
+  int n_front;
+  unsigned* clear;
+  int clear_words;
 };
+
+// Sets the launch's clear words, a grid-wide stride of threads.
+__device__ __forceinline__ void clear_words(const TransposeSet& set) {
+  if (blockIdx.y == 0)
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < set.clear_words; i += gridDim.x * blockDim.x) set.clear[i] = 0u;
+}
 
 // Page geometry of a paged launch.
 struct PageGeo {
@@ -53,6 +65,7 @@ __global__ __launch_bounds__(kTBlock) void transpose_v_kernel(
   constexpr int PITCH = D + E;       // LDS row pitch in elements (one unit of padding)
   __shared__ __attribute__((aligned(16))) T tile[kTK * PITCH];
 
+  clear_words(set);
   const int kt = blockIdx.x % n_kt;
   const int rest = blockIdx.x / n_kt;
   const int seq = rest % nseq;
@@ -61,7 +74,7 @@ __global__ __launch_bounds__(kTBlock) void transpose_v_kernel(
   vt_seq_range(cu, seq, total_k, sel, s, L);
   const int k0 = kt * kTK;
   const int lpad = round_up_pad(L);
-  if (k0 >= lpad) return;
+  if (k0 >= ((int)blockIdx.y < set.n_front ? round_up_pad(L >> 1) : lpad)) return;
   const int64_t P = vt_seq_start(cu, seq, total_k, sel);
   if (P + lpad > vt_ds) return;  // malformed cu: the sequence would not fit V^T
 
@@ -147,6 +160,7 @@ __global__ __launch_bounds__(kTBlock) void transpose_reg_kernel(
   const T* __restrict__ v = reinterpret_cast<const T*>(set.v[blockIdx.y]);
   const int32_t* __restrict__ pt = set.pt[blockIdx.y];
   T* __restrict__ vt = reinterpret_cast<T*>(set.vt[blockIdx.y]);
+  clear_words(set);
   const int kt = blockIdx.x % n_kt;
   const int rest = blockIdx.x / n_kt;
   const int seq = rest % nseq;
@@ -157,7 +171,8 @@ __global__ __launch_bounds__(kTBlock) void transpose_reg_kernel(
   const int slab = wave % SL;
   const int k0 = kt * kRegKeys<T, D>() + KB * (wave / SL);  // the wavefront's first key
   const int lpad = round_up_pad(L);
-  if (k0 >= lpad) return;  // (lpad is a multiple of KB: a started block lies inside)
+  // (the limits are multiples of KB: a started block lies inside)
+  if (k0 >= ((int)blockIdx.y < set.n_front ? round_up_pad(L >> 1) : lpad)) return;
   const int64_t P = vt_seq_start(cu, seq, total_k, sel);
   if (P + lpad > vt_ds) return;  // malformed cu: the sequence would not fit V^T
   const int g = lane & 7, c = lane >> 3;
@@ -331,11 +346,23 @@ extern "C" int fa4cp_transpose_v(const fa4cp_transpose_args* a, void* stream) {
 
 extern "C" int fa4cp_transpose_v_many(const fa4cp_transpose_args* a, const void* const* v, void* const* v_t,
                                       int32_t count, void* stream) {
+  return fa4cp_transpose_v_ring(a, v, v_t, count, 0, nullptr, 0, stream);
+}
+
+extern "C" int fa4cp_transpose_v_ring(const fa4cp_transpose_args* a, const void* const* v, void* const* v_t,
+                                      int32_t count, int32_t n_front, void* clear, int32_t clear_words, void* stream) {
   clear_error();
   if (a == nullptr || v == nullptr || v_t == nullptr) return set_error(FA4CP_EINVAL, "transpose_v: null pointer");
   if (count < 1 || count > FA4CP_MAX_CP)
     return set_error(FA4CP_EINVAL, "transpose_v_many: count %d out of [1, %d]", count, FA4CP_MAX_CP);
+  if (n_front < 0 || clear_words < 0 || (clear_words > 0 && clear == nullptr) || reinterpret_cast<uintptr_t>(clear) % 4 != 0)
+    return set_error(FA4CP_EINVAL, "transpose_v_ring: bad n_front %d or clear words (%d at %p)", n_front, clear_words, clear);
+  if (n_front > 0 && a->k_sel != FA4CP_SEL_ALL)
+    return set_error(FA4CP_EINVAL, "transpose_v_ring: n_front needs k_sel = ALL");
   TransposeSet set{};
+  set.n_front = n_front;
+  set.clear = static_cast<unsigned*>(clear);
+  set.clear_words = clear_words;
   for (int i = 0; i < count; ++i) {
     set.v[i] = v[i];
     set.vt[i] = v_t[i];
@@ -346,6 +373,13 @@ extern "C" int fa4cp_transpose_v_many(const fa4cp_transpose_args* a, const void*
 extern "C" int fa4cp_transpose_v_paged_many(const fa4cp_paged_args* a, const void* const* v_cache,
                                             const int32_t* const* page_table, void* const* v_t, int64_t vt_d_stride,
                                             int32_t count, void* stream) {
+  return fa4cp_transpose_v_paged_ring(a, v_cache, page_table, v_t, vt_d_stride, count, 0, nullptr, 0, stream);
+}
+
+extern "C" int fa4cp_transpose_v_paged_ring(const fa4cp_paged_args* a, const void* const* v_cache,
+                                            const int32_t* const* page_table, void* const* v_t, int64_t vt_d_stride,
+                                            int32_t count, int32_t n_front, void* clear, int32_t clear_words,
+                                            void* stream) {
   clear_error();
   if (a == nullptr || v_cache == nullptr || page_table == nullptr || v_t == nullptr)
     return set_error(FA4CP_EINVAL, "transpose_v_paged: null pointer");
@@ -364,7 +398,12 @@ extern "C" int fa4cp_transpose_v_paged_many(const fa4cp_paged_args* a, const voi
   t.d = a->d;
   t.dtype = a->dtype;
   t.vt_d_stride = vt_d_stride;
+  if (n_front < 0 || clear_words < 0 || (clear_words > 0 && clear == nullptr) || reinterpret_cast<uintptr_t>(clear) % 4 != 0)
+    return set_error(FA4CP_EINVAL, "transpose_v_paged: bad n_front %d or clear words (%d at %p)", n_front, clear_words, clear);
   TransposeSet set{};
+  set.n_front = n_front;
+  set.clear = static_cast<unsigned*>(clear);
+  set.clear_words = clear_words;
   for (int i = 0; i < count; ++i) {
     if (a->total > 0 && page_table[i] == nullptr)
       return set_error(FA4CP_EINVAL, "transpose_v_paged: page table %d is null", i);

@@ -272,6 +272,21 @@ SIGNATURES = {
     "fa4cp_ring_sweep_fwd": (ctypes.c_int, [ctypes.POINTER(SweepArgs), ctypes.c_void_p]),
     "fa4cp_ring_sweep_fwd_paged": (
         ctypes.c_int, [ctypes.POINTER(SweepArgs), ctypes.POINTER(SweepKPages), ctypes.c_void_p]),
+    "fa4cp_ring_sweep_fwd_ws": (
+        ctypes.c_int, [ctypes.POINTER(SweepArgs), ctypes.POINTER(SweepKPages), ctypes.c_void_p, ctypes.c_int64,
+                       ctypes.c_void_p]),
+    "fa4cp_ring_sweep_workspace_bytes": (ctypes.c_int64, [ctypes.POINTER(SweepArgs), ctypes.POINTER(ctypes.c_int32)]),
+    "fa4cp_transpose_v_ring": (
+        ctypes.c_int,
+        [ctypes.POINTER(TransposeArgs), ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_void_p),
+         ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p],
+    ),
+    "fa4cp_transpose_v_paged_ring": (
+        ctypes.c_int,
+        [ctypes.POINTER(PagedArgs), ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_void_p),
+         ctypes.POINTER(ctypes.c_void_p), ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p,
+         ctypes.c_int32, ctypes.c_void_p],
+    ),
     "fa4cp_ring_sweep_bwd": (ctypes.c_int, [ctypes.POINTER(SweepBwdArgs), ctypes.c_void_p]),
     "fa4cp_ring_sweep_bwd_workspace_bytes": (ctypes.c_int64, [ctypes.POINTER(SweepBwdArgs)]),
     "fa4cp_quantize_e4m3": (ctypes.c_int, [ctypes.POINTER(QuantArgs), ctypes.c_void_p]),

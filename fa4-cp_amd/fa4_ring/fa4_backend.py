@@ -159,9 +159,12 @@ def transpose_v(v: torch.Tensor, *, cu_seqlens_k: Optional[torch.Tensor] = None,
 
 
 def transpose_v_many(vs: Sequence[torch.Tensor], *, cu_seqlens_k: Optional[torch.Tensor] = None,
-                     max_seqlen_k: Optional[int] = None) -> Tuple[List[torch.Tensor], int]:
+                     max_seqlen_k: Optional[int] = None, n_front: int = 0,
+                     clear: Optional[Tuple[torch.Tensor, int]] = None) -> Tuple[List[torch.Tensor], int]:
     """transpose_v (k_sel = all) of up to 16 tensors of one shape and stride in one launch
-    (fa4cp_transpose_v_many), e.g. every source rank's V before a fused sweep."""
+    (fa4cp_transpose_v_ring), e.g. every source rank's V before a fused sweep.  Of the first
+    ``n_front`` tensors (a sweep's earlier sources) only the front half of every sequence is
+    transposed, and the launch clears the first n 32-bit words of ``clear`` = (tensor, n)."""
     lib = _lib.load()
     _require(1 <= len(vs) <= _lib.MAX_CP, f"1..{_lib.MAX_CP} tensors")
     v = vs[0]
@@ -175,7 +178,9 @@ def transpose_v_many(vs: Sequence[torch.Tensor], *, cu_seqlens_k: Optional[torch
         _require(max_seqlen_k is not None, "max_seqlen_k required with cu_seqlens_k")
         nseq = cu_seqlens_k.shape[0] - 1
     stride = int(lib.fa4cp_vt_min_d_stride(t_k, nseq))
-    vts = [torch.empty(h_kv * d * stride, dtype=v.dtype, device=v.device) for _ in vs]
+    n = h_kv * d * stride  # (a multiple of 128: every slice of the one buffer is 128-byte aligned)
+    buf = torch.empty(len(vs) * n, dtype=v.dtype, device=v.device)
+    vts = list(buf.split(n)) if n else [buf for _ in vs]
     a = _lib.TransposeArgs()
     a.v_row_stride, a.v_head_stride = v.stride(0), v.stride(1)
     a.cu_k = _lib.ptr(cu_seqlens_k)
@@ -188,8 +193,9 @@ def transpose_v_many(vs: Sequence[torch.Tensor], *, cu_seqlens_k: Optional[torch
     a.vt_d_stride = stride
     src = (ctypes.c_void_p * len(vs))(*[x.data_ptr() for x in vs])
     dst = (ctypes.c_void_p * len(vs))(*[x.data_ptr() for x in vts])
-    _lib.check(lib.fa4cp_transpose_v_many(ctypes.byref(a), src, dst, len(vs), _lib.stream_handle(v.device)),
-               "fa4cp_transpose_v_many")
+    words, n_words = (None, 0) if clear is None else (clear[0].data_ptr(), clear[1])
+    _lib.check(lib.fa4cp_transpose_v_ring(ctypes.byref(a), src, dst, len(vs), n_front, words, n_words,
+                                          _lib.stream_handle(v.device)), "fa4cp_transpose_v_ring")
     return vts, stride
 
 

@@ -134,17 +134,23 @@ def gather_kv_pages(ring: PagedKVRing, which: str, total: int, cu_seqlens: Optio
 
 
 def transpose_v_paged_many(ring: PagedKVRing, total: int, cu_seqlens: Optional[torch.Tensor] = None,
-                           max_seqlen: Optional[int] = None) -> Tuple[List[torch.Tensor], int]:
+                           max_seqlen: Optional[int] = None, n_front: int = 0,
+                           clear: Optional[Tuple[torch.Tensor, int]] = None) -> Tuple[List[torch.Tensor], int]:
     """Every source's V^T (the fa4cp_transpose_v layout of the contiguous V with the same
-    ``cu_seqlens``) written from its V pages in one launch; returns (V^T list, row stride)."""
+    ``cu_seqlens``) written from its V pages in one launch; returns (V^T list, row stride).
+    ``n_front`` / ``clear`` as for transpose_v_many."""
     lib = _lib.load()
     n, (_, _, h_kv, d) = ring.cp_size, ring.v[0].shape
     nseq = 1 if cu_seqlens is None else cu_seqlens.shape[0] - 1
     stride = int(lib.fa4cp_vt_min_d_stride(total, nseq))
-    vts = [torch.empty(h_kv * d * stride, dtype=ring.v[0].dtype, device=ring.v[0].device) for _ in range(n)]
+    size = h_kv * d * stride
+    buf = torch.empty(n * size, dtype=ring.v[0].dtype, device=ring.v[0].device)
+    vts = list(buf.split(size))
     a = _paged_args(ring, total, cu_seqlens, max_seqlen)
     arr = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])  # noqa: E731
-    _lib.check(lib.fa4cp_transpose_v_paged_many(ctypes.byref(a), arr(ring.v), arr(ring.page_tables), arr(vts),
-                                                stride, n, _lib.stream_handle(ring.v[0].device)),
-               "fa4cp_transpose_v_paged_many")
+    words, n_words = (None, 0) if clear is None else (clear[0].data_ptr(), clear[1])
+    _lib.check(lib.fa4cp_transpose_v_paged_ring(ctypes.byref(a), arr(ring.v), arr(ring.page_tables), arr(vts),
+                                                stride, n, n_front, words, n_words,
+                                                _lib.stream_handle(ring.v[0].device)),
+               "fa4cp_transpose_v_paged_ring")
     return vts, stride

@@ -330,9 +330,9 @@ def ring_sweep(local_q: torch.Tensor, local_k: torch.Tensor, local_v: torch.Tens
         # the sweep's arguments carry K's row and head strides only: D must be contiguous
         assert k.stride(2) == 1 and v.stride(2) == 1, "K and V shards must be contiguous in D"
     assert all(v.stride() == vs[0].stride() for v in vs), "all V shards must share strides"
-    vts, stride = transpose_v_many(vs, cu_seqlens_k=cu_seqlens, max_seqlen_k=max_seqlen)
-    return _sweep_launch(local_q, [k.data_ptr() for k in ks], (ks[0].stride(0), ks[0].stride(1)), h_kv, vts,
-                         stride, cfg, cu_seqlens, max_seqlen, out, lse, descales)
+    return _sweep_launch(local_q, [k.data_ptr() for k in ks], (ks[0].stride(0), ks[0].stride(1)), h_kv,
+                         lambda **kw: transpose_v_many(vs, cu_seqlens_k=cu_seqlens, max_seqlen_k=max_seqlen, **kw),
+                         cfg, cu_seqlens, max_seqlen, out, lse, descales)
 
 
 def ring_sweep_paged(local_q: torch.Tensor, cfg: RingConfig, ring: "PagedKVRing",
@@ -351,7 +351,6 @@ def ring_sweep_paged(local_q: torch.Tensor, cfg: RingConfig, ring: "PagedKVRing"
         "caches must match local_q's dtype, head dim and device"
     nseq = 1 if cu_seqlens is None else cu_seqlens.shape[0] - 1
     assert ring.page_tables[0].shape[0] == nseq, "page tables need one row per local sequence"
-    vts, stride = transpose_v_paged_many(ring, total, cu_seqlens, max_seqlen)
     kp = _lib.SweepKPages()
     for i, pt in enumerate(ring.page_tables):
         kp.page_table[i] = pt.data_ptr()
@@ -360,16 +359,18 @@ def ring_sweep_paged(local_q: torch.Tensor, cfg: RingConfig, ring: "PagedKVRing"
     kp.num_pages = kc.shape[0]
     # a cache is [num_pages, page_size, H_kv, D]: rows at stride(1), heads at stride(2)
     return _sweep_launch(local_q, [k.data_ptr() for k in ring.k], (kc.stride(1), kc.stride(2)), kc.shape[2],
-                         vts, stride, cfg, cu_seqlens, max_seqlen, out, lse, descales, kpages=kp)
+                         lambda **kw: transpose_v_paged_many(ring, total, cu_seqlens, max_seqlen, **kw),
+                         cfg, cu_seqlens, max_seqlen, out, lse, descales, kpages=kp)
 
 
 def _sweep_launch(local_q: torch.Tensor, k_ptrs: List[int], k_strides: Tuple[int, int], h_kv: int,
-                  vts: List[torch.Tensor], stride: int, cfg: RingConfig, cu_seqlens: Optional[torch.Tensor],
+                  transpose, cfg: RingConfig, cu_seqlens: Optional[torch.Tensor],
                   max_seqlen: Optional[int], out: Optional[torch.Tensor], lse: Optional[torch.Tensor],
                   descales: Optional[Descales], kpages: Optional["_lib.SweepKPages"] = None) -> torch.Tensor:
-    """Queues fa4cp_ring_sweep_fwd over every source rank's K (device addresses `k_ptrs`, row
-    and head strides `k_strides`) and V^T buffers `vts` (row stride `stride`); with `kpages`,
-    fa4cp_ring_sweep_fwd_paged, the K addresses being the sources' paged caches."""
+    """Queues `transpose` (every source's V^T as this rank reads it: transpose_v_many or its paged
+    form, given n_front and clear) and the sweep over every source rank's K (device addresses
+    `k_ptrs`, row and head strides `k_strides`) and V^T; with `kpages` the K addresses are the
+    sources' paged caches."""
     S, rank = cfg.cp_size, cfg.cp_rank
     total, h_q, d = local_q.shape
     dev = local_q.device
@@ -388,8 +389,6 @@ def _sweep_launch(local_q: torch.Tensor, k_ptrs: List[int], k_strides: Tuple[int
         f"out must be [{total}, {h_q}, {d}] {odt} on {dev}, contiguous in D"
     assert lse.shape == (total, h_q) and lse.dtype == torch.float32 and lse.device == dev and lse.stride(1) == 1, \
         f"lse must be [{total}, {h_q}] float32 on {dev} with unit head stride"
-    for i, vt in enumerate(vts):
-        assert vt.device == dev, f"source {i}'s V^T must be on {dev}"
     if cu_seqlens is not None:
         assert cu_seqlens.dtype == torch.int32 and cu_seqlens.device == dev and cu_seqlens.is_contiguous(), \
             "cu_seqlens must be contiguous int32 on the device"
@@ -401,9 +400,7 @@ def _sweep_launch(local_q: torch.Tensor, k_ptrs: List[int], k_strides: Tuple[int
     a.lse_row_stride = lse.stride(0)
     for i in range(S):
         a.k[i] = k_ptrs[i]
-        a.v_t[i] = vts[i].data_ptr()
     a.k_row_stride, a.k_head_stride = k_strides
-    a.vt_d_stride = stride
     a.cu = _lib.ptr(cu_seqlens)
     a.nseq = nseq
     a.max_seqlen = int(max_seqlen) if cu_seqlens is not None else total
@@ -413,18 +410,25 @@ def _sweep_launch(local_q: torch.Tensor, k_ptrs: List[int], k_strides: Tuple[int
     a.cp_rank, a.cp_size = rank, S
     a.softmax_scale = float(cfg.softmax_scale if cfg.softmax_scale is not None else 1.0 / math.sqrt(d))
     a.q_descale, a.k_descale, a.v_descale = _lib.ptr(qd), _lib.ptr(kd), _lib.ptr(vd)
-    launch_sweep(a, dev, kpages)
+    # where the sweep is split over few row tiles: its partial results, and its counters, which
+    # the V^T launch clears
+    words = ctypes.c_int32()
+    need = _lib.load().fa4cp_ring_sweep_workspace_bytes(ctypes.byref(a), ctypes.byref(words))
+    _lib.check(int(min(need, 0)), "fa4cp_ring_sweep_workspace_bytes")
+    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need > 0 else None
+    vts, a.vt_d_stride = transpose(n_front=rank, clear=None if ws is None else (ws, words.value))
+    for i, vt in enumerate(vts):
+        assert vt.device == dev, f"source {i}'s V^T must be on {dev}"
+        a.v_t[i] = vt.data_ptr()
+    launch_sweep(a, dev, kpages, ws)
     return out
 
 
-def launch_sweep(args: "_lib.SweepArgs", device: torch.device,
-                 kpages: Optional["_lib.SweepKPages"] = None) -> None:
+def launch_sweep(args: "_lib.SweepArgs", device: torch.device, kpages: Optional["_lib.SweepKPages"] = None,
+                 workspace: Optional[torch.Tensor] = None) -> None:
     """Queues the fused sweep kernel on the current stream of `device` (with `kpages`: the
-    paged-K sweep)."""
-    lib = _lib.load()
-    if kpages is None:
-        _lib.check(lib.fa4cp_ring_sweep_fwd(ctypes.byref(args), _lib.stream_handle(device)),
-                   "fa4cp_ring_sweep_fwd")
-    else:
-        _lib.check(lib.fa4cp_ring_sweep_fwd_paged(ctypes.byref(args), ctypes.byref(kpages),
-                                                  _lib.stream_handle(device)), "fa4cp_ring_sweep_fwd_paged")
+    paged-K sweep; with `workspace`: split where its shape asks for it)."""
+    _lib.check(_lib.load().fa4cp_ring_sweep_fwd_ws(
+        ctypes.byref(args), None if kpages is None else ctypes.byref(kpages), _lib.ptr(workspace),
+        0 if workspace is None else workspace.numel(), _lib.stream_handle(device)),
+        "fa4cp_ring_sweep_fwd" if kpages is None else "fa4cp_ring_sweep_fwd_paged")

@@ -174,6 +174,16 @@ int fa4cp_transpose_v_many(const fa4cp_transpose_args* args, const void* const* 
                            int32_t count, void* stream);
 
 /*
+ * fa4cp_transpose_v_many (k_sel = ALL) as a ring sweep of rank n_front needs it: of v[i], i <
+ * n_front (the sources of which the rank attends the front half of every sequence's keys), only
+ * that half, rounded up to 128 positions, is read and written.  The launch also sets the
+ * clear_words 32-bit words at `clear` (device memory, 4-byte aligned; NULL with 0 words) to
+ * zero: the counters of fa4cp_ring_sweep_fwd_ws.
+ */
+int fa4cp_transpose_v_ring(const fa4cp_transpose_args* args, const void* const* v, void* const* v_t,
+                           int32_t count, int32_t n_front, void* clear, int32_t clear_words, void* stream);
+
+/*
  * Paged K / V caches.  No counterpart in the reference, which keeps every rotated K/V shard
  * contiguous (README.md:139-140: "no paged KV yet"); these two calls feed paged caches to
  * fa4cp_ring_sweep_fwd.  A source rank's cache holds num_pages pages of page_size rows;
@@ -210,6 +220,10 @@ int fa4cp_gather_kv_pages(const fa4cp_paged_args* args, const void* const* cache
 int fa4cp_transpose_v_paged_many(const fa4cp_paged_args* args, const void* const* v_cache,
                                  const int32_t* const* page_table, void* const* v_t, int64_t vt_d_stride,
                                  int32_t count, void* stream);
+/* The same as a ring sweep of rank n_front needs it, with the words to clear (fa4cp_transpose_v_ring). */
+int fa4cp_transpose_v_paged_ring(const fa4cp_paged_args* args, const void* const* v_cache,
+                                 const int32_t* const* page_table, void* const* v_t, int64_t vt_d_stride,
+                                 int32_t count, int32_t n_front, void* clear, int32_t clear_words, void* stream);
 
 /*
  * One rank's whole causal zig-zag ring sweep in a single launch (fa4_ring/ring_attention.py:61-174
@@ -266,6 +280,23 @@ typedef struct fa4cp_sweep_kpages {
 } fa4cp_sweep_kpages;
 
 int fa4cp_ring_sweep_fwd_paged(const fa4cp_sweep_args* args, const fa4cp_sweep_kpages* k_pages, void* stream);
+
+/*
+ * fa4cp_ring_sweep_fwd (k_pages == NULL) or fa4cp_ring_sweep_fwd_paged with a caller-owned
+ * workspace of fa4cp_ring_sweep_workspace_bytes(args) bytes of device memory, 16-byte aligned.
+ * Where a sweep has too few row tiles to fill the chip (short sequences, few heads) those bytes
+ * are above 0, and with them several workgroups share a row tile's keys: each leaves an fp32
+ * partial result in the workspace, and the last of a row tile merges them.  The workspace's
+ * first *clear_words 32-bit words (counters) must be zero when the sweep starts
+ * (fa4cp_transpose_v_ring can clear them); they are zero again when it has ended, and nothing
+ * else is kept across calls.  With a NULL workspace, and where 0 bytes are asked for, the call
+ * is the unsplit sweep.
+ */
+int fa4cp_ring_sweep_fwd_ws(const fa4cp_sweep_args* args, const fa4cp_sweep_kpages* k_pages, void* workspace,
+                            int64_t workspace_bytes, void* stream);
+/* Reads args' shape only (of cu, whether it is NULL); a negative FA4CP_E* code for a bad one.
+ * clear_words may be NULL. */
+int64_t fa4cp_ring_sweep_workspace_bytes(const fa4cp_sweep_args* args, int32_t* clear_words);
 
 /*
  * Backward of fa4cp_ring_sweep_fwd (BF16 / FP16, d = 64, 128 or 256).  No counterpart in the

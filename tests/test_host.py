@@ -268,6 +268,51 @@ def test_backward_workspace_size_and_checks():
     assert lib.fa4cp_ring_sweep_bwd(ctypes.byref(args(total=0, workspace=None)), None) == 0
 
 
+def test_ring_sweep_workspace_contract():
+    """fa4cp_ring_sweep_workspace_bytes: 0 bytes where the row tiles fill the chip (256 CUs) or all
+    cost alike on one CU each, more for short sequences and few heads, with one counter per row tile
+    and head group; bad shapes and a short or misaligned workspace are refused.  The pointers are
+    fake, so this never runs where a device is visible."""
+    if torch.cuda.is_available():
+        pytest.skip("fake device pointers: host-only test")
+    lib = _lib.load()
+    fake = 1 << 20
+
+    def args(**kw):
+        a = _lib.SweepArgs()
+        a.q = a.out = a.lse = fake
+        a.h_q, a.h_kv, a.d, a.dtype, a.total = 8, 2, 128, _lib.dtype_code(torch.bfloat16), 512
+        a.nseq, a.cp_size, a.cp_rank = 1, 4, 1
+        for k, v in kw.items():
+            setattr(a, k, v)
+        a.q_row_stride = a.o_row_stride = a.h_q * a.d
+        a.q_head_stride = a.o_head_stride = a.k_head_stride = a.d
+        a.k_row_stride, a.lse_row_stride = a.h_kv * a.d, a.h_q
+        a.vt_d_stride = int(lib.fa4cp_vt_min_d_stride(max(a.total, 0), a.nseq))
+        for i in range(a.cp_size):
+            a.k[i] = a.v_t[i] = fake
+        return a
+
+    words = ctypes.c_int32(-1)
+    need = lib.fa4cp_ring_sweep_workspace_bytes(ctypes.byref(args()), ctypes.byref(words))
+    assert need > 0 and words.value == 2 * 8  # two head groups of eight 64-row tiles
+    assert (need - 256) % (256 * 129 * 4) == 0  # counters, then slots of 256 rows x (128 + 1) floats
+    assert lib.fa4cp_ring_sweep_workspace_bytes(ctypes.byref(args(total=0)), ctypes.byref(words)) == 0
+    assert words.value == 0
+    packed = args(cu=fake, nseq=5, max_seqlen=640, total=1090, h_q=4, h_kv=1)
+    assert lib.fa4cp_ring_sweep_workspace_bytes(ctypes.byref(packed), ctypes.byref(words)) > 0
+    assert words.value == 1090 // 64 + 5  # at most one partial row tile per sequence
+    for kw in (dict(total=16384, h_q=32, h_kv=8, cp_size=8, cp_rank=3),  # the headline ring
+               dict(total=2048, h_q=32, h_kv=8, cp_size=8, cp_rank=7),  # 256 equal row tiles
+               dict(total=2, h_q=4, h_kv=1, cp_size=2, cp_rank=0)):
+        assert lib.fa4cp_ring_sweep_workspace_bytes(ctypes.byref(args(**kw)), None) == 0, kw
+    for kw in (dict(total=-1), dict(h_kv=3), dict(cp_rank=4), dict(cu=fake, nseq=0), dict(d=0)):
+        assert lib.fa4cp_ring_sweep_workspace_bytes(ctypes.byref(args(**kw)), None) < 0, kw
+    for ws, n in ((fake, need - 1), (fake + 8, need)):
+        rc = lib.fa4cp_ring_sweep_fwd_ws(ctypes.byref(args()), None, ws, n, None)
+        assert rc != 0 and b"workspace" in lib.fa4cp_last_error()
+
+
 @pytest.mark.parametrize("struct,cname", [(_lib.AttnArgs, "fa4cp_attn_args"),
                                            (_lib.TransposeArgs, "fa4cp_transpose_args"),
                                            (_lib.SweepArgs, "fa4cp_sweep_args"),
