@@ -14,6 +14,13 @@
 // chunks, and every thread owns the same NS chunk slots of every group: slot k of thread t
 // is chunk t + 256 k of the group.  Its row, head, position and scale are fixed, so they are
 // computed once, and a thread issues the loads of all its slots before it uses any.
+//
+// fa4cp_quantize_e4m3_many takes a ring's tensors (one q, every source's k and v) through the
+// same three launches: the workgroups are shared out over the tensors by their row groups, and
+// the second pass goes through tensors and groups in reverse, so that it starts on what the
+// first one left in the 256 MB last-level cache.  17 tensors of 335 MB (65536 tokens, H 32/8, cp
+// 8): 51 launches and 17 calls took 347 us of GPU time and 420 us with the host's; together they
+// take 166 us, 838 MB at 5.0 TB/s (175 us in forward order; 174 with 2048 workgroups).
 #include <mutex>
 
 #include "common.h"
@@ -35,9 +42,36 @@ struct QuantGeo {
   int rb;                // rows per group
 };
 
-__global__ void clear_words(unsigned* p, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0u;
+// One tensor of a launch, and the workgroups [first, first + wgs) that work on it.
+struct QuantItem {
+  const void* x;
+  unsigned* amax;
+  float* descale;
+  uint8_t* y;
+  QuantGeo g;
+  int first, wgs;
+};
+template <int N>
+struct QuantSet {
+  QuantItem item[N];
+  int count;
+};
+// The tensor of workgroup b.
+template <int N>
+__device__ __forceinline__ const QuantItem& item_of(const QuantSet<N>& set, int b) {
+  int i = 0;
+  if constexpr (N > 1)
+    while (i + 1 < set.count && b >= set.item[i + 1].first) ++i;
+  return set.item[i];
+}
+
+__device__ __forceinline__ int scales_of(const QuantGeo& g) { return g.cps ? g.cpr / g.cps : 1; }
+
+// A workgroup per tensor clears its amax words.
+template <int N>
+__global__ void clear_words(QuantSet<N> set) {
+  const QuantItem& it = set.item[N > 1 ? blockIdx.x : 0];
+  for (int i = threadIdx.x; i < scales_of(it.g); i += blockDim.x) it.amax[i] = 0u;
 }
 
 // The slots of this thread: x offset in a group (elements), y offset (bytes), row in the
@@ -83,17 +117,21 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-template <typename T, int NS>
-__global__ __launch_bounds__(kQBlock) void amax_kernel(const T* __restrict__ x, QuantGeo g, unsigned* amax) {
+template <typename T, int NS, int N>
+__global__ __launch_bounds__(kQBlock) void amax_kernel(QuantSet<N> set) {
   constexpr int E = 16 / sizeof(T);
-  const int nscale = g.cps ? g.cpr / g.cps : 1;
+  const QuantItem& it = item_of(set, blockIdx.x);
+  const QuantGeo g = it.g;
+  const T* __restrict__ x = reinterpret_cast<const T*>(it.x);
+  unsigned* const amax = it.amax;
+  const int nscale = scales_of(g);
   __shared__ unsigned smax[kQMaxScales];
   for (int i = threadIdx.x; i < nscale; i += kQBlock) smax[i] = 0u;
   const Slots<T, NS> sl(g);
   float acc[NS];
 #pragma unroll
   for (int k = 0; k < NS; ++k) acc[k] = 0.f;
-  for (int64_t grp = blockIdx.x; grp < g.groups; grp += gridDim.x) {
+  for (int64_t grp = (int)blockIdx.x - it.first; grp < g.groups; grp += it.wgs) {
     const int64_t r0 = grp * g.rb;
     const T* xb = x + r0 * g.rs;
     u32x4 w[NS];
@@ -143,12 +181,18 @@ __device__ __forceinline__ float div_rn(float x, float s, float rc) {
   return fmaf(-fmaf(q, s, -x), rc, q);
 }
 
-template <typename T, int NS>
-__global__ __launch_bounds__(kQBlock) void quant_kernel(const T* __restrict__ x, QuantGeo g, const unsigned* amax,
-                                                        float* descale, uint8_t* __restrict__ y) {
+template <typename T, int NS, int N>
+__global__ __launch_bounds__(kQBlock) void quant_kernel(QuantSet<N> set) {
   constexpr int E = 16 / sizeof(T);
-  const int nscale = g.cps ? g.cpr / g.cps : 1;
-  if (blockIdx.x == 0)
+  const int b = N > 1 ? (int)(gridDim.x - 1 - blockIdx.x) : (int)blockIdx.x;
+  const QuantItem& it = item_of(set, b);
+  const QuantGeo g = it.g;
+  const T* __restrict__ x = reinterpret_cast<const T*>(it.x);
+  const unsigned* const amax = it.amax;
+  float* const descale = it.descale;
+  uint8_t* __restrict__ y = it.y;
+  const int nscale = scales_of(g);
+  if (b == it.first)
     for (int i = threadIdx.x; i < nscale; i += kQBlock) descale[i] = scale_of(amax[i]);
   const Slots<T, NS> sl(g);
   float sc[NS], rc[NS];
@@ -158,7 +202,8 @@ __global__ __launch_bounds__(kQBlock) void quant_kernel(const T* __restrict__ x,
     rc[k] = 1.f / sc[k];  // correctly rounded
   }
   const int64_t y_gs = (int64_t)g.rb * g.cpr * E;  // y bytes per row group
-  for (int64_t grp = blockIdx.x; grp < g.groups; grp += gridDim.x) {
+  for (int64_t k0 = b - it.first; k0 < g.groups; k0 += it.wgs) {
+    const int64_t grp = N > 1 ? g.groups - 1 - k0 : k0;
     const int64_t r0 = grp * g.rb;
     const T* xb = x + r0 * g.rs;
     uint8_t* yb = y + grp * y_gs;
@@ -189,32 +234,50 @@ __global__ __launch_bounds__(kQBlock) void quant_kernel(const T* __restrict__ x,
   }
 }
 
-template <typename T, int NS>
-void launch_ns(const fa4cp_quant_args& a, const QuantGeo& g, int nscale, hipStream_t st) {
-  unsigned* amax = reinterpret_cast<unsigned*>(a.amax);
-  hipLaunchKernelGGL(clear_words, dim3((nscale + kQBlock - 1) / kQBlock), dim3(kQBlock), 0, st, amax, nscale);
-  const T* x = reinterpret_cast<const T*>(a.x);
-  const int grid = (int)(g.groups < kQMaxGrid ? (g.groups > 0 ? g.groups : 1) : kQMaxGrid);
-  if (g.rows > 0) hipLaunchKernelGGL((amax_kernel<T, NS>), dim3(grid), dim3(kQBlock), 0, st, x, g, amax);
-  hipLaunchKernelGGL((quant_kernel<T, NS>), dim3(grid), dim3(kQBlock), 0, st, x, g, amax, a.descale,
-                     reinterpret_cast<uint8_t*>(a.y));
+template <typename T, int NS, int N>
+void launch_ns(const QuantSet<N>& set, int grid, bool rows, hipStream_t st) {
+  hipLaunchKernelGGL(clear_words<N>, dim3(set.count), dim3(kQBlock), 0, st, set);
+  if (rows) hipLaunchKernelGGL((amax_kernel<T, NS, N>), dim3(grid), dim3(kQBlock), 0, st, set);
+  hipLaunchKernelGGL((quant_kernel<T, NS, N>), dim3(grid), dim3(kQBlock), 0, st, set);
 }
 
-template <typename T>
-int launch(const fa4cp_quant_args& a, int cps, hipStream_t st) {
+// a[i] with cps[i] 16-byte chunks per scale, i < count <= N.  Every tensor gets its share of
+// kQMaxGrid workgroups by its row groups, at least one and at most one per group.
+template <typename T, int N>
+int launch(const fa4cp_quant_args* a, const int* cps, int count, hipStream_t st) {
   constexpr int E = 16 / sizeof(T);
-  QuantGeo g;
-  g.rows = a.rows;
-  g.rs = a.row_stride;
-  g.hs = a.head_stride;
-  g.cph = a.d / E;
-  g.cpr = a.h * g.cph;
-  g.cps = cps;
-  g.rb = g.cpr <= kQSpan ? kQSpan / g.cpr : 1;
-  g.groups = (a.rows + g.rb - 1) / g.rb;
-  const int nscale = cps ? g.cpr / cps : 1;
-  if (g.rb * g.cpr <= kQSpan) launch_ns<T, kQSpan / kQBlock>(a, g, nscale, st);
-  else launch_ns<T, kQMaxSlots>(a, g, nscale, st);
+  QuantSet<N> set;
+  set.count = count;
+  int64_t groups = 0;
+  bool wide = false;
+  for (int i = 0; i < count; ++i) {
+    QuantItem& it = set.item[i];
+    QuantGeo& g = it.g;
+    g.rows = a[i].rows;
+    g.rs = a[i].row_stride;
+    g.hs = a[i].head_stride;
+    g.cph = a[i].d / E;
+    g.cpr = a[i].h * g.cph;
+    g.cps = cps[i];
+    g.rb = g.cpr <= kQSpan ? kQSpan / g.cpr : 1;
+    g.groups = (g.rows + g.rb - 1) / g.rb;
+    groups += g.groups;
+    wide = wide || g.rb * g.cpr > kQSpan;
+    it.x = a[i].x;
+    it.amax = reinterpret_cast<unsigned*>(a[i].amax);
+    it.descale = a[i].descale;
+    it.y = reinterpret_cast<uint8_t*>(a[i].y);
+  }
+  int grid = 0;
+  for (int i = 0; i < count; ++i) {
+    QuantItem& it = set.item[i];
+    const int64_t share = groups > kQMaxGrid ? (it.g.groups * kQMaxGrid + groups - 1) / groups : it.g.groups;
+    it.first = grid;
+    it.wgs = (int)(share > 1 ? share : 1);
+    grid += it.wgs;
+  }
+  if (wide) launch_ns<T, kQMaxSlots, N>(set, grid, groups > 0, st);
+  else launch_ns<T, kQSpan / kQBlock, N>(set, grid, groups > 0, st);
   return check_launch("quantize_e4m3");
 }
 
@@ -259,11 +322,12 @@ int quant_check(const char* what, const fa4cp_quant_args* a, bool need_amax, int
   return FA4CP_OK;
 }
 
-int quant_launch(const fa4cp_quant_args& a, int cps, hipStream_t st) {
-  switch (a.dtype) {
-    case FA4CP_BF16: return launch<__bf16>(a, cps, st);
-    case FA4CP_FP16: return launch<_Float16>(a, cps, st);
-    default: return launch<float>(a, cps, st);
+template <int N>
+int quant_launch(const fa4cp_quant_args* a, const int* cps, int count, hipStream_t st) {
+  switch (a->dtype) {
+    case FA4CP_BF16: return launch<__bf16, N>(a, cps, count, st);
+    case FA4CP_FP16: return launch<_Float16, N>(a, cps, count, st);
+    default: return launch<float, N>(a, cps, count, st);
   }
 }
 
@@ -275,7 +339,24 @@ extern "C" int fa4cp_quantize_e4m3(const fa4cp_quant_args* a, void* stream) {
   int cps = 0, nscale = 0;
   const int rc = quant_check("quantize_e4m3", a, true, &cps, &nscale);
   if (rc != FA4CP_OK) return rc;
-  return quant_launch(*a, cps, (hipStream_t)stream);
+  return quant_launch<1>(a, &cps, 1, (hipStream_t)stream);
+}
+
+extern "C" int fa4cp_quantize_e4m3_many(const fa4cp_quant_args* a, int32_t count, void* stream) {
+  clear_error();
+  const char* what = "quantize_e4m3_many";
+  if (a == nullptr) return set_error(FA4CP_EINVAL, "%s: null pointer", what);
+  if (count < 1 || count > FA4CP_QUANT_MAX_TENSORS)
+    return set_error(FA4CP_EINVAL, "%s: count %d out of [1, %d]", what, count, FA4CP_QUANT_MAX_TENSORS);
+  int cps[FA4CP_QUANT_MAX_TENSORS];
+  for (int i = 0; i < count; ++i) {
+    int nscale = 0;
+    const int rc = quant_check(what, a + i, true, cps + i, &nscale);
+    if (rc != FA4CP_OK) return rc;
+    if (a[i].dtype != a[0].dtype)
+      return set_error(FA4CP_EINVAL, "%s: tensor %d has dtype %d, the first %d", what, i, a[i].dtype, a[0].dtype);
+  }
+  return quant_launch<FA4CP_QUANT_MAX_TENSORS>(a, cps, count, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -338,5 +419,5 @@ extern "C" int fa4cp_quantize_e4m3_noalloc(const fa4cp_quant_args* a, void* stre
   if (rc != FA4CP_OK) return rc;
   fa4cp_quant_args b = *a;
   b.amax = reinterpret_cast<float*>(words);
-  return fa4cp::quant_launch(b, cps, st);
+  return fa4cp::quant_launch<1>(&b, &cps, 1, st);
 }

@@ -20,6 +20,9 @@ constexpr int kMaxShards = 64;
 struct ShardTable {
   const char* p[kMaxShards];
 };
+struct LocalTable {
+  char* p[kMaxShards];
+};
 
 // Source row (in the full tensor) of local row i of rank `rank`.
 __device__ __forceinline__ int64_t shard_src_row(const int32_t* __restrict__ full_cu, int nseq,
@@ -108,6 +111,24 @@ __global__ __launch_bounds__(kBlock) void unshard_kernel(ShardTable shards, char
   for (int u = threadIdx.x % lanes_per_row; u < units_per_row; u += lanes_per_row) d[u] = s[u];
 }
 
+// Every rank's shard at once: full row n goes to its owner's local row.  The reads are one
+// stream and the writes 2 cp_size of them; one launch instead of cp_size short ones.
+template <typename U>
+__global__ __launch_bounds__(kBlock) void shard_all_kernel(const char* __restrict__ src, LocalTable locals,
+                                                           int64_t n_full, int units_per_row, int lanes_per_row,
+                                                           const int32_t* __restrict__ full_cu, int nseq, int S) {
+  const int rows_per_block = kBlock / lanes_per_row;
+  const int64_t n = (int64_t)blockIdx.x * rows_per_block + threadIdx.x / lanes_per_row;
+  if (n >= n_full) return;
+  int rank;
+  int64_t local;
+  unshard_src(full_cu, nseq, n_full, S, n, rank, local);
+  if (rank < 0 || rank >= S || local < 0 || local >= n_full / S) return;  // malformed full_cu
+  const U* s = reinterpret_cast<const U*>(src) + n * units_per_row;
+  U* d = reinterpret_cast<U*>(locals.p[rank]) + local * units_per_row;
+  for (int u = threadIdx.x % lanes_per_row; u < units_per_row; u += lanes_per_row) d[u] = s[u];
+}
+
 // Picks the widest copy unit the row size and the pointers allow.
 int unit_bytes(int64_t row_bytes, uintptr_t align_bits) {
   if (row_bytes % 16 == 0 && (align_bits % 16) == 0) return 16;
@@ -174,6 +195,41 @@ extern "C" int fa4cp_zigzag_shard(const void* src_full, void* dst_local, int64_t
     hipLaunchKernelGGL(shard_kernel<uint8_t>, dim3((unsigned)blocks), dim3(kBlock), 0, st, s, d,
                        n_local, (int)units, lanes, full_cu, nseq, total_full, cp_rank, cp_size);
   return check_launch("zigzag_shard");
+}
+
+extern "C" int fa4cp_zigzag_shard_all(const void* src_full, void* const* dst_locals, int64_t row_bytes,
+                                      const int32_t* full_cu, int32_t nseq, int64_t total_full, int32_t cp_size,
+                                      void* stream) {
+  clear_error();
+  if (!dst_locals || (total_full > 0 && !src_full))  // the tensors may be NULL with no rows
+    return set_error(FA4CP_EINVAL, "zigzag_shard_all: null pointer");
+  int rc = check_zigzag_args(row_bytes, nseq, total_full, cp_size, full_cu, "zigzag_shard_all");
+  if (rc) return rc;
+  LocalTable tab = {};
+  uintptr_t bits = (uintptr_t)src_full;
+  for (int r = 0; r < cp_size; ++r) {
+    if (total_full > 0 && !dst_locals[r]) return set_error(FA4CP_EINVAL, "zigzag_shard_all: shard %d is null", r);
+    tab.p[r] = (char*)dst_locals[r];
+    bits |= (uintptr_t)dst_locals[r];
+  }
+  if (total_full == 0) return FA4CP_OK;
+  const int ub = unit_bytes(row_bytes, bits);
+  const int64_t units = row_bytes / ub;
+  if (units > 0x7fffffff) return set_error(FA4CP_EINVAL, "zigzag_shard_all: row too large");
+  const int lanes = lanes_for(units);
+  const int rows_per_block = kBlock / lanes;
+  const int64_t blocks = (total_full + rows_per_block - 1) / rows_per_block;
+  if (blocks > 0x7fffffffLL) return set_error(FA4CP_EINVAL, "zigzag_shard_all: too many rows");
+  hipStream_t st = (hipStream_t)stream;
+  const char* s = (const char*)src_full;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kBlock), 0, st, s, tab, total_full, (int)units, lanes, full_cu,
+                       nseq, cp_size);
+  };
+  if (ub == 16) go(shard_all_kernel<u32x4>);
+  else if (ub == 4) go(shard_all_kernel<uint32_t>);
+  else go(shard_all_kernel<uint8_t>);
+  return check_launch("zigzag_shard_all");
 }
 
 extern "C" int fa4cp_zigzag_unshard(const void* const* shard_ptrs, void* dst_full,

@@ -257,6 +257,11 @@ SIGNATURES = {
         [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int32,
          ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p],
     ),
+    "fa4cp_zigzag_shard_all": (
+        ctypes.c_int,
+        [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p), ctypes.c_int64, ctypes.c_void_p, ctypes.c_int32,
+         ctypes.c_int64, ctypes.c_int32, ctypes.c_void_p],
+    ),
     "fa4cp_zigzag_unshard": (
         ctypes.c_int,
         [ctypes.POINTER(ctypes.c_void_p), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
@@ -290,6 +295,7 @@ SIGNATURES = {
     "fa4cp_ring_sweep_bwd": (ctypes.c_int, [ctypes.POINTER(SweepBwdArgs), ctypes.c_void_p]),
     "fa4cp_ring_sweep_bwd_workspace_bytes": (ctypes.c_int64, [ctypes.POINTER(SweepBwdArgs)]),
     "fa4cp_quantize_e4m3": (ctypes.c_int, [ctypes.POINTER(QuantArgs), ctypes.c_void_p]),
+    "fa4cp_quantize_e4m3_many": (ctypes.c_int, [ctypes.POINTER(QuantArgs), ctypes.c_int32, ctypes.c_void_p]),
     "fa4cp_quantize_e4m3_noalloc": (ctypes.c_int, [ctypes.POINTER(QuantArgs), ctypes.c_void_p]),
     "fa4cp_last_error": (ctypes.c_char_p, []),
     "fa4cp_abi_version": (ctypes.c_int, []),

@@ -49,6 +49,41 @@ def quantize_e4m3(x: torch.Tensor, *, heads_per_scale: int = 0,
     return out, (descale.reshape(()) if g == 0 else descale)
 
 
+QUANT_MAX_TENSORS = 33  # FA4CP_QUANT_MAX_TENSORS
+
+
+def quantize_e4m3_many(xs: Sequence[torch.Tensor], *, heads_per_scale: Sequence[int]
+                       ) -> List[Tuple[torch.Tensor, torch.Tensor]]:
+    """quantize_e4m3 of every xs[i] with heads_per_scale[i], three launches for up to 33 tensors
+    (fa4cp_quantize_e4m3_many).  The tensors share a device and dtype; the descales are views of
+    one small tensor."""
+    lib = _lib.load()
+    dev, nscale = xs[0].device, []
+    for x, g in zip(xs, heads_per_scale):
+        assert x.is_cuda and x.dim() == 3 and x.stride(2) == 1, \
+            "x must be a [rows, h, d] device tensor, unit stride in d"
+        assert x.device == dev and x.dtype == xs[0].dtype, "the tensors must share a device and dtype"
+        assert g == 0 or (g > 0 and x.shape[1] % g == 0), f"heads_per_scale {g} must be 0 or divide h = {x.shape[1]}"
+        nscale.append(1 if g == 0 else x.shape[1] // g)
+    words = torch.empty(2 * sum(nscale), dtype=torch.float32, device=dev)  # amax words, then descales
+    amax, descales = words.data_ptr(), words[sum(nscale):].split(nscale)
+    code, stream, out = _lib.dtype_code(xs[0].dtype), _lib.stream_handle(dev), []
+    for at in range(0, len(xs), QUANT_MAX_TENSORS):
+        part = range(at, min(at + QUANT_MAX_TENSORS, len(xs)))
+        args = (_lib.QuantArgs * len(part))()
+        for a, i in zip(args, part):
+            x = xs[i]
+            rows, a.h, a.d = x.shape
+            y = torch.empty((rows, a.h, a.d), dtype=torch.float8_e4m3fn, device=dev)
+            a.x, a.rows, a.dtype, a.heads_per_scale = x.data_ptr(), rows, code, heads_per_scale[i]
+            a.row_stride, a.head_stride, _ = x.stride()
+            a.amax, a.descale, a.y = amax, descales[i].data_ptr(), y.data_ptr()
+            amax += 4 * nscale[i]
+            out.append((y, descales[i] if heads_per_scale[i] else descales[i].reshape(())))
+        _lib.check(lib.fa4cp_quantize_e4m3_many(args, len(part), stream), "fa4cp_quantize_e4m3_many")
+    return out
+
+
 QUANT_MAX_SCALES = 1024  # FA4CP_QUANT_MAX_SCALES
 
 
@@ -90,8 +125,14 @@ def quantize_ring(local_q: torch.Tensor, k_shards: Sequence[torch.Tensor], v_sha
     ``per_head`` scales q per kv-head group and k / v per kv head; otherwise per tensor."""
     h_q, h_kv = local_q.shape[1], k_shards[0].shape[1]
     assert h_q % h_kv == 0
-    q8, qd = quantize_e4m3(local_q, heads_per_scale=(h_q // h_kv) if per_head else 0)
     g = 1 if per_head else 0
-    k8, kd = zip(*(quantize_e4m3(k, heads_per_scale=g) for k in k_shards))
-    v8, vd = zip(*(quantize_e4m3(v, heads_per_scale=g) for v in v_shards))
+    n = len(k_shards)
+    xs = [local_q, *k_shards, *v_shards]
+    groups = [(h_q // h_kv) if per_head else 0] + [g] * (n + len(v_shards))
+    if all(x.dtype == local_q.dtype and x.device == local_q.device for x in xs):
+        (q8, qd), *kv = quantize_e4m3_many(xs, heads_per_scale=groups)
+    else:
+        (q8, qd), *kv = [quantize_e4m3(x, heads_per_scale=hs) for x, hs in zip(xs, groups)]
+    k8, kd = zip(*kv[:n])
+    v8, vd = zip(*kv[n:])
     return q8, list(k8), list(v8), Descales(q=qd, k=list(kd), v=list(vd))

@@ -40,7 +40,7 @@ from .fa4_backend import (SEL_ALL, SEL_BACK_HALF, SEL_FRONT_HALF, SUPPORTED_HEAD
                           out_dtype_for, pad_head_dim, sweep_descales, transpose_v, transpose_v_many, uses_vt)
 from .merge import merge_state_in_place, merge_states
 from .paged import PagedKVRing, gather_kv_pages, transpose_v_paged_many
-from .zigzag import zigzag_shard, zigzag_shard_varlen
+from .zigzag import zigzag_shard_all
 
 
 @dataclass
@@ -79,14 +79,8 @@ class LocalKVRing:
 
     @classmethod
     def from_full(cls, k: torch.Tensor, v: torch.Tensor, cp_size: int, full_cu_seqlens=None):
-        """Shards full-sequence K and V for every rank with the zig-zag gather kernel."""
-        if full_cu_seqlens is None:
-            ks = [zigzag_shard(k, r, cp_size) for r in range(cp_size)]
-            vs = [zigzag_shard(v, r, cp_size) for r in range(cp_size)]
-        else:
-            ks = [zigzag_shard_varlen(k, full_cu_seqlens, r, cp_size)[0] for r in range(cp_size)]
-            vs = [zigzag_shard_varlen(v, full_cu_seqlens, r, cp_size)[0] for r in range(cp_size)]
-        return cls(ks, vs)
+        """Shards full-sequence K and V for every rank with the zig-zag kernel, one launch each."""
+        return cls(zigzag_shard_all(k, cp_size, full_cu_seqlens), zigzag_shard_all(v, cp_size, full_cu_seqlens))
 
 
 _checked_cu = {}  # id(cu tensor) -> (weak reference, tensor version, longest sequence) of cu tables found even

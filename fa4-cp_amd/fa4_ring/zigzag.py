@@ -60,6 +60,31 @@ def _shard(x: torch.Tensor, cp_rank: int, cp_size: int, full_cu_dev, nseq: int) 
     return out
 
 
+def zigzag_shard_all(x: torch.Tensor, cp_size: int, full_cu_seqlens=None) -> List[torch.Tensor]:
+    """zigzag_shard (zigzag_shard_varlen with ``full_cu_seqlens``) of x for every rank, in one
+    launch: the cp_size local shards."""
+    lib = _lib.load()
+    _require(x.is_cuda, "zig-zag sharding runs on the GPU: x must be a device tensor")
+    _require(x.is_contiguous(), "x must be contiguous")
+    n, nseq, cu_dev = x.shape[0], 1, None
+    if full_cu_seqlens is None:
+        local_seqlen(n, cp_size)
+    else:
+        cu = _as_cu_list(full_cu_seqlens)
+        for a, b in zip(cu, cu[1:]):
+            local_seqlen(b - a, cp_size)
+        _require(cu[0] == 0 and cu[-1] == n, "full_cu_seqlens must span x from row 0")
+        if len(cu) < 2:
+            return [x.new_empty((0,) + tuple(x.shape[1:])) for _ in range(cp_size)]
+        nseq, cu_dev = len(cu) - 1, _device_cu(full_cu_seqlens, x.device)
+    outs = [x.new_empty((n // cp_size,) + tuple(x.shape[1:])) for _ in range(cp_size)]
+    ptrs = (ctypes.c_void_p * cp_size)(*[o.data_ptr() for o in outs])
+    rc = lib.fa4cp_zigzag_shard_all(x.data_ptr(), ptrs, _row_bytes(x), _lib.ptr(cu_dev), nseq, n, cp_size,
+                                    _lib.stream_handle(x.device))
+    _lib.check(rc, "fa4cp_zigzag_shard_all")
+    return outs
+
+
 def zigzag_shard(x: torch.Tensor, cp_rank: int, cp_size: int) -> torch.Tensor:
     """Full [N, ...] sequence -> this rank's local [2h, ...] shard."""
     n = x.shape[0]

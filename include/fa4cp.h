@@ -413,6 +413,14 @@ typedef struct fa4cp_quant_args {
 int fa4cp_quantize_e4m3(const fa4cp_quant_args* args, void* stream);
 
 /*
+ * The same for `count` tensors (1..FA4CP_QUANT_MAX_TENSORS: a rank's q and every source's k and
+ * v) of one dtype, args[0..count), each with its own shape, strides, scales and workspace; in
+ * three launches altogether.  The results are those of `count` calls.
+ */
+#define FA4CP_QUANT_MAX_TENSORS 33
+int fa4cp_quantize_e4m3_many(const fa4cp_quant_args* args, int32_t count, void* stream);
+
+/*
  * fa4cp_quantize_e4m3 without the caller's workspace, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  No counterpart in the reference.  args->amax is ignored (may be NULL): the
@@ -438,6 +446,14 @@ int fa4cp_quantize_e4m3_noalloc(const fa4cp_quant_args* args, void* stream);
 int fa4cp_zigzag_shard(const void* src_full, void* dst_local, int64_t row_bytes,
                        const int32_t* full_cu, int32_t nseq, int64_t total_full,
                        int32_t cp_rank, int32_t cp_size, void* stream);
+
+/*
+ * fa4cp_zigzag_shard for every rank in one launch: dst_locals is a HOST array of cp_size device
+ * pointers (rank r's local tensor).
+ */
+int fa4cp_zigzag_shard_all(const void* src_full, void* const* dst_locals, int64_t row_bytes,
+                           const int32_t* full_cu, int32_t nseq, int64_t total_full, int32_t cp_size,
+                           void* stream);
 
 /*
  * Inverse of fa4cp_zigzag_shard over all ranks: shard_ptrs is a HOST array of cp_size

@@ -98,6 +98,30 @@ def test_quantize_strided_input():
     assert torch.equal(ds.cpu(), ds_ref) and torch.equal(y.view(torch.uint8).cpu(), y_ref)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_quantize_many_equals_single_calls(dtype):
+    """quantize_e4m3_many over tensors of unlike shapes, strides and scale groups (no rows, one row,
+    all zero, a strided head, 41 tensors: two launches' worth) gives the bytes and descales of one
+    call each; with a row of more than 2048 16-byte chunks among them too."""
+    from fa4_ring.fp8 import quantize_e4m3_many
+
+    say(f"quantize_e4m3_many {dtype}")
+    shapes = [(300, 8, 128, 0), (0, 2, 128, 1), (1, 2, 128, 1), (4097, 2, 64, 1), (64, 6, 128, 3), (33, 1, 256, 0)]
+    shapes += [(17 * i + 5, 2, 128, i % 2) for i in range(35)]
+    for wide in (False, True):
+        xs = [_heads_scaled(r, h, d, dtype, seed=i).to(DEV) for i, (r, h, d, _) in enumerate(shapes)]
+        groups = [g for *_, g in shapes]
+        xs[4] = torch.zeros_like(xs[4])
+        xs.append(_heads_scaled(70, 4, 136, dtype, seed=99).to(DEV)[:, :, :128])
+        groups.append(2)
+        if wide:
+            xs[2] = _heads_scaled(3, 96, 256 if dtype != torch.float32 else 128, dtype, seed=5).to(DEV)
+        for x, g, (y, ds) in zip(xs, groups, quantize_e4m3_many(xs, heads_per_scale=groups)):
+            y1, ds1 = quantize_e4m3(x, heads_per_scale=g)
+            assert torch.equal(y.view(torch.uint8), y1.view(torch.uint8)) and torch.equal(ds, ds1), (x.shape, g)
+            assert ds.shape == ds1.shape
+
+
 def test_quantize_zero_and_empty():
     say("quantize_e4m3 all-zero and empty")
     y, ds = quantize_e4m3(torch.zeros(64, 2, 128, dtype=torch.bfloat16, device=DEV), heads_per_scale=1)

@@ -587,3 +587,26 @@ def test_attention_rejects_unsupported():
     w = torch.zeros(64, 2, 128, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(AssertionError, match="multiple"):
         fa4_attn(z, w, w, causal=True)
+
+
+@pytest.mark.parametrize("cp", [1, 2, 8])
+@pytest.mark.parametrize("shape,dtype", [((2, 64), torch.bfloat16), ((3, 5), torch.float16), ((7,), torch.uint8),
+                                         ((), torch.float32)])
+def test_zigzag_shard_all_equals_every_shard(shape, dtype, cp):
+    """One launch for every rank equals zigzag_shard rank by rank, bit for bit: rows of 16-, 4- and
+    1-byte units, one sequence and packed ones (an empty one among them)."""
+    from fa4_ring.zigzag import zigzag_shard, zigzag_shard_all, zigzag_shard_varlen
+
+    say(f"zigzag_shard_all rows {shape} {dtype} cp={cp}")
+    lens = [2 * cp * n for n in (37, 0, 1, 5)]
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    x = torch.randint(0, 255, (cu[-1], *shape), device=DEV).to(dtype)
+    for r, y in enumerate(zigzag_shard_all(x, cp)):
+        assert torch.equal(y, zigzag_shard(x, r, cp))
+    for r, y in enumerate(zigzag_shard_all(x, cp, cu)):
+        assert torch.equal(y, zigzag_shard_varlen(x, cu, r, cp)[0])
+    assert [y.shape for y in zigzag_shard_all(x[:0], cp)] == [(0, *shape)] * cp
+    with pytest.raises(AssertionError):
+        zigzag_shard_all(x[:2 * cp + 1], cp)
