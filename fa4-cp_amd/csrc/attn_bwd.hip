@@ -17,6 +17,9 @@
 // of src's keys.  dK / dV go to one buffer per source rank: this rank's contribution to that
 // source's gradient (a multi-GPU ring sends them back to their owners).
 //
+// Where the tiles of the last two kernels are few, several workgroups share one's blocks
+// (take_share) and the last of them sums the parts (merge_shares).
+//
 // Four launches:
 // * bwd_pack_kernel (HBM-bound): delta, and every 32-row block of Q and dO copied into the
 //   operand order of the dK / dV products, in rows and transposed;
@@ -41,6 +44,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "share_model.h"
 
 namespace fa4cp {
 namespace {
@@ -109,7 +113,85 @@ struct BwdParams {
   float scale;
   int accumulate;
   int n_tiles;  // row tiles (dq) or key tiles (dkdv) per sequence
+  // dq / dk / dv are stored in the input type (grad16) or in float32
+  int grad16;
+  // Up to ns workgroups share a tile's blocks, about `chunk` each (of a tile of at most top2
+  // blocks, about chunk2): the partial sums of workgroup b's
+  // share i are in slot ns b + i of `part` (a workgroup's accumulators, in lane order) and done[b]
+  // counts the shares that finished (zero between launches).
+  int ns, chunk, top2, chunk2;
+  float* part;
+  unsigned* done;
+  int clear_words;  // words bwd_pack_kernel sets to zero: both kernels' counters, from done on
 };
+
+// Cache policy sc1 (agent scope): stores go through to the memory that every XCD sees, loads
+// are not served from a stale line of this XCD's L2.
+constexpr int kAgent = 16;
+
+// The share of a tile's n blocks that workgroup i of the launch's ns takes: [lo, hi), of `shares`;
+// false: the tile has fewer shares.
+__device__ __forceinline__ bool take_share(const BwdParams& p, int i, int n, int& lo, int& hi, int& shares) {
+  const int chunk = n > p.top2 ? p.chunk : p.chunk2;
+  shares = max(1, min(p.ns, (n + chunk - 1) / chunk));
+  lo = n * i / shares;
+  hi = n * (i + 1) / shares;
+  return i < shares;
+}
+
+// The shares of tile b meet here: every wavefront below `waves` leaves its accumulators in the
+// share's slot, and the last workgroup to finish sums all of them in order (the same bits whoever
+// is last).  Returns whether this one is the last: acc then holds the tile's sums.
+template <int NDT>
+__device__ __forceinline__ bool merge_shares(const BwdParams& p, int b, int i, int shares, int waves,
+                                             f32x16 (&acc)[NDT]) {
+  if (shares == 1) return true;
+  __shared__ int last;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int slot_bytes = waves * NDT * 4096, at = wave * NDT * 4096 + 16 * (int)(threadIdx.x & 63);
+  const char* slots = reinterpret_cast<const char*>(p.part) + (int64_t)b * p.ns * slot_bytes;
+  if (wave < waves) {
+    const auto r = make_rsrc32(uniform_ptr(slots + (int64_t)i * slot_bytes), slot_bytes);
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 v = {acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]};
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, at + 1024 * (4 * dt + g), 0, kAgent);
+      }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    last = atomicAdd(p.done + b, 1u) == (unsigned)shares - 1u;
+    if (last) atomicExch(p.done + b, 0u);
+  }
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(last) == 0) return false;
+  if (wave >= waves) return true;
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) acc[dt] = f32x16{};
+  for (int j = 0; j < shares; ++j) {
+    const auto r = make_rsrc32(uniform_ptr(slots + (int64_t)j * slot_bytes), slot_bytes);
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 v =
+            __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at + 1024 * (4 * dt + g), 0, kAgent));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[dt][4 * g + e] += v[e];
+      }
+  }
+  return true;
+}
+
+// One element of a gradient tensor: float32 (added to what is there with `accumulate`) or T.
+template <typename T>
+__device__ __forceinline__ void put_grad(const BwdParams& p, float* base, int64_t at, float x) {
+  if (p.grad16) reinterpret_cast<T*>(base)[at] = (T)x;
+  else base[at] = p.accumulate ? base[at] + x : x;
+}
 
 // Which local rows attend which keys of source `src` (one sequence of L rows): keys
 // [0, key_lim), rows [row_min, L), and key <= row when causal.
@@ -161,6 +243,7 @@ __global__ __launch_bounds__(256) void bwd_pack_kernel(BwdParams p) {
   __shared__ __align__(16) T ql[kBwdRows * RS];
   __shared__ __align__(16) T dl[kBwdRows * RS];
   __shared__ float dsum[kBwdRows];
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < p.clear_words; i += (int64_t)gridDim.x * 256) p.done[i] = 0u;
   int b = blockIdx.x;
   const int hq = b % p.h_q;
   b /= p.h_q;
@@ -459,12 +542,9 @@ __global__ __launch_bounds__(128 * HP) void bwd_dq_pair_kernel(BwdParams p) {
   for (int r = 0; r < 16; ++r) {
     const int row = r0 + 8 * (r >> 2) + 4 * h + (r & 3);
     if (row >= L) continue;
-    float* o = p.dq + ((int64_t)(qs + row) * p.h_q + head) * D + lq;
+    const int64_t at = ((int64_t)(qs + row) * p.h_q + head) * D + lq;
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-      const float x = acc[dt][r] * p.scale;
-      o[32 * dt] = p.accumulate ? o[32 * dt] + x : x;
-    }
+    for (int dt = 0; dt < NDT; ++dt) put_grad<T>(p, p.dq, at + 32 * dt, acc[dt][r] * p.scale);
   }
 }
 
@@ -507,10 +587,14 @@ __global__ __launch_bounds__(512) void bwd_dq_pp_kernel(BwdParams p) {
   };
 
   // longest first: the back-half row tiles attend the later sources and come out first
+  // (head groups fastest: with eight of them an XCD keeps to one, whose key blocks its L2 serves)
   const int n_hg = p.h_q / HP;
   int b = blockIdx.x;
   const int hg = b % n_hg;
   b /= n_hg;
+  const int share = b % p.ns;
+  b /= p.ns;
+  const int tile = b * n_hg + hg;
   const int rt = p.n_tiles - 1 - b % p.n_tiles;
   const int seq = b / p.n_tiles;
   const int64_t pstart = vt_seq_start(p.cu, seq, p.total, FA4CP_SEL_ALL) / kBwdRows;
@@ -553,8 +637,13 @@ __global__ __launch_bounds__(512) void bwd_dq_pp_kernel(BwdParams p) {
     if (r_end <= sp.row_min) return 0;
     return sp.causal ? min(sp.key_lim, r_end) : sp.key_lim;
   };
-  int n_blk = 0;
-  for (int s = 0; s < p.S; ++s) n_blk += (key_end_of(s) + kBwdRows - 1) / kBwdRows;
+  int lo, hi, shares;
+  {
+    int n = 0;
+    for (int s = 0; s < p.S; ++s) n += (key_end_of(s) + kBwdRows - 1) / kBwdRows;
+    if (!take_share(p, share, n, lo, hi, shares)) return;
+  }
+  const int n_blk = hi - lo;  // this workgroup's
   struct Cursor {
     int s, k0, kend;
   };
@@ -565,8 +654,23 @@ __global__ __launch_bounds__(512) void bwd_dq_pp_kernel(BwdParams p) {
       if (cu.s < p.S) cu.kend = key_end_of(cu.s);
     }
   };
-  Cursor lc{0, 0, key_end_of(0)};  // the next block to load
-  settle(lc);
+  auto seek = [&]() {  // block lo
+    Cursor cu{0, 0, key_end_of(0)};
+    settle(cu);
+    for (int x = lo; x > 0;) {
+      const int n = (cu.kend + kBwdRows - 1) / kBwdRows;
+      if (x < n) {
+        cu.k0 = kBwdRows * x;
+        break;
+      }
+      x -= n;
+      cu.k0 = cu.kend;
+      settle(cu);
+      if (cu.s >= p.S) break;
+    }
+    return cu;
+  };
+  Cursor lc = seek();  // the next block to load
   // this wavefront's share of the block at cursor lc into stage bi % 4: fragments w + 8 j
   auto load = [&](int bi) {
     const char* g = p.pkv + (((int64_t)src_of(lc.s) * p.h_kv + kvh) * p.n_pb + pstart + lc.k0 / kBwdRows) * KB;
@@ -582,8 +686,7 @@ __global__ __launch_bounds__(512) void bwd_dq_pp_kernel(BwdParams p) {
   };
   auto frag_at = [&](const char* st, int off) { return *reinterpret_cast<const frag*>(st + off + 16 * l); };
 
-  Cursor cc{0, 0, key_end_of(0)};  // the block of the wavefront's MFMA phase
-  settle(cc);
+  Cursor cc = seek();  // the block of the wavefront's MFMA phase
   frag ds0 = {}, ds1 = {};  // dS of the block before (A operands of dQ)
   f32x16 st = {}, dpt = {};
   // Every block the workgroup loads meets some row of the workgroup, not necessarily one of
@@ -698,18 +801,67 @@ __global__ __launch_bounds__(512) void bwd_dq_pp_kernel(BwdParams p) {
   wg_barrier();
   if (grp == 0) wg_barrier();  // both groups pass the same number of barriers
   __builtin_amdgcn_s_waitcnt(kWaitAll);
+  if (!merge_shares<NDT>(p, tile, share, shares, 8, acc)) return;
   // accumulator register r of lane l: query row 8 (r / 4) + 4h + r % 4, column 32 dt + lq
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int row = wr0 + 8 * (r >> 2) + 4 * h + (r & 3);
     if (row >= L) continue;
-    float* o = p.dq + ((int64_t)(qs + row) * p.h_q + head) * D + lq;
+    const int64_t at = ((int64_t)(qs + row) * p.h_q + head) * D + lq;
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-      const float x = acc[dt][r] * p.scale;
-      o[32 * dt] = p.accumulate ? o[32 * dt] + x : x;
+    for (int dt = 0; dt < NDT; ++dt) put_grad<T>(p, p.dq, at + 32 * dt, acc[dt][r] * p.scale);
+  }
+}
+
+// Workgroup b of the dK / dV kernel: its share, tile (the slot number), key tile, sequence, kv head
+// and source.  Longest first: the earlier sources' front halves (every row attends them), the
+// first half of the own key tiles (a tile's causal rows fall from all to none), the later
+// sources (the back-half rows), the rest of the own tiles, and the earlier sources' back
+// halves (no row; zeros are written).  The XCDs take the workgroups in turn, so within a class
+// of equal tiles the key tiles of one kv head are consecutive (the XCDs then stream the same query
+// blocks at a time), and the own tiles, of falling length, go kv head by kv head, so that every
+// XCD gets its share of each length.  With the sources in order and key tiles fastest everywhere
+// an XCD had the same own tiles of all heads, and long ones came last: dk / dv 335-342 us at 8192
+// tokens (H 32/8, cp 4, rank 1), where the workgroups' times add up to 220 us a CU; now 304-316.
+// The whole backward at 32768 tokens (cp 8, rank 3): 3997 -> 3498 us.
+__device__ __forceinline__ void dkdv_tile(const BwdParams& p, int b, int ns, int& share, int& tile, int& kt, int& seq,
+                                          int& kvh, int& src) {
+  const int per_kt = p.nseq * p.h_kv, late = p.S - 1 - p.rank;
+  const int front = min(p.n_tiles, ((p.max_seqlen >> 1) + kDkdvKeys - 1) / kDkdvKeys), own = (p.n_tiles + 1) / 2;
+  int n_src[5] = {p.rank, 1, late, 1, p.rank};
+  int n_kt[5] = {front, own, p.n_tiles, p.n_tiles - own, p.n_tiles - front};
+  int at = 0, c = 0, n = 0;  // tiles before class c, and its own
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    const int m = n_src[i] * n_kt[i] * per_kt;
+    if (c == i) {
+      n = m;
+      if (i < 4 && b >= ns * m) {
+        b -= ns * m;
+        at += m;
+        c = i + 1;
+      }
     }
   }
+  const int k = c == 0 ? front : c == 1 ? own : c == 2 ? p.n_tiles : c == 3 ? p.n_tiles - own : p.n_tiles - front;
+  share = b / n;
+  b -= share * n;
+  tile = at + b;
+  int r;
+  if (c == 1 || c == 3) {
+    src = p.rank;
+    kt = b / per_kt;
+    r = b - kt * per_kt;
+  } else {
+    const int s = b / (k * per_kt);
+    b -= s * k * per_kt;
+    r = b / k;
+    kt = b - r * k;
+    src = c == 2 ? p.rank + 1 + s : s;
+  }
+  kt += c == 3 ? own : c == 4 ? front : 0;
+  kvh = r / p.nseq;
+  seq = r - kvh * p.nseq;
 }
 
 // dK / dV: one workgroup per 128 keys of one source rank's sequence and kv head, eight
@@ -746,6 +898,7 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
   constexpr int R = pack_region_bytes<D>();
   constexpr int BB = pack_block_bytes<D>();
   constexpr bool HALVES = D > 128;
+  constexpr bool kShares = !HALVES;  // (at head dim 256 the kernel has no register to spare for them)
   constexpr int HB = 2 * R + 256;   // a half-stage: two regions and the per-row values
   // head dim 256: 1 KB fragments each wavefront loads per half-stage (below it the ninth
   // wavefront loads every fragment of a stage)
@@ -774,13 +927,8 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
   constexpr int OQ = 0, ODO = HALVES ? R : 2 * R, ODOT = HALVES ? 0 : R, OQT = HALVES ? R : 3 * R;
   constexpr int OVAL = HALVES ? 2 * R : 4 * R;
 
-  int b = blockIdx.x;
-  const int kt = b % p.n_tiles;
-  b /= p.n_tiles;
-  const int seq = b % p.nseq;
-  b /= p.nseq;
-  const int kvh = b % p.h_kv;
-  const int src = b / p.h_kv;
+  int share, tile, kt, seq, kvh, src;
+  dkdv_tile(p, blockIdx.x, kShares ? p.ns : 1, share, tile, kt, seq, kvh, src);
   const int64_t pstart = vt_seq_start(p.cu, seq, p.total, FA4CP_SEL_ALL) / kBwdRows;
   int qs, L;
   seq_range(p.cu, seq, p.total, FA4CP_SEL_ALL, qs, L);
@@ -798,6 +946,7 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
 #pragma unroll
   for (int i = 0; i < NDT; ++i) acc[i] = f32x16{};
 
+  int shares = 1;
   if (kb0 < sp.key_lim) {
     // K (first wavefront) or V (second) of the lane's key: B operands of S and dP
     frag kv[NKS];
@@ -815,13 +964,21 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
     // query rows that can see a key of this workgroup: from the first key on when causal
     const int row_begin = max(sp.row_min, sp.causal ? kb0 : 0) / kBwdRows * kBwdRows;
     const int n_rb = (L - row_begin + kBwdRows - 1) / kBwdRows;
-    const int n_blk = n_rb * p.group;  // (query head, 32-row block) pairs, head-major
+    // (query head, 32-row block) pairs, head-major: this workgroup's share of them, from `lo` on
+    int lo, hi;
+    if (kShares) {
+      if (!take_share(p, share, n_rb * p.group, lo, hi, shares)) return;
+    } else {
+      lo = 0;
+      hi = n_rb * p.group;
+    }
+    const int n_blk = hi - lo;
     const int64_t blk0 = pstart + row_begin / kBwdRows;
     // query head (within the group) and row block of the next block a load takes
     struct Cursor {
       int lh, lr;
     };
-    Cursor rc{0, 0}, tc{0, 0};
+    Cursor rc{lo / n_rb, lo % n_rb}, tc = rc;
     // head dim 256: the half of the block at cursor cu made of regions r0 and r0 + 2 into
     // half-stage st, then the per-row values
     auto load = [&](Cursor& cu, char* st, int r0) {
@@ -856,7 +1013,7 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
       constexpr bool PW = decltype(role)::value;
       frag pb0, pb1;  // first wavefront: P of the previous block (operands of dV)
       f32x16 dpt;     // second wavefront: dP of the previous block
-      int cr = 0;     // row block (within the head) of block i
+      int cr = lo % n_rb;  // row block (within the head) of block i
       load(rc, rows_of(0), 0);
       __builtin_amdgcn_s_waitcnt(kWaitAll);
       wg_barrier();
@@ -965,9 +1122,9 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
       // the next block to load (wave-uniform, advanced block by block: the blocks of one query
       // head are consecutive, the next head's start n_pb blocks after the previous one's)
       const char* gnext = reinterpret_cast<const char*>(
-          uniform_ptr(p.pk + ((int64_t)(kvh * p.group) * p.n_pb + blk0) * BB));
+          uniform_ptr(p.pk + ((int64_t)(kvh * p.group + lo / n_rb) * p.n_pb + blk0 + lo % n_rb) * BB));
       const int64_t head_jump = (int64_t)(p.n_pb - n_rb) * BB;
-      int lr = 0;
+      int lr = lo % n_rb;
       auto load_block = [&](char* st) __attribute__((always_inline)) {
         const __amdgpu_buffer_rsrc_t rs = make_rsrc32(gnext, BB);
         gnext += BB;
@@ -995,7 +1152,7 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
       constexpr bool PW = decltype(role)::value;
       frag pb0, pb1;  // first wavefront: P of the previous block (operands of dV)
       f32x16 dpt;     // second wavefront: dP of the previous block
-      int cr = 0;     // row block (within the head) of block i
+      int cr = lo % n_rb;  // row block (within the head) of block i
       wg_barrier();
       for (int i = 0; i <= n_blk; ++i) {
         const char* cur = stage_of(i);       // block i: its row regions
@@ -1074,11 +1231,14 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
       }
     }
   }
+  if constexpr (kShares) {
+    if (share >= shares || !merge_shares<NDT>(p, tile, share, shares, 8, acc)) return;
+  }
   // accumulator register r of lane l: head-dim element 32 dt + 8 (r / 4) + 4h + r % 4 of key
   // `key`; keys no query of this rank attends (past key_lim) get zeros
   if (producer || key >= L) return;
-  float* o = pwave ? p.dv[src] + ((int64_t)(qs + key) * p.h_kv + kvh) * D
-                   : p.dk[src] + ((int64_t)(qs + key) * p.h_kv + kvh) * D;
+  float* const base = pwave ? p.dv[src] : p.dk[src];
+  const int64_t at = ((int64_t)(qs + key) * p.h_kv + kvh) * D;
   const float sc = pwave ? 1.f : p.scale;
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt)
@@ -1086,15 +1246,111 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
     for (int g = 0; g < 4; ++g) {
       const int d = 32 * dt + 8 * g + 4 * h;
       f32x4 a = {acc[dt][4 * g] * sc, acc[dt][4 * g + 1] * sc, acc[dt][4 * g + 2] * sc, acc[dt][4 * g + 3] * sc};
-      if (p.accumulate) a += *reinterpret_cast<const f32x4*>(o + d);
-      *reinterpret_cast<f32x4*>(o + d) = a;
+      if (p.grad16) {
+        typedef T t4 __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<t4*>(reinterpret_cast<T*>(base) + at + d) = t4{(T)a[0], (T)a[1], (T)a[2], (T)a[3]};
+      } else {
+        float* const o = base + at + d;
+        if (p.accumulate) a += *reinterpret_cast<const f32x4*>(o);
+        *reinterpret_cast<f32x4*>(o) = a;
+      }
     }
 }
 
 
+// Tiles of the two gradient kernels and the workgroups that share one.
+struct BwdPlan {
+  int64_t dq_tiles = 0, kv_tiles = 0;
+  int dq_rows = 0;  // rows of a dq tile
+  Shares dq, kv;
+};
+
+// A 32-key block of dq takes 1.2 us and a 32-row block of dk / dv 1.02 (measured, head dim 128, the
+// chip full).  dq's row tiles are shared wherever best_shares finds it faster (backward, GPU time in
+// us, shares of the back-half / other row tiles: 8192 tokens, H 32/8, cp 4, rank 1: none 622, 2/1 584,
+// 2/2 564 (chosen), 3/2 589; 16384, cp 8, rank 3: 1098, 1046, 1000 (chosen), 1054; rank 7, equal row
+// tiles: 985 (chosen), 1071, 992, 1050).  dk / dv's key tiles only where all shares run at once: the
+// workgroups stream the query blocks in step, and shares at other blocks cost more in L2
+// misses than the even split gains (8192 tokens: none 622, two shares 628-651, three 634-650; 24576
+// tokens, H 16/2: 1311, 1337-1389), but 32 key tiles leave the chip idle (2048 tokens, H 8/2: 138,
+// 120, 113; four 112).
+BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
+  constexpr int kMaxTiles = 1024, kMaxSlots = 2048;  // slots of 128 KB at head dim 128
+  BwdPlan pl;
+  const int group = a.h_q / a.h_kv, nseq = a.cu ? a.nseq : 1;
+  const int hp = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+  const int longest = a.cu ? std::min(a.max_seqlen, a.total) : a.total;
+  const int rows = a.d == 256 ? kBwdRows : kBwdRows * 2 * (4 / hp);
+  const int64_t row_tiles = (longest + rows - 1) / rows, key_tiles = (longest + kDkdvKeys - 1) / kDkdvKeys;
+  pl.dq_rows = rows;
+  pl.dq_tiles = nseq * row_tiles * (a.h_q / hp);
+  pl.kv_tiles = (int64_t)a.cp_size * a.h_kv * nseq * key_tiles;
+  if (longest <= 0) return pl;
+  const int L = nseq > 1 ? std::max(1, a.total / nseq) : longest;  // an average sequence when packed
+  const int late = a.cp_size - 1 - a.cp_rank;
+  auto blocks = [](int n) { return (n + kBwdRows - 1) / kBwdRows; };
+  if (a.d == 256) return pl;  // (its kernels have no register to spare for the shares)
+  if (pl.dq_tiles <= kMaxTiles) {
+    auto cost = [&](int len, int rt, bool back) {
+      return blocks(std::min((rt + 1) * rows, len)) + a.cp_rank * blocks(len / 2) + (back ? late * blocks(len) : 0);
+    };
+    const int rts = (L + rows - 1) / rows, fronts = late > 0 ? L / 2 / rows : 0;
+    ShareLoad w;
+    w.top = cost(longest, (int)row_tiles - 1, true);
+    w.avg = 0.5f * (cost(L, rts - 1, true) + cost(L, fronts, true));
+    w.n = (a.h_q / hp) * (rts - fronts) * nseq;
+    w.top2 = fronts ? cost(L, fronts - 1, false) : 0;
+    w.avg2 = fronts ? 0.5f * (w.top2 + cost(L, 0, false)) : 0.f;
+    w.n2 = (a.h_q / hp) * fronts * nseq;
+    w.us = 1.2f * a.d / 128.f;
+    w.merge = 5.f;
+    w.read = 1.25f * a.d / 128.f;
+    w.packed = nseq > 1;
+    w.free2 = true;
+    pl.dq = best_shares(w, std::min<int64_t>(kMaxShares, kMaxSlots / pl.dq_tiles));
+  }
+  if (2 * pl.kv_tiles <= kCus) {
+    // earlier sources: every row, the front half of the keys; own: half of the rows on average, the
+    // first half of the tiles three quarters; later sources: the back-half rows
+    const int kts = (L + kDkdvKeys - 1) / kDkdvKeys, own1 = (kts + 1) / 2;
+    const int early = a.cp_rank * ((L / 2 + kDkdvKeys - 1) / kDkdvKeys);
+    ShareLoad w;
+    w.top = blocks(longest) * group;
+    const float all = (float)(blocks(L) * group);
+    w.n = a.h_kv * nseq * (early + own1);
+    w.avg = all * (early + 0.75f * own1) / (early + own1);
+    w.top2 = (int)(0.5f * all);
+    w.n2 = a.h_kv * nseq * (late * kts + kts - own1);
+    w.avg2 = w.n2 ? all * (0.5f * late * kts + 0.25f * (kts - own1)) / (late * kts + kts - own1) : 0.f;
+    w.us = 1.02f * a.d / 128.f;
+    w.merge = 5.f;
+    w.read = 1.25f * a.d / 128.f;
+    w.packed = nseq > 1;
+    w.free2 = true;
+    pl.kv = best_shares(w, std::min<int64_t>(kMaxShares, kCus / pl.kv_tiles));
+  }
+  return pl;
+}
+// Their workspace: the counters (dq's tiles, then dk / dv's), then the slots of one kernel at a time.
+int64_t share_words(const BwdPlan& pl) { return (pl.dq.k > 1 || pl.kv.k > 1) ? pl.dq_tiles + pl.kv_tiles : 0; }
+int64_t share_count_bytes(const BwdPlan& pl) { return (share_words(pl) * 4 + 255) / 256 * 256; }
+int64_t share_bytes(const BwdPlan& pl, int d) {
+  if (share_words(pl) == 0) return 0;
+  const int64_t dq = pl.dq.k > 1 ? pl.dq_tiles * pl.dq.k : 0, kv = pl.kv.k > 1 ? pl.kv_tiles * pl.kv.k : 0;
+  return share_count_bytes(pl) + std::max(dq, kv) * 8 * 32 * d * 4;
+}
+
 template <typename T, int D>
-int launch_bwd(const BwdParams& base, const fa4cp_sweep_bwd_args& a, hipStream_t st) {
+int launch_bwd(const BwdParams& base, const BwdPlan& pl, hipStream_t st) {
   BwdParams p = base;
+  const bool shared = base.part != nullptr;
+  auto use = [&](const Shares& s) {
+    p.ns = shared ? s.k : 1;
+    p.chunk = shared ? s.chunk : 0x3fffffff;
+    p.top2 = shared ? s.top2 : 0;
+    p.chunk2 = s.chunk2;
+  };
+  p.clear_words = shared ? (int)share_words(pl) : 0;
   // delta and the packed Q / dO blocks
   p.n_tiles = (p.max_seqlen + kBwdRows - 1) / kBwdRows;
   if (p.n_tiles == 0) return FA4CP_OK;  // every sequence empty: nothing to launch
@@ -1103,7 +1359,8 @@ int launch_bwd(const BwdParams& base, const fa4cp_sweep_bwd_args& a, hipStream_t
   hipLaunchKernelGGL((bwd_pack_kernel<T, D>), dim3((unsigned)pack_blocks), dim3(256), 0, st, p);
   // dq
   const int hp = p.group % 4 == 0 ? 4 : p.group % 2 == 0 ? 2 : 1;
-  const int64_t dq_blocks = (int64_t)p.nseq * p.n_tiles * (p.h_q / hp);
+  use(pl.dq);
+  const int64_t dq_blocks = pl.dq_tiles * p.ns;
   if (dq_blocks > 0x7fffffffLL) return set_error(FA4CP_EINVAL, "ring_sweep_bwd: too many row tiles");
   if constexpr (D == 256) {  // the packed K / V blocks, then the paired kernel
     const int64_t kv_pack_blocks = (int64_t)p.S * p.h_kv * p.nseq * p.n_tiles;
@@ -1118,18 +1375,19 @@ int launch_bwd(const BwdParams& base, const fa4cp_sweep_bwd_args& a, hipStream_t
     const int64_t kv_pack_blocks = (int64_t)p.S * p.h_kv * p.nseq * p.n_tiles;
     if (kv_pack_blocks > 0x7fffffffLL) return set_error(FA4CP_EINVAL, "ring_sweep_bwd: too many key blocks");
     hipLaunchKernelGGL((bwd_pack_kv_kernel<T, D>), dim3((unsigned)kv_pack_blocks), dim3(256), 0, st, p);
-    const int rows = kBwdRows * 2 * (4 / hp);  // rows per workgroup
-    p.n_tiles = (p.max_seqlen + rows - 1) / rows;
-    const int64_t blocks = (int64_t)p.nseq * p.n_tiles * (p.h_q / hp);
+    p.n_tiles = (p.max_seqlen + pl.dq_rows - 1) / pl.dq_rows;
+    const dim3 grid((unsigned)dq_blocks);
     switch (hp) {
-      case 4: hipLaunchKernelGGL((bwd_dq_pp_kernel<T, D, 4>), dim3((unsigned)blocks), dim3(512), 0, st, p); break;
-      case 2: hipLaunchKernelGGL((bwd_dq_pp_kernel<T, D, 2>), dim3((unsigned)blocks), dim3(512), 0, st, p); break;
-      default: hipLaunchKernelGGL((bwd_dq_pp_kernel<T, D, 1>), dim3((unsigned)blocks), dim3(512), 0, st, p); break;
+      case 4: hipLaunchKernelGGL((bwd_dq_pp_kernel<T, D, 4>), grid, dim3(512), 0, st, p); break;
+      case 2: hipLaunchKernelGGL((bwd_dq_pp_kernel<T, D, 2>), grid, dim3(512), 0, st, p); break;
+      default: hipLaunchKernelGGL((bwd_dq_pp_kernel<T, D, 1>), grid, dim3(512), 0, st, p); break;
     }
   }
   // dk / dv
   p.n_tiles = (p.max_seqlen + kDkdvKeys - 1) / kDkdvKeys;
-  const int64_t kv_blocks = (int64_t)p.S * p.h_kv * p.nseq * p.n_tiles;
+  use(pl.kv);
+  if (shared) p.done += pl.dq_tiles;
+  const int64_t kv_blocks = pl.kv_tiles * p.ns;
   if (kv_blocks > 0x7fffffffLL) return set_error(FA4CP_EINVAL, "ring_sweep_bwd: too many key tiles");
   hipLaunchKernelGGL((bwd_dkdv_kernel<T, D>), dim3((unsigned)kv_blocks), dim3(D > 128 ? 512 : 576), 0, st, p);
   return check_launch("ring_sweep_bwd");
@@ -1164,7 +1422,21 @@ extern "C" int64_t fa4cp_ring_sweep_bwd_workspace_bytes(const fa4cp_sweep_bwd_ar
   return delta_bytes(a->total, a->h_q) + (int64_t)a->h_q * n_pb * block_bytes(a->d) + kv;
 }
 
+extern "C" int64_t fa4cp_ring_sweep_bwd_share_bytes(const fa4cp_sweep_bwd_args* a) {
+  const int64_t ok = fa4cp_ring_sweep_bwd_workspace_bytes(a);
+  if (ok < 0) return ok;
+  if (a->h_q % a->h_kv != 0 || a->cp_rank < 0 || a->cp_rank >= a->cp_size || (a->cu != nullptr && a->max_seqlen < 0))
+    return set_error(FA4CP_EINVAL, "ring_sweep_bwd_share_bytes: bad shape h_q=%d h_kv=%d cp_rank=%d", a->h_q, a->h_kv,
+                     a->cp_rank);
+  return share_bytes(bwd_plan(*a), a->d);
+}
+
 extern "C" int fa4cp_ring_sweep_bwd(const fa4cp_sweep_bwd_args* a, void* stream) {
+  return fa4cp_ring_sweep_bwd_shared(a, FA4CP_FP32, nullptr, 0, stream);
+}
+
+extern "C" int fa4cp_ring_sweep_bwd_shared(const fa4cp_sweep_bwd_args* a, int32_t grad_dtype, void* shares,
+                                           int64_t shares_bytes, void* stream) {
   clear_error();
   if (a == nullptr) return set_error(FA4CP_EINVAL, "ring_sweep_bwd: null args");
   if (a->total < 0 || a->h_q <= 0 || a->h_kv <= 0 || a->h_q % a->h_kv != 0)
@@ -1178,6 +1450,9 @@ extern "C" int fa4cp_ring_sweep_bwd(const fa4cp_sweep_bwd_args* a, void* stream)
     return set_error(FA4CP_EUNSUPPORTED, "ring_sweep_bwd: head dim %d (64 / 128 / 256)", a->d);
   if (a->cu != nullptr && a->nseq <= 0) return set_error(FA4CP_EINVAL, "ring_sweep_bwd: nseq must be >= 1 with cu");
   if (a->cu != nullptr && a->max_seqlen < 0) return set_error(FA4CP_EINVAL, "ring_sweep_bwd: negative max_seqlen");
+  if (grad_dtype != FA4CP_FP32 && (grad_dtype != a->dtype || a->accumulate != 0))
+    return set_error(FA4CP_EINVAL, "ring_sweep_bwd: grad_dtype %d (FP32, or without accumulate the inputs' %d)", grad_dtype,
+                     a->dtype);
   if (a->total == 0) return FA4CP_OK;
   if (!a->q || !a->dout || !a->out || !a->lse || !a->workspace || !a->dq)
     return set_error(FA4CP_EINVAL, "ring_sweep_bwd: null tensor or workspace");
@@ -1198,7 +1473,17 @@ extern "C" int fa4cp_ring_sweep_bwd(const fa4cp_sweep_bwd_args* a, void* stream)
                              a->v_row_stride, a->v_head_stride};
   for (int64_t s : strides) ok = ok && (s * esz) % 16 == 0;
   if (!ok) return set_error(FA4CP_EINVAL, "ring_sweep_bwd: tensors and their strides must be 16-byte aligned");
+  const BwdPlan pl = bwd_plan(*a);
+  const int64_t share_need = share_bytes(pl, a->d);
+  if (shares != nullptr && (shares_bytes < share_need || reinterpret_cast<uintptr_t>(shares) % 16 != 0))
+    return set_error(FA4CP_EINVAL, "ring_sweep_bwd: share workspace of %lld bytes at %p; %lld bytes, 16-byte aligned, needed",
+                     (long long)shares_bytes, shares, (long long)share_need);
   BwdParams p{};
+  p.grad16 = grad_dtype != FA4CP_FP32;
+  if (shares != nullptr && share_need > 0) {
+    p.done = reinterpret_cast<unsigned*>(shares);
+    p.part = reinterpret_cast<float*>(reinterpret_cast<char*>(shares) + share_count_bytes(pl));
+  }
   p.q = a->q;
   p.dout = a->dout;
   p.lse = a->lse;
@@ -1238,8 +1523,8 @@ extern "C" int fa4cp_ring_sweep_bwd(const fa4cp_sweep_bwd_args* a, void* stream)
   p.accumulate = a->accumulate != 0;
   hipStream_t st = (hipStream_t)stream;
   if (a->dtype == FA4CP_BF16)
-    return a->d == 256 ? launch_bwd<__bf16, 256>(p, *a, st)
-           : a->d == 128 ? launch_bwd<__bf16, 128>(p, *a, st) : launch_bwd<__bf16, 64>(p, *a, st);
-  return a->d == 256 ? launch_bwd<_Float16, 256>(p, *a, st)
-         : a->d == 128 ? launch_bwd<_Float16, 128>(p, *a, st) : launch_bwd<_Float16, 64>(p, *a, st);
+    return a->d == 256 ? launch_bwd<__bf16, 256>(p, pl, st)
+           : a->d == 128 ? launch_bwd<__bf16, 128>(p, pl, st) : launch_bwd<__bf16, 64>(p, pl, st);
+  return a->d == 256 ? launch_bwd<_Float16, 256>(p, pl, st)
+         : a->d == 128 ? launch_bwd<_Float16, 128>(p, pl, st) : launch_bwd<_Float16, 64>(p, pl, st);
 }

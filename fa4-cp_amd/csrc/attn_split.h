@@ -2,15 +2,17 @@
 #pragma once
 
 #include "common.h"
+#include "share_model.h"
 
 namespace fa4cp {
 
 struct SweepParams;
 
-// How a sweep is split (see SweepSplit); ns_back == ns_front == 1: not at all.
+// How a sweep is split (see SweepSplit).
 struct SplitPlan {
-  int chunk = 0, ns_back = 1, ns_front = 1, n_front = 0, n_row = 0, per_hg = 0;
-  bool split() const { return ns_back > 1 || ns_front > 1; }
+  Shares shares;
+  int ns_back = 1, ns_front = 1, n_front = 0, n_row = 0, per_hg = 0;
+  bool split() const { return shares.k > 1; }
 };
 
 // The plan for a sweep's shape (no pointer of `a` is followed).

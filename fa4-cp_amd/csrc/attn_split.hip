@@ -13,6 +13,7 @@
 
 #include "attn_kernels.h"
 #include "attn_split.h"
+#include "share_model.h"
 
 namespace fa4cp {
 namespace {
@@ -269,13 +270,10 @@ int64_t done_bytes(int64_t words) { return (words * 4 + 255) / 256 * 256; }
 
 }  // namespace
 
-// The number of shares is the one with the least estimated time, the unsplit sweep unless one
-// is 7 % faster.  The model (in key tiles of the launch): a workgroup costs its tiles plus
-// kOver for its start and end (Q, the first K / V^T tiles, the store of its share: 11.5 us); a
-// split adds its merge, a fixed part and the last workgroup's read of every share; the chip runs
-// 256 workgroups at a time, the row tiles that meet the later sources (about `ab` tiles each)
-// before the others (`af`).  Tiles last 1.65 us, at head dim 64 1 us.  It orders the measured
-// times of 15 shapes (one and four rings, D 64 / 128 / 256, 16 to 512 row tiles; GPU time, us):
+// The number of shares comes from best_shares' estimate: the row tiles that meet the later sources
+// (about `avg` key tiles each) before the others, 1.65 us a key tile (1 us at head dim 64), a merge
+// of 5 us plus 1.25 us per share and 128 columns.  It orders the measured times of 15 shapes
+// (one and four rings, D 64 / 128 / 256, 16 to 512 row tiles; GPU time, us):
 //   shares                                1     2     3     4     6     8
 //   2048 tokens, H 8/2, cp 4, rank 1     52    42    39    38    38    40   (chosen: 5)
 //   8192, H 32/8, cp 8, rank 3          144    96    88   107   103   116   (3)
@@ -285,7 +283,7 @@ int64_t done_bytes(int64_t words) { return (words * 4 + 255) / 256 * 256; }
 //   8192, e4m3, rank 3                  113    80    69    85    84   100   (3)
 //   16384, H 16/2, D 256, rank 3        476   301   278   353   335   400   (3)
 SplitPlan split_plan(const fa4cp_sweep_args* a) {
-  constexpr int kCus = 256, kMaxShares = 8, kMaxRowTiles = 1024;
+  constexpr int kMaxRowTiles = 1024, kMaxSlots = 2048;  // slots of 128 KB at head dim 128
   SplitPlan pl;
   const bool fp8 = a->dtype == FA4CP_E4M3;
   const int bn = fp8 ? (a->d == 256 ? 64 : 128) : (a->d == 256 ? 32 : 64);
@@ -310,48 +308,26 @@ SplitPlan split_plan(const fa4cp_sweep_args* a) {
   const int fronts = late_steps > 0 ? (L / 2) / rows : 0;
   const int top = cost(longest, (int)n_rt - 1, true);
   if (top > 1 << 20) return pl;
-  const float ab = 0.5f * (cost(L, rts - 1, true) + cost(L, fronts, true));
-  const float af = fronts ? 0.5f * (cost(L, fronts - 1, false) + cost(L, 0, false)) : 0.f;
   const int front_top = fronts ? cost(L, fronts - 1, false) : 0;
-  const int n_back = n_hg * (nseq > 1 ? (rts - fronts) * nseq : rts - fronts);
-  const int n_frontal = n_hg * (nseq > 1 ? fronts * nseq : fronts);
-  const float us = a->d == 64 ? 1.f : 1.65f;
-  const float over = 11.5f / us;
-  float one = 0.f, least = 0.f;
-  int best = 1;
-  for (int k = 1; k <= kMaxShares; ++k) {
-    const int chunk = (top + k - 1) / k;
-    const int kb = nseq > 1 ? std::max(1, std::min(k, ((int)ab + chunk - 1) / chunk)) : k;
-    const int kf = fronts ? std::max(1, std::min(k, (front_top + chunk - 1) / chunk)) : 1;
-    const float wb = ab / kb + over, wf = af / kf + over;
-    const int nb = n_back * kb, nf = n_frontal * kf;
-    const int q = nb / kCus, r = nb % kCus;
-    float t;
-    if (nb + nf <= kCus) {
-      t = std::max((float)top / k, (float)front_top / kf) + over;
-    } else if (nf == 0) {
-      t = q < 3 ? (q + (r > 0)) * wb : nb * wb / kCus + 0.5f * wb;
-    } else {
-      const int more = (int)(wb / wf) * (kCus - r);  // front workgroups that fit beside the last back ones
-      const float backs = (q + (r > 0)) * wb;
-      t = nf <= more ? std::max(backs, q * wb + (nf + kCus - r - 1) / (kCus - r) * wf)
-                     : std::max(backs, (nb * wb + nf * wf) / kCus + 0.5f * wf);
-    }
-    t = std::max(t, (float)top / k + over);
-    if (k > 1) t += (5.f + 1.25f * k * a->d / 128.f) / us;
-    if (k == 1) one = least = t;
-    else if (t < least) {
-      least = t;
-      best = k;
-    }
-  }
-  if (best == 1 || least > 0.93f * one) return pl;
-  pl.chunk = (top + best - 1) / best;
-  pl.ns_back = best;
+  ShareLoad w;
+  w.top = top;
+  w.avg = 0.5f * (cost(L, rts - 1, true) + cost(L, fronts, true));
+  w.n = n_hg * (rts - fronts) * nseq;
+  w.top2 = front_top;
+  w.avg2 = fronts ? 0.5f * (front_top + cost(L, 0, false)) : 0.f;
+  w.n2 = n_hg * fronts * nseq;
+  w.us = a->d == 64 ? 1.f : 1.65f;
+  w.merge = 5.f;
+  w.read = 1.25f * a->d / 128.f;
+  w.packed = nseq > 1;
+  w.free2 = false;
+  pl.shares = best_shares(w, std::min(kMaxShares, kMaxSlots / (int)(n_hg * n_row)));
+  if (pl.shares.k == 1) return pl;
   pl.n_row = (int)n_row;
+  pl.ns_back = pl.shares.k;
   if (nseq == 1 && fronts > 0) {
     pl.n_front = fronts;
-    pl.ns_front = std::max(1, std::min(best, (front_top + pl.chunk - 1) / pl.chunk));
+    pl.ns_front = pl.shares.k2;
   }
   pl.per_hg = ((pl.n_row - pl.n_front) * pl.ns_back + pl.n_front * pl.ns_front + 7) / 8 * 8;
   return pl;
@@ -370,7 +346,7 @@ int launch_split(const SweepParams& p, const SplitPlan& pl, void* ws, int dtype,
   sp.done = reinterpret_cast<unsigned*>(ws);
   sp.po = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + done_bytes(split_words(pl, p.n_hg)));
   sp.pl = sp.po + split_rows(pl, p.n_hg) * d;
-  sp.chunk = pl.chunk;
+  sp.chunk = pl.shares.chunk;
   sp.ns_back = pl.ns_back;
   sp.ns_front = pl.ns_front;
   sp.n_front = pl.n_front;

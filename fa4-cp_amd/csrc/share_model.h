@@ -1,0 +1,75 @@
+// How many workgroups should share one tile's work (a sweep's row tile, the backward's row or key
+// tile) where the tiles alone leave the chip idle or uneven.  Host code.
+#pragma once
+
+#include <algorithm>
+
+namespace fa4cp {
+
+constexpr int kCus = 256;     // workgroups the chip runs at a time (one per CU)
+constexpr int kMaxShares = 8;
+
+// Two classes of tiles, the long ones handed out first.  Work is counted in steps (key tiles,
+// 32-row blocks) of `us` microseconds.
+struct ShareLoad {
+  int top;            // steps of the longest tile
+  float avg;          // of the first class's average one
+  int n;              // tiles of the first class
+  int top2;           // the same of the second class (n2 = 0: none)
+  float avg2;
+  int n2;
+  float us;           // microseconds per step
+  float merge, read;  // merging k shares takes merge + k read microseconds
+  bool packed;        // tiles of several sequences, whose lengths only the device knows: the classes are guesses
+  bool free2;         // the second class's shares are chosen apart (false: chunks as long as the first one's)
+};
+
+// What best_shares chose: at most k workgroups for a tile, about `chunk` steps each; of a tile of
+// at most top2 steps k2, about chunk2 each.  k == 1: no tile is shared.
+struct Shares {
+  int k = 1, k2 = 1, chunk = 1, top2 = 0, chunk2 = 1;
+};
+
+// The shares with the least estimated time, none unless they are 7 % faster (15 % for packed
+// sequences).  A workgroup costs its steps plus 11.5 us for its start and end.
+inline Shares best_shares(const ShareLoad& w, int most = kMaxShares) {
+  const float over = 11.5f / w.us;
+  float one = 0.f, least = 0.f;
+  Shares best;
+  for (int k = 1; k <= most; ++k) {
+    const int chunk = (w.top + k - 1) / k;
+    const int k1 = w.packed ? std::max(1, std::min(k, ((int)w.avg + chunk - 1) / chunk)) : k;
+    const int tied = w.n2 ? std::max(1, std::min(k, (w.top2 + chunk - 1) / chunk)) : 1;
+    for (int k2 = w.free2 ? 1 : tied; k2 <= (w.free2 && w.n2 ? k : tied); ++k2) {
+      const float c1 = w.avg / k1 + over, c2 = w.avg2 / k2 + over;
+      const int n1 = w.n * k1, n2 = w.n2 * k2;
+      const int q = n1 / kCus, r = n1 % kCus;
+      const float longs = (q + (r > 0)) * c1;
+      float t;
+      if (n1 + n2 <= kCus) {
+        t = std::max((float)w.top / k, (float)w.top2 / k2) + over;
+      } else if (n2 == 0) {
+        t = q < 3 ? longs : n1 * c1 / kCus + 0.5f * c1;
+      } else {
+        const int beside = (int)(c1 / c2) * (kCus - r);  // second-class workgroups that fit beside the last first-class ones
+        t = n2 <= beside ? std::max(longs, q * c1 + (n2 + kCus - r - 1) / (kCus - r) * c2)
+                         : std::max(longs, (n1 * c1 + n2 * c2) / kCus + 0.5f * c2);
+      }
+      t = std::max(t, (float)w.top / k + over);
+      if (k > 1) t += (w.merge + w.read * k) / w.us;
+      if (k == 1) one = least = t;
+      else if (t < least) {
+        least = t;
+        best.k = k;
+        best.k2 = k2;
+      }
+    }
+  }
+  if (least > (w.packed ? 0.85f : 0.93f) * one) return Shares{};
+  best.chunk = (w.top + best.k - 1) / best.k;
+  best.top2 = w.free2 && w.n2 ? w.top2 : 0;
+  best.chunk2 = std::max(1, (w.top2 + best.k2 - 1) / best.k2);
+  return best;
+}
+
+}  // namespace fa4cp

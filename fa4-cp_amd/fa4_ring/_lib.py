@@ -294,6 +294,9 @@ SIGNATURES = {
     ),
     "fa4cp_ring_sweep_bwd": (ctypes.c_int, [ctypes.POINTER(SweepBwdArgs), ctypes.c_void_p]),
     "fa4cp_ring_sweep_bwd_workspace_bytes": (ctypes.c_int64, [ctypes.POINTER(SweepBwdArgs)]),
+    "fa4cp_ring_sweep_bwd_shared": (
+        ctypes.c_int, [ctypes.POINTER(SweepBwdArgs), ctypes.c_int32, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
+    "fa4cp_ring_sweep_bwd_share_bytes": (ctypes.c_int64, [ctypes.POINTER(SweepBwdArgs)]),
     "fa4cp_quantize_e4m3": (ctypes.c_int, [ctypes.POINTER(QuantArgs), ctypes.c_void_p]),
     "fa4cp_quantize_e4m3_many": (ctypes.c_int, [ctypes.POINTER(QuantArgs), ctypes.c_int32, ctypes.c_void_p]),
     "fa4cp_quantize_e4m3_noalloc": (ctypes.c_int, [ctypes.POINTER(QuantArgs), ctypes.c_void_p]),

@@ -46,6 +46,14 @@ def ring_flash_attn_backward(dout: torch.Tensor, local_q: torch.Tensor, local_k:
     ``return_lse=True``) for one rank: (dq, dk per source rank, dv per source rank), float32.
     ``dq`` / ``dk`` / ``dv`` may be given (float32, contiguous); with ``accumulate`` the
     gradients are added to them."""
+    return _backward(dout, local_q, local_k, local_v, out, lse, cfg, group, cu_seqlens, max_seqlen, dq, dk, dv,
+                     accumulate, torch.float32)
+
+
+def _backward(dout, local_q, local_k, local_v, out, lse, cfg, group, cu_seqlens, max_seqlen, dq, dk, dv, accumulate,
+              grad_dtype):
+    """ring_flash_attn_backward with gradients of ``grad_dtype``: float32, or the inputs' type (the
+    kernels round their float32 sums once; not with ``accumulate``)."""
     lib = _lib.load()
     S, rank = cfg.cp_size, cfg.cp_rank
     total, h_q, d = local_q.shape
@@ -82,9 +90,9 @@ def ring_flash_attn_backward(dout: torch.Tensor, local_q: torch.Tensor, local_k:
 
     def buf(x, shape, what):
         if x is None:
-            return (torch.zeros if accumulate else torch.empty)(shape, dtype=torch.float32, device=dev)
-        _require(x.shape == shape and x.dtype == torch.float32 and x.is_contiguous() and x.device == dev,
-                 f"{what} must be a contiguous float32 tensor of shape {tuple(shape)} on {dev}")
+            return (torch.zeros if accumulate else torch.empty)(shape, dtype=grad_dtype, device=dev)
+        _require(x.shape == shape and x.dtype == grad_dtype and x.is_contiguous() and x.device == dev,
+                 f"{what} must be a contiguous {str(grad_dtype)[6:]} tensor of shape {tuple(shape)} on {dev}")
         return x
 
     dq = buf(dq, (total, h_q, d), "dq")
@@ -112,10 +120,15 @@ def ring_flash_attn_backward(dout: torch.Tensor, local_q: torch.Tensor, local_k:
     a.accumulate = 1 if accumulate else 0
     ws_bytes = lib.fa4cp_ring_sweep_bwd_workspace_bytes(ctypes.byref(a))
     _lib.check(int(min(ws_bytes, 0)), "fa4cp_ring_sweep_bwd_workspace_bytes")
-    # delta and the packed q / dout blocks (caching allocator blocks are 512-byte aligned)
+    # delta and the packed q / dout blocks, then the parts of tiles that several workgroups share
+    # (caching allocator blocks are 512-byte aligned)
+    share_bytes = lib.fa4cp_ring_sweep_bwd_share_bytes(ctypes.byref(a))
+    _lib.check(int(min(share_bytes, 0)), "fa4cp_ring_sweep_bwd_share_bytes")
     ws = torch.empty((max(int(ws_bytes), 1),), dtype=torch.uint8, device=dev)
+    shares = torch.empty((share_bytes,), dtype=torch.uint8, device=dev) if share_bytes else None
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes
-    _lib.check(lib.fa4cp_ring_sweep_bwd(ctypes.byref(a), _lib.stream_handle(dev)), "fa4cp_ring_sweep_bwd")
+    _lib.check(lib.fa4cp_ring_sweep_bwd_shared(ctypes.byref(a), _lib.dtype_code(grad_dtype), _lib.ptr(shares), share_bytes,
+                                               _lib.stream_handle(dev)), "fa4cp_ring_sweep_bwd")
     return dq, dk, dv
 
 
@@ -138,9 +151,9 @@ class _RingAttention(torch.autograd.Function):
         cfg = ctx.cfg
         S = cfg.cp_size
         ring = LocalKVRing(kv[:S], kv[S:])
-        dq, dk, dv = ring_flash_attn_backward(dout.contiguous(), q, ring.k[cfg.cp_rank], ring.v[cfg.cp_rank], out, lse,
-                                              cfg, group=ring, cu_seqlens=ctx.cu, max_seqlen=ctx.max_seqlen)
-        return (dq.to(q.dtype), None, None, None, *[g.to(q.dtype) for g in dk], *[g.to(q.dtype) for g in dv])
+        dq, dk, dv = _backward(dout.contiguous(), q, ring.k[cfg.cp_rank], ring.v[cfg.cp_rank], out, lse, cfg, ring, ctx.cu,
+                               ctx.max_seqlen, None, None, None, False, q.dtype)
+        return (dq, None, None, None, *dk, *dv)
 
 
 def ring_flash_attn_func(local_q: torch.Tensor, ring: LocalKVRing, cfg: RingConfig, *,

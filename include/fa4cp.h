@@ -345,6 +345,19 @@ int fa4cp_ring_sweep_bwd(const fa4cp_sweep_bwd_args* args, void* stream);
 int64_t fa4cp_ring_sweep_bwd_workspace_bytes(const fa4cp_sweep_bwd_args* args);
 
 /*
+ * fa4cp_ring_sweep_bwd with gradients of grad_dtype: FA4CP_FP32, or args->dtype (dq, dk and dv are
+ * then tensors of the inputs' type, the float32 sums rounded once; without accumulate), and
+ * with a second workspace of fa4cp_ring_sweep_bwd_share_bytes(args) bytes, 16-byte aligned (NULL:
+ * none): where the gradient kernels' tiles are too few to fill the chip, that is above 0 and
+ * several workgroups share a tile, their float32 parts summed there in a fixed order.  It
+ * holds nothing across calls.
+ */
+int fa4cp_ring_sweep_bwd_shared(const fa4cp_sweep_bwd_args* args, int32_t grad_dtype, void* shares,
+                                int64_t share_bytes, void* stream);
+/* Reads args' shape only; a negative FA4CP_E* code for a bad one. */
+int64_t fa4cp_ring_sweep_bwd_share_bytes(const fa4cp_sweep_bwd_args* args);
+
+/*
  * In-place online-softmax merge (flashinfer.cascade.merge_state_in_place semantics, natural
  * log LSE):
  *     m = max(s, s_o);  w = e^(s-m);  w_o = e^(s_o-m)

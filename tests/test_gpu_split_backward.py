@@ -1,0 +1,91 @@
+"""The backward where several workgroups share a tile, and its gradients in the inputs' type
+(fa4cp_ring_sweep_bwd_shared).
+
+The shared sums are the unshared ones' float32 terms in another order: every partial sum of n terms is
+off by at most n 2^-24 of the sum of their magnitudes, far below the 1e-5 of the largest gradient
+allowed here.  The gradients in 16 bits are the float32 ones rounded once, so they equal them
+bit for bit after that rounding."""
+
+import ctypes
+
+import pytest
+import torch
+
+from fa4_ring import LocalKVRing, RingConfig, _lib, ring_flash_attn, ring_flash_attn_backward, ring_flash_attn_func
+from fa4_ring.backward import _backward
+from gpu_helpers import DEV, say
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # (local lens, H, H_kv, D, cp, rank, dtype, shared)
+    ([512], 8, 2, 128, 4, 1, torch.bfloat16, True),    # dq and dk / dv shared
+    ([386], 4, 4, 64, 8, 2, torch.float16, True),      # one query head per kv head, partial blocks
+    ([1024], 8, 2, 128, 2, 0, torch.bfloat16, True),   # no earlier source
+    ([640], 16, 2, 128, 8, 7, torch.float16, True),    # no later source
+    ([1024, 66, 0, 514], 4, 1, 128, 8, 3, torch.bfloat16, True),  # packed
+    ([2048], 16, 4, 64, 4, 1, torch.bfloat16, True),   # dq alone
+    ([512], 8, 2, 256, 4, 1, torch.bfloat16, False),   # head dim 256: not shared
+    ([2], 4, 2, 128, 4, 2, torch.bfloat16, False),
+]
+
+
+@pytest.mark.parametrize("lens,h,h_kv,d,cp,rank,dtype,shared", CASES)
+def test_shared_backward(lens, h, h_kv, d, cp, rank, dtype, shared, monkeypatch):
+    say(f"shared backward lens={lens} h={h}/{h_kv} d={d} cp={cp} rank={rank} {dtype}")
+    g = torch.Generator(device="cuda").manual_seed(23)
+    total, packed = sum(lens), len(lens) > 1
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=DEV) if packed else None
+    kw = dict(cu_seqlens=cu, max_seqlen=max(lens) if packed else None)
+    mk = lambda hh: torch.randn(total, hh, d, generator=g, device=DEV).to(dtype)  # noqa: E731
+    q, dout = mk(h), mk(h)
+    ring = LocalKVRing([mk(h_kv) for _ in range(cp)], [mk(h_kv) for _ in range(cp)])
+    cfg = RingConfig(cp_size=cp, cp_rank=rank)
+    lk, lv = ring.kv(rank)
+    out, lse = ring_flash_attn(q, lk, lv, cfg, group=ring, return_lse=True, **kw)
+
+    a = _lib.SweepBwdArgs()
+    a.total, a.h_q, a.h_kv, a.d, a.cp_rank, a.cp_size = total, h, h_kv, d, rank, cp
+    if packed:
+        a.cu, a.nseq, a.max_seqlen = cu.data_ptr(), len(lens), max(lens)
+    lib = _lib.load()
+    need = lib.fa4cp_ring_sweep_bwd_share_bytes(ctypes.byref(a))
+    assert (need > 0) == shared
+
+    def grads(dt=torch.float32):
+        r = _backward(dout, q, lk, lv, out, lse, cfg, ring, cu, kw["max_seqlen"], None, None, None, False, dt)
+        return [r[0], *r[1], *r[2]]
+
+    got = grads()
+    for _ in range(6):  # the same bits every time, whichever workgroup sums
+        assert all(torch.equal(x, y) for x, y in zip(grads(), got))
+    for x, y in zip(grads(dtype), got):
+        assert x.dtype == dtype and torch.equal(x, y.to(dtype))
+    # unshared: the entry point without the second workspace
+    monkeypatch.setattr(lib, "fa4cp_ring_sweep_bwd_share_bytes", lambda _: 0)  # (an attribute of the loaded library)
+    for x, y in zip(grads(), got):
+        assert (x - y).abs().max() <= 1e-5 * max(1e-3, float(x.abs().max()))
+    monkeypatch.undo()
+    # adding to what is there
+    base = [torch.randn(x.shape, generator=g, device=DEV) for x in got]
+    acc = [b.clone() for b in base]
+    ring_flash_attn_backward(dout, q, lk, lv, out, lse, cfg, group=ring, dq=acc[0], dk=acc[1:1 + cp], dv=acc[1 + cp:],
+                             accumulate=True, **kw)
+    for x, b, y in zip(acc, base, got):
+        assert torch.equal(x, b + y)
+    with pytest.raises(RuntimeError, match="grad_dtype"):
+        _backward(dout, q, lk, lv, out, lse, cfg, ring, cu, kw["max_seqlen"], None, None, None, True, dtype)
+
+
+def test_autograd_gradients_are_the_rounded_ones():
+    say("autograd gradients in the inputs' type")
+    g = torch.Generator(device="cuda").manual_seed(4)
+    mk = lambda hh: torch.randn(512, hh, 128, generator=g, device=DEV).to(torch.bfloat16).requires_grad_()  # noqa: E731
+    q, ks, vs = mk(8), [mk(2) for _ in range(4)], [mk(2) for _ in range(4)]
+    ring, cfg = LocalKVRing(ks, vs), RingConfig(cp_size=4, cp_rank=2)
+    out = ring_flash_attn_func(q, ring, cfg)
+    dout = torch.randn(out.shape, generator=g, device=DEV).to(torch.bfloat16)
+    got = torch.autograd.grad(out, [q, *ks, *vs], dout)
+    with torch.no_grad():
+        o, lse = ring_flash_attn(q, ks[2], vs[2], cfg, group=ring, return_lse=True)
+        dq, dk, dv = ring_flash_attn_backward(dout, q, ks[2], vs[2], o, lse, cfg, group=ring)
+    assert all(torch.equal(x, y.to(torch.bfloat16)) for x, y in zip(got, [dq, *dk, *dv]))
