@@ -136,14 +136,14 @@ def timed_sweeps(fn, steps: int, warmup: int, clock: KernelClock = None):
         fn()
     torch.cuda.synchronize()
     saved = (RA.fa4_attn, RA.merge_state_in_place, RA.merge_states, RA.transpose_v, RA.launch_sweep,
-             RA.transpose_v_many)
+             RA.transpose_v_into)
     if clock is not None:
         RA.fa4_attn = clock.wrap("attn", saved[0])
         RA.merge_state_in_place = clock.wrap("merge_inplace", saved[1])
         RA.merge_states = clock.wrap("merge_states", saved[2])
         RA.transpose_v = clock.wrap("transpose_v", saved[3])
         RA.launch_sweep = clock.wrap("sweep_kernel", saved[4])
-        RA.transpose_v_many = clock.wrap("transpose_v_many", saved[5])
+        RA.transpose_v_into = clock.wrap("transpose_v_many", saved[5])
     try:
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -153,7 +153,7 @@ def timed_sweeps(fn, steps: int, warmup: int, clock: KernelClock = None):
         dt = (time.perf_counter() - t0) / steps
     finally:
         (RA.fa4_attn, RA.merge_state_in_place, RA.merge_states, RA.transpose_v, RA.launch_sweep,
-         RA.transpose_v_many) = saved
+         RA.transpose_v_into) = saved
     return dt
 
 
@@ -819,9 +819,10 @@ def main():
     value = flops / sec / 1e12
     sw_ms = clock.mean_ms("sweep_kernel")
     sw_tflops = flops / (sw_ms * 1e-3) / 1e12
-    # V -> V^T: every source's whole shard, read and written once, all 8 in one launch
+    # V -> V^T: every source's keys that the rank attends (of the earlier ones the front half),
+    # read and written once, all in one launch
     tr_ms = clock.mean_ms("transpose_v_many")
-    tr_bytes = CP * 2.0 * t_local * HKV * D * 2
+    tr_bytes = (CP - 0.5 * rank) * 2.0 * t_local * HKV * D * 2
 
     # ---------------- the reference's per-step sweep (attention + LSE merge per step)
     # the per-step form: its wall time unclocked (two events around each of its ~23 launches

@@ -111,6 +111,7 @@ class QuantArgs(ctypes.Structure):
 
 
 MAX_CP = 16  # FA4CP_MAX_CP
+Pointers = ctypes.c_void_p * MAX_CP  # one device address per source rank
 
 
 class SweepArgs(ctypes.Structure):
@@ -125,8 +126,8 @@ class SweepArgs(ctypes.Structure):
         ("o_row_stride", ctypes.c_int64),
         ("o_head_stride", ctypes.c_int64),
         ("lse_row_stride", ctypes.c_int64),
-        ("k", ctypes.c_void_p * MAX_CP),
-        ("v_t", ctypes.c_void_p * MAX_CP),
+        ("k", Pointers),
+        ("v_t", Pointers),
         ("k_row_stride", ctypes.c_int64),
         ("k_head_stride", ctypes.c_int64),
         ("vt_d_stride", ctypes.c_int64),
@@ -354,8 +355,14 @@ def dtype_code(dt: torch.dtype) -> int:
     return _DTYPE_CODE[dt]
 
 
+# the current stream's handle without the Stream object around it (0.2 us instead of 5)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(device: torch.device) -> int:
     """hipStream_t of torch's current stream on `device` (kernels are queued there)."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

@@ -96,12 +96,20 @@ def descale_table(ds, h_kv: int, device) -> torch.Tensor:
 def sweep_descales(q, ks, vs, h_kv: int, device):
     """The fused sweep's descales -> (q [h_kv], k [len(ks), h_kv], v [len(vs), h_kv]), float32
     rows of one contiguous table built by a single stack (one device copy per call instead of
-    three); a part given as None comes back None."""
+    three, two where every descale is a scalar); a part given as None comes back None."""
     parts = [[] if q is None else [q], list(ks or []), list(vs or [])]
-    views = [_descale_view(d, h_kv, device) for part in parts for d in part]
-    if not views:
+    flat = [d for part in parts for d in part]
+    if not flat:
         return None, None, None
-    table = torch.stack(views)
+    shape = flat[0].shape if torch.is_tensor(flat[0]) else None
+    if shape in ((), (h_kv,)) and all(torch.is_tensor(d) and d.shape == shape and d.dtype == torch.float32
+                                      and d.device == device for d in flat):
+        # (a view of each would take 7 us of host time per descale: 130 us for cp_size 8)
+        table = torch.stack(flat)
+        if shape == ():
+            table = table.view(-1, 1).repeat(1, h_kv)
+    else:
+        table = torch.stack([_descale_view(d, h_kv, device) for d in flat])
     out, row = [], 0
     for part, given in zip(parts, (q is not None, ks is not None, vs is not None)):
         out.append(table[row:row + len(part)] if given else None)
@@ -178,25 +186,28 @@ def transpose_v_many(vs: Sequence[torch.Tensor], *, cu_seqlens_k: Optional[torch
         _require(max_seqlen_k is not None, "max_seqlen_k required with cu_seqlens_k")
         nseq = cu_seqlens_k.shape[0] - 1
     stride = int(lib.fa4cp_vt_min_d_stride(t_k, nseq))
-    n = h_kv * d * stride  # (a multiple of 128: every slice of the one buffer is 128-byte aligned)
+    n = h_kv * d * stride  # (a multiple of 128: every part of the one buffer is 128-byte aligned)
     buf = torch.empty(len(vs) * n, dtype=v.dtype, device=v.device)
-    vts = list(buf.split(n)) if n else [buf for _ in vs]
-    a = _lib.TransposeArgs()
-    a.v_row_stride, a.v_head_stride = v.stride(0), v.stride(1)
-    a.cu_k = _lib.ptr(cu_seqlens_k)
-    a.nseq = nseq
-    a.total_k = t_k
-    a.max_seqlen_k = int(max_seqlen_k) if cu_seqlens_k is not None else t_k
-    a.k_sel = SEL_ALL
-    a.h_kv, a.d = h_kv, d
-    a.dtype = _lib.dtype_code(v.dtype)
-    a.vt_d_stride = stride
-    src = (ctypes.c_void_p * len(vs))(*[x.data_ptr() for x in vs])
-    dst = (ctypes.c_void_p * len(vs))(*[x.data_ptr() for x in vts])
-    words, n_words = (None, 0) if clear is None else (clear[0].data_ptr(), clear[1])
-    _lib.check(lib.fa4cp_transpose_v_ring(ctypes.byref(a), src, dst, len(vs), n_front, words, n_words,
-                                          _lib.stream_handle(v.device)), "fa4cp_transpose_v_ring")
-    return vts, stride
+    transpose_v_into(vs, buf.data_ptr(), stride, cu_seqlens_k, max_seqlen_k, n_front,
+                     *((None, 0) if clear is None else (clear[0].data_ptr(), clear[1])))
+    return list(buf.split(n)), stride
+
+
+def transpose_v_into(vs: Sequence[torch.Tensor], vt: int, stride: int, cu: Optional[torch.Tensor],
+                     max_seqlen: Optional[int], n_front: int, clear: Optional[int], clear_words: int) -> None:
+    """Queues transpose_v_many's launch into device memory at ``vt`` (the tensors' V^T one after the
+    other, row stride ``stride``), its arguments checked by the caller; ``clear``: the address
+    of the words to clear."""
+    v = vs[0]
+    t_k, h_kv, d = v.shape
+    rs, hs, _ = v.stride()
+    n = len(vs)
+    step = h_kv * d * stride * v.element_size()
+    a = _lib.TransposeArgs(None, rs, hs, _lib.ptr(cu), 1 if cu is None else cu.shape[0] - 1, t_k,
+                           t_k if cu is None else int(max_seqlen), SEL_ALL, h_kv, d, _lib.dtype_code(v.dtype), None, stride)
+    _lib.check(_lib.load().fa4cp_transpose_v_ring(
+        ctypes.byref(a), _lib.Pointers(*[x.data_ptr() for x in vs]), _lib.Pointers(*range(vt, vt + n * step, step)), n,
+        n_front, clear, clear_words, _lib.stream_handle(v.device)), "fa4cp_transpose_v_ring")
 
 
 def fa4_attn(

@@ -145,12 +145,19 @@ def transpose_v_paged_many(ring: PagedKVRing, total: int, cu_seqlens: Optional[t
     stride = int(lib.fa4cp_vt_min_d_stride(total, nseq))
     size = h_kv * d * stride
     buf = torch.empty(n * size, dtype=ring.v[0].dtype, device=ring.v[0].device)
-    vts = list(buf.split(size))
-    a = _paged_args(ring, total, cu_seqlens, max_seqlen)
+    transpose_v_paged_into(ring, total, buf.data_ptr(), stride, cu_seqlens, max_seqlen, n_front,
+                           *((None, 0) if clear is None else (clear[0].data_ptr(), clear[1])))
+    return list(buf.split(size)), stride
+
+
+def transpose_v_paged_into(ring: PagedKVRing, total: int, vt: int, stride: int, cu_seqlens: Optional[torch.Tensor],
+                           max_seqlen: Optional[int], n_front: int, clear: Optional[int], clear_words: int) -> None:
+    """Queues transpose_v_paged_many's launch into device memory at ``vt`` (the sources' V^T one after
+    the other, row stride ``stride``); ``clear``: the address of the words to clear."""
+    n, v = ring.cp_size, ring.v[0]
+    step = v.shape[2] * v.shape[3] * stride * v.element_size()
     arr = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])  # noqa: E731
-    words, n_words = (None, 0) if clear is None else (clear[0].data_ptr(), clear[1])
-    _lib.check(lib.fa4cp_transpose_v_paged_ring(ctypes.byref(a), arr(ring.v), arr(ring.page_tables), arr(vts),
-                                                stride, n, n_front, words, n_words,
-                                                _lib.stream_handle(ring.v[0].device)),
-               "fa4cp_transpose_v_paged_ring")
-    return vts, stride
+    _lib.check(_lib.load().fa4cp_transpose_v_paged_ring(
+        ctypes.byref(_paged_args(ring, total, cu_seqlens, max_seqlen)), arr(ring.v), arr(ring.page_tables),
+        (ctypes.c_void_p * n)(*range(vt, vt + n * step, step)), stride, n, n_front, clear, clear_words,
+        _lib.stream_handle(v.device)), "fa4cp_transpose_v_paged_ring")

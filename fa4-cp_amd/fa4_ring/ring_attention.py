@@ -37,9 +37,9 @@ import torch
 from . import _lib
 from .config import RingConfig
 from .fa4_backend import (SEL_ALL, SEL_BACK_HALF, SEL_FRONT_HALF, SUPPORTED_HEAD_DIMS, fa4_attn, kernel_head_dim,
-                          out_dtype_for, pad_head_dim, sweep_descales, transpose_v, transpose_v_many, uses_vt)
+                          out_dtype_for, pad_head_dim, sweep_descales, transpose_v, transpose_v_into, uses_vt)
 from .merge import merge_state_in_place, merge_states
-from .paged import PagedKVRing, gather_kv_pages, transpose_v_paged_many
+from .paged import PagedKVRing, gather_kv_pages, transpose_v_paged_into
 from .zigzag import zigzag_shard_all
 
 
@@ -312,21 +312,26 @@ def ring_sweep(local_q: torch.Tensor, local_k: torch.Tensor, local_v: torch.Tens
     _lib.load()  # fails here, before any allocation, without the library
     S, rank = cfg.cp_size, cfg.cp_rank
     total, h_q, d = local_q.shape
-    dev = local_q.device
-    assert local_q.is_cuda and local_q.stride(2) == 1, "local_q must be a device tensor, contiguous in D"
-    nseq = 1 if cu_seqlens is None else cu_seqlens.shape[0] - 1
+    dtype = local_q.dtype
+    q_stride = local_q.stride()
+    assert local_q.is_cuda and q_stride[2] == 1, "local_q must be a device tensor, contiguous in D"
     ks = [local_k if i == rank else group.k[i] for i in range(S)]
     vs = [local_v if i == rank else group.v[i] for i in range(S)]
     h_kv = ks[0].shape[1]
+    shape, k_stride, v_stride, v_dtype = (total, h_kv, d), ks[0].stride(), vs[0].stride(), vs[0].dtype
     for k, v in zip(ks, vs):
-        assert k.shape == (total, h_kv, d) and v.shape == k.shape and k.dtype == local_q.dtype
-        assert k.stride() == ks[0].stride(), "all K shards must share strides"
-        # the sweep's arguments carry K's row and head strides only: D must be contiguous
-        assert k.stride(2) == 1 and v.stride(2) == 1, "K and V shards must be contiguous in D"
-    assert all(v.stride() == vs[0].stride() for v in vs), "all V shards must share strides"
-    return _sweep_launch(local_q, [k.data_ptr() for k in ks], (ks[0].stride(0), ks[0].stride(1)), h_kv,
-                         lambda **kw: transpose_v_many(vs, cu_seqlens_k=cu_seqlens, max_seqlen_k=max_seqlen, **kw),
-                         cfg, cu_seqlens, max_seqlen, out, lse, descales)
+        assert k.shape == shape and v.shape == shape and k.dtype == dtype
+        assert k.stride() == k_stride, "all K shards must share strides"
+        assert v.stride() == v_stride and v.dtype == v_dtype, "all V shards must share strides and dtype"
+    # the sweep's arguments carry K's row and head strides only: D must be contiguous
+    assert k_stride[2] == 1 and v_stride[2] == 1, "K and V shards must be contiguous in D"
+    assert vs[0].device == local_q.device, f"V must be on {local_q.device}"
+
+    def transpose(*args):
+        transpose_v_into(vs, *args)
+
+    return _sweep_launch(local_q, q_stride, [k.data_ptr() for k in ks], k_stride, h_kv, transpose, v_dtype, cfg,
+                         cu_seqlens, max_seqlen, out, lse, descales)
 
 
 def ring_sweep_paged(local_q: torch.Tensor, cfg: RingConfig, ring: "PagedKVRing",
@@ -351,78 +356,78 @@ def ring_sweep_paged(local_q: torch.Tensor, cfg: RingConfig, ring: "PagedKVRing"
     kp.pt_stride = ring.page_tables[0].shape[1]
     kp.page_size = ring.page_size
     kp.num_pages = kc.shape[0]
+    assert ring.v[0].device == local_q.device, f"V must be on {local_q.device}"
+
+    def transpose(*args):
+        transpose_v_paged_into(ring, total, *args)
+
     # a cache is [num_pages, page_size, H_kv, D]: rows at stride(1), heads at stride(2)
-    return _sweep_launch(local_q, [k.data_ptr() for k in ring.k], (kc.stride(1), kc.stride(2)), kc.shape[2],
-                         lambda **kw: transpose_v_paged_many(ring, total, cu_seqlens, max_seqlen, **kw),
-                         cfg, cu_seqlens, max_seqlen, out, lse, descales, kpages=kp)
+    return _sweep_launch(local_q, local_q.stride(), [k.data_ptr() for k in ring.k], kc.stride()[1:], kc.shape[2],
+                         transpose, ring.v[0].dtype, cfg, cu_seqlens, max_seqlen, out, lse, descales, kpages=kp)
 
 
-def _sweep_launch(local_q: torch.Tensor, k_ptrs: List[int], k_strides: Tuple[int, int], h_kv: int,
-                  transpose, cfg: RingConfig, cu_seqlens: Optional[torch.Tensor],
+def _sweep_launch(local_q: torch.Tensor, q_stride: Tuple[int, ...], k_ptrs: List[int], k_stride: Tuple[int, ...],
+                  h_kv: int, transpose, v_dtype: torch.dtype, cfg: RingConfig, cu_seqlens: Optional[torch.Tensor],
                   max_seqlen: Optional[int], out: Optional[torch.Tensor], lse: Optional[torch.Tensor],
                   descales: Optional[Descales], kpages: Optional["_lib.SweepKPages"] = None) -> torch.Tensor:
-    """Queues `transpose` (every source's V^T as this rank reads it: transpose_v_many or its paged
-    form, given n_front and clear) and the sweep over every source rank's K (device addresses
-    `k_ptrs`, row and head strides `k_strides`) and V^T; with `kpages` the K addresses are the
-    sources' paged caches."""
+    """Queues `transpose` (every source's V^T as this rank reads it: transpose_v_into or its paged
+    form, given the address and row stride on) and the sweep over every source rank's K (device
+    addresses `k_ptrs`, row and head stride first in `k_stride`) and V^T; with `kpages` the K
+    addresses are the sources' paged caches."""
+    lib = _lib.load()
     S, rank = cfg.cp_size, cfg.cp_rank
     total, h_q, d = local_q.shape
     dev = local_q.device
-    nseq = 1 if cu_seqlens is None else cu_seqlens.shape[0] - 1
     e4m3 = local_q.dtype == torch.float8_e4m3fn
+    odt = torch.bfloat16 if e4m3 else local_q.dtype
     if out is None:
-        out = torch.empty(local_q.shape, dtype=torch.bfloat16 if e4m3 else local_q.dtype, device=dev)
+        out = torch.empty((total, h_q, d), dtype=odt, device=dev)
+    else:
+        assert out.shape == local_q.shape and out.dtype == odt and out.device == dev and out.stride(2) == 1, \
+            f"out must be [{total}, {h_q}, {d}] {odt} on {dev}, contiguous in D"
     qd = kd = vd = None
     if e4m3 and descales is not None:
         qd, kd, vd = sweep_descales(descales.q, None if descales.k is None else descales.k[:S],
                                     None if descales.v is None else descales.v[:S], h_kv, dev)
     if lse is None:
         lse = torch.empty((total, h_q), dtype=torch.float32, device=dev)
-    odt = torch.bfloat16 if e4m3 else local_q.dtype
-    assert out.shape == local_q.shape and out.dtype == odt and out.device == dev and out.stride(2) == 1, \
-        f"out must be [{total}, {h_q}, {d}] {odt} on {dev}, contiguous in D"
-    assert lse.shape == (total, h_q) and lse.dtype == torch.float32 and lse.device == dev and lse.stride(1) == 1, \
-        f"lse must be [{total}, {h_q}] float32 on {dev} with unit head stride"
+    else:
+        assert lse.shape == (total, h_q) and lse.dtype == torch.float32 and lse.device == dev and lse.stride(1) == 1, \
+            f"lse must be [{total}, {h_q}] float32 on {dev} with unit head stride"
+    nseq, longest = 1, total
     if cu_seqlens is not None:
-        assert cu_seqlens.dtype == torch.int32 and cu_seqlens.device == dev and cu_seqlens.is_contiguous(), \
-            "cu_seqlens must be contiguous int32 on the device"
+        assert cu_seqlens.dtype == torch.int32 and cu_seqlens.device == dev and cu_seqlens.is_contiguous() \
+            and cu_seqlens.dim() == 1 and cu_seqlens.shape[0] >= 2, "cu_seqlens must be contiguous int32 [num_seq + 1] on the device"
         assert max_seqlen is not None, "max_seqlen required when cu_seqlens is given"
-    a = _lib.SweepArgs()
-    a.q, a.out, a.lse = local_q.data_ptr(), out.data_ptr(), lse.data_ptr()
-    a.q_row_stride, a.q_head_stride = local_q.stride(0), local_q.stride(1)
-    a.o_row_stride, a.o_head_stride = out.stride(0), out.stride(1)
-    a.lse_row_stride = lse.stride(0)
-    for i in range(S):
-        a.k[i] = k_ptrs[i]
-    a.k_row_stride, a.k_head_stride = k_strides
-    a.cu = _lib.ptr(cu_seqlens)
-    a.nseq = nseq
-    a.max_seqlen = int(max_seqlen) if cu_seqlens is not None else total
-    a.total = total
-    a.h_q, a.h_kv, a.d = h_q, h_kv, d
-    a.dtype = _lib.dtype_code(local_q.dtype)
-    a.cp_rank, a.cp_size = rank, S
-    a.softmax_scale = float(cfg.softmax_scale if cfg.softmax_scale is not None else 1.0 / math.sqrt(d))
-    a.q_descale, a.k_descale, a.v_descale = _lib.ptr(qd), _lib.ptr(kd), _lib.ptr(vd)
-    # where the sweep is split over few row tiles: its partial results, and its counters, which
-    # the V^T launch clears
+        nseq, longest = cu_seqlens.shape[0] - 1, int(max_seqlen)
+    stride = lib.fa4cp_vt_min_d_stride(total, nseq)
+    o_stride = out.stride()
+    a = _lib.SweepArgs(local_q.data_ptr(), out.data_ptr(), lse.data_ptr(), q_stride[0], q_stride[1], o_stride[0],
+                       o_stride[1], lse.stride(0), _lib.Pointers(*k_ptrs), _lib.Pointers(), k_stride[0], k_stride[1], stride,
+                       _lib.ptr(cu_seqlens), nseq, longest, total, h_q, h_kv, d, _lib.dtype_code(local_q.dtype), rank, S,
+                       1.0 / math.sqrt(d) if cfg.softmax_scale is None else float(cfg.softmax_scale), _lib.ptr(qd),
+                       _lib.ptr(kd), _lib.ptr(vd))
+    # one buffer: every source's V^T, and, where the sweep is split over few row tiles, its partial
+    # results and the counters that the V^T launch clears
     words = ctypes.c_int32()
-    need = _lib.load().fa4cp_ring_sweep_workspace_bytes(ctypes.byref(a), ctypes.byref(words))
-    _lib.check(int(min(need, 0)), "fa4cp_ring_sweep_workspace_bytes")
-    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need > 0 else None
-    vts, a.vt_d_stride = transpose(n_front=rank, clear=None if ws is None else (ws, words.value))
-    for i, vt in enumerate(vts):
-        assert vt.device == dev, f"source {i}'s V^T must be on {dev}"
-        a.v_t[i] = vt.data_ptr()
-    launch_sweep(a, dev, kpages, ws)
+    need = lib.fa4cp_ring_sweep_workspace_bytes(ctypes.byref(a), ctypes.byref(words))
+    if need < 0:
+        _lib.check(int(need), "fa4cp_ring_sweep_workspace_bytes")
+    step = h_kv * d * stride * v_dtype.itemsize  # (the stride is a multiple of 128)
+    buf = torch.empty(S * step + need, dtype=torch.uint8, device=dev)
+    vt = buf.data_ptr()
+    ws = vt + S * step if need else None
+    transpose(vt, stride, cu_seqlens, max_seqlen, rank, ws, words.value)
+    a.v_t = _lib.Pointers(*range(vt, vt + S * step, step))
+    launch_sweep(a, dev, kpages, ws, need)
     return out
 
 
 def launch_sweep(args: "_lib.SweepArgs", device: torch.device, kpages: Optional["_lib.SweepKPages"] = None,
-                 workspace: Optional[torch.Tensor] = None) -> None:
+                 workspace: Optional[int] = None, workspace_bytes: int = 0) -> None:
     """Queues the fused sweep kernel on the current stream of `device` (with `kpages`: the
-    paged-K sweep; with `workspace`: split where its shape asks for it)."""
-    _lib.check(_lib.load().fa4cp_ring_sweep_fwd_ws(
-        ctypes.byref(args), None if kpages is None else ctypes.byref(kpages), _lib.ptr(workspace),
-        0 if workspace is None else workspace.numel(), _lib.stream_handle(device)),
-        "fa4cp_ring_sweep_fwd" if kpages is None else "fa4cp_ring_sweep_fwd_paged")
+    paged-K sweep; with the address of a `workspace`: split where its shape asks for it)."""
+    rc = _lib.load().fa4cp_ring_sweep_fwd_ws(ctypes.byref(args), None if kpages is None else ctypes.byref(kpages),
+                                             workspace, workspace_bytes, _lib.stream_handle(device))
+    if rc:
+        _lib.check(rc, "fa4cp_ring_sweep_fwd" if kpages is None else "fa4cp_ring_sweep_fwd_paged")

@@ -41,7 +41,7 @@ CASES = [  # (local lens, H, H_kv, D, cp, rank, dtype, page size): row tiles of 
 
 def _unsplit(monkeypatch):
     launch = RA.launch_sweep
-    monkeypatch.setattr(RA, "launch_sweep", lambda a, dev, kp=None, ws=None: launch(a, dev, kp, None))
+    monkeypatch.setattr(RA, "launch_sweep", lambda a, dev, kp=None, ws=None, n=0: launch(a, dev, kp))
 
 
 def _shares(lens, h, h_kv, d, cp, rank, dtype):
