@@ -822,14 +822,21 @@ __global__ __launch_bounds__(512) void bwd_dq_pp_kernel(BwdParams p) {
 // blocks at a time), and the own tiles, of falling length, go kv head by kv head, so that every
 // XCD gets its share of each length.  With the sources in order and key tiles fastest everywhere
 // an XCD had the same own tiles of all heads, and long ones came last: dk / dv 335-342 us at 8192
-// tokens (H 32/8, cp 4, rank 1), where the workgroups' times add up to 220 us a CU; now 304-316.
-// The whole backward at 32768 tokens (cp 8, rank 3): 3997 -> 3498 us.
+// tokens (H 32/8, cp 4, rank 1), where the workgroups' times add up to 250 us a CU; in this order
+// 304-316.  The whole backward at 32768 tokens (cp 8, rank 3): 3997 -> 3498 us.
+// PAIR: the workgroup of the own tile kt < n / 2 goes on with tile n - 1 - kt, so that the two
+// take about as long as a tile every row attends (class 3 is then empty).  Within an XCD the
+// hardware hands the workgroups to its four shader engines strictly in turn and in order: one
+// that is due on a full engine holds up all later ones, and a short own tile started last behind
+// one on a CU that was already late (of 299 us the last 50 had a fifth of the CUs busy).  With equal
+// workgroups it cannot: 272 us, the whole backward 559 -> 536 us; H 24/8 at rank 0 of 8 288 -> 266.
+template <bool PAIR>
 __device__ __forceinline__ void dkdv_tile(const BwdParams& p, int b, int ns, int& share, int& tile, int& kt, int& seq,
                                           int& kvh, int& src) {
   const int per_kt = p.nseq * p.h_kv, late = p.S - 1 - p.rank;
   const int front = min(p.n_tiles, ((p.max_seqlen >> 1) + kDkdvKeys - 1) / kDkdvKeys), own = (p.n_tiles + 1) / 2;
   int n_src[5] = {p.rank, 1, late, 1, p.rank};
-  int n_kt[5] = {front, own, p.n_tiles, p.n_tiles - own, p.n_tiles - front};
+  int n_kt[5] = {front, own, p.n_tiles, PAIR ? 0 : p.n_tiles - own, p.n_tiles - front};
   int at = 0, c = 0, n = 0;  // tiles before class c, and its own
 #pragma unroll
   for (int i = 0; i < 5; ++i) {
@@ -889,7 +896,7 @@ __device__ __forceinline__ void dkdv_tile(const BwdParams& p, int b, int ns, int
 // each kind double-buffered by block parity: iteration i reads rows(i) and transposed(i - 1)
 // and loads rows(i + 1) and transposed(i) over those of blocks i - 1 and i - 2 (4 x 64.25 KB).
 // (The halves measured 7 % slower at 128, where whole stages fit.)
-template <typename T, int D>
+template <typename T, int D, bool PAIR>
 __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams p) {
   using M = BwdMfma<T>;
   typedef typename M::frag frag;
@@ -928,335 +935,347 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
   constexpr int OVAL = HALVES ? 2 * R : 4 * R;
 
   int share, tile, kt, seq, kvh, src;
-  dkdv_tile(p, blockIdx.x, kShares ? p.ns : 1, share, tile, kt, seq, kvh, src);
-  const int64_t pstart = vt_seq_start(p.cu, seq, p.total, FA4CP_SEL_ALL) / kBwdRows;
-  int qs, L;
-  seq_range(p.cu, seq, p.total, FA4CP_SEL_ALL, qs, L);
-  const int kb0 = kt * kDkdvKeys;
-  if (kb0 >= L) return;
-  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int l = threadIdx.x & 63, h = l >> 5, lk = l & 31;
-  const bool pwave = w < 4;
-  const bool producer = !HALVES && w == 8;   // up to head dim 128: the ninth wavefront loads the blocks
-  const int kg0 = kb0 + kBwdRows * (w & 3);  // first key of the pair's group
-  const int key = kg0 + lk;                  // this lane's key in the sequence
-  const StepPairs sp = step_pairs(p.rank, p.S, src, L);
+  dkdv_tile<PAIR>(p, blockIdx.x, kShares && !PAIR ? p.ns : 1, share, tile, kt, seq, kvh, src);
+  // PAIR (one sequence, see dkdv_tile): the distance to the second of the two own tiles
+  int next = PAIR && src == p.rank ? p.n_tiles - 1 - 2 * kt : 0;
+  auto another = [&]() __attribute__((always_inline)) {
+    if (next <= 0) return false;
+    kt += next;
+    next = 0;
+    wg_barrier();  // the second tile's blocks go where the first one's were read
+    return true;
+  };
+  do {
+    const int64_t pstart = vt_seq_start(p.cu, seq, p.total, FA4CP_SEL_ALL) / kBwdRows;
+    int qs, L;
+    seq_range(p.cu, seq, p.total, FA4CP_SEL_ALL, qs, L);
+    const int kb0 = kt * kDkdvKeys;
+    if (kb0 >= L) continue;
+    int t = threadIdx.x;
+    if constexpr (PAIR) asm volatile("" : "+v"(t));  // else addresses are formed before the loop over the tiles, and spill
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int l = t & 63, h = l >> 5, lk = l & 31;
+    const bool pwave = w < 4;
+    const bool producer = !HALVES && w == 8;   // up to head dim 128: the ninth wavefront loads the blocks
+    const int kg0 = kb0 + kBwdRows * (w & 3);  // first key of the pair's group
+    const int key = kg0 + lk;                  // this lane's key in the sequence
+    const StepPairs sp = step_pairs(p.rank, p.S, src, L);
 
-  f32x16 acc[NDT];  // dV (first wavefront of a pair) or dK (second)
+    f32x16 acc[NDT];  // dV (first wavefront of a pair) or dK (second)
 #pragma unroll
-  for (int i = 0; i < NDT; ++i) acc[i] = f32x16{};
+    for (int i = 0; i < NDT; ++i) acc[i] = f32x16{};
 
-  int shares = 1;
-  if (kb0 < sp.key_lim) {
-    // K (first wavefront) or V (second) of the lane's key: B operands of S and dP
-    frag kv[NKS];
-    if (!producer) {
-      const bool ok = key < sp.key_lim;
-      const T* r = pwave ? reinterpret_cast<const T*>(p.k[src]) + (int64_t)(qs + key) * p.k_rs + (int64_t)kvh * p.k_hs
-                         : reinterpret_cast<const T*>(p.v[src]) + (int64_t)(qs + key) * p.v_rs + (int64_t)kvh * p.v_hs;
+    int shares = 1;
+    if (kb0 < sp.key_lim) {
+      // K (first wavefront) or V (second) of the lane's key: B operands of S and dP
+      frag kv[NKS];
+      if (!producer) {
+        const bool ok = key < sp.key_lim;
+        const T* r = pwave ? reinterpret_cast<const T*>(p.k[src]) + (int64_t)(qs + key) * p.k_rs + (int64_t)kvh * p.k_hs
+                           : reinterpret_cast<const T*>(p.v[src]) + (int64_t)(qs + key) * p.v_rs + (int64_t)kvh * p.v_hs;
 #pragma unroll
-      for (int t = 0; t < NKS; ++t) {
-        frag z = {};
-        kv[t] = ok ? *reinterpret_cast<const frag*>(r + 8 * h + 16 * t) : z;
-      }
-    }
-    const float c = p.scale * kLog2e;
-    // query rows that can see a key of this workgroup: from the first key on when causal
-    const int row_begin = max(sp.row_min, sp.causal ? kb0 : 0) / kBwdRows * kBwdRows;
-    const int n_rb = (L - row_begin + kBwdRows - 1) / kBwdRows;
-    // (query head, 32-row block) pairs, head-major: this workgroup's share of them, from `lo` on
-    int lo, hi;
-    if (kShares) {
-      if (!take_share(p, share, n_rb * p.group, lo, hi, shares)) return;
-    } else {
-      lo = 0;
-      hi = n_rb * p.group;
-    }
-    const int n_blk = hi - lo;
-    const int64_t blk0 = pstart + row_begin / kBwdRows;
-    // query head (within the group) and row block of the next block a load takes
-    struct Cursor {
-      int lh, lr;
-    };
-    Cursor rc{lo / n_rb, lo % n_rb}, tc = rc;
-    // head dim 256: the half of the block at cursor cu made of regions r0 and r0 + 2 into
-    // half-stage st, then the per-row values
-    auto load = [&](Cursor& cu, char* st, int r0) {
-      const char* g = p.pk + ((int64_t)(kvh * p.group + cu.lh) * p.n_pb + blk0 + cu.lr) * BB;
-      const __amdgpu_buffer_rsrc_t rs = make_rsrc32(uniform_ptr(g), BB);
-#pragma unroll
-      for (int j = 0; j < CPW; ++j) {
-        const int f = w + 8 * j;  // region r0 + 2 (f / NKS), fragment f % NKS
-        dma16(rs, st + 1024 * f, (r0 + 2 * (f / NKS)) * R + 1024 * (f % NKS) + 16 * l);
-      }
-      dma4(rs, st + OVAL, 4 * R + 4 * l);  // every wavefront writes the same per-row values
-      if (++cu.lr == n_rb) {
-        cu.lr = 0;
-        ++cu.lh;
-      }
-    };
-    // lse * log2(e) (off 0) or delta (off 128) of the rows of accumulator registers 0..15
-    auto row_vals = [&](const char* st, int off, float (&v)[16]) {
-      const f32x4* s4 = reinterpret_cast<const f32x4*>(st + OVAL + off);
-      const f32x4 a = s4[2 * h], bq = s4[2 * h + 1], cq = s4[4 + 2 * h], dq = s4[5 + 2 * h];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[j] = a[j];
-        v[4 + j] = bq[j];
-        v[8 + j] = cq[j];
-        v[12 + j] = dq[j];
-      }
-    };
-    auto frag_at = [&](const char* st, int off) { return *reinterpret_cast<const frag*>(st + off + 16 * l); };
-    // head dim 256: half-stages, loaded one iteration ahead
-    auto run_halves = [&](auto role) {
-      constexpr bool PW = decltype(role)::value;
-      frag pb0, pb1;  // first wavefront: P of the previous block (operands of dV)
-      f32x16 dpt;     // second wavefront: dP of the previous block
-      int cr = lo % n_rb;  // row block (within the head) of block i
-      load(rc, rows_of(0), 0);
-      __builtin_amdgcn_s_waitcnt(kWaitAll);
-      wg_barrier();
-      for (int i = 0; i <= n_blk; ++i) {
-        // this iteration's loads, issued in the VALU section of each wavefront (the first after
-        // writing P, the second after forming dS): 1.3 % faster than at the iteration start
-        auto loads = [&]() __attribute__((always_inline)) {
-          if (i + 1 < n_blk) load(rc, rows_of(i + 1), 0);
-          if (i < n_blk) load(tc, trans_of(i), 1);
-        };
-        const char* cur = rows_of(i);       // block i: its row regions
-        const char* prev = trans_of(i + 1);  // block i - 1: its transposed regions and the values
-        if constexpr (PW) {
-          __builtin_amdgcn_s_setprio(1);
-          if (i > 0) {
-            // the two 16-row halves in turn over the d tiles, so that consecutive MFMAs update
-            // different accumulators (each still sums its terms in the same order): 1.5-2 % off
-            // this kernel, where the same order made the head-dim-128 backward 1.2 % slower
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) acc[dt] = M::mma(frag_at(prev, ODOT + 1024 * (2 * dt)), pb0, acc[dt]);
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) acc[dt] = M::mma(frag_at(prev, ODOT + 1024 * (2 * dt + 1)), pb1, acc[dt]);
-          }
-          if (i < n_blk) {
-            f32x16 st = {};
-#pragma unroll
-            for (int t = 0; t < NKS; ++t) st = M::mma(frag_at(cur, OQ + 1024 * t), kv[t], st);
-            __builtin_amdgcn_s_setprio(0);
-            float lse[16], pv[16];
-            row_vals(cur, 0, lse);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) pv[r] = __builtin_amdgcn_exp2f(fmaf(st[r], c, -lse[r]));
-            const int row0 = row_begin + cr * kBwdRows;
-            const bool full = row0 >= sp.row_min && kg0 + kBwdRows <= sp.key_lim &&
-                              (!sp.causal || row0 >= kg0 + kBwdRows - 1);
-            if (!full) {
-#pragma unroll
-              for (int r = 0; r < 16; ++r) {
-                const int row = row0 + acc_pos(r, h);
-                const bool ok = row >= sp.row_min && key < sp.key_lim && (!sp.causal || key <= row);
-                pv[r] = ok ? pv[r] : 0.f;
-              }
-            }
-            pb0 = to_frag<T>(pv);
-            pb1 = to_frag<T>(pv + 8);
-            char* xb = xch + ((i & 1) * 4 + (w & 3)) * 2048;
-            *reinterpret_cast<f16x8*>(xb + 16 * l) = to_frag<_Float16>(pv);
-            *reinterpret_cast<f16x8*>(xb + 1024 + 16 * l) = to_frag<_Float16>(pv + 8);
-          }
-          loads();
-        } else {
-          if (i > 0) {
-            const char* xb = xch + (((i - 1) & 1) * 4 + (w & 3)) * 2048;
-            const f16x8 e0 = *reinterpret_cast<const f16x8*>(xb + 16 * l);
-            const f16x8 e1 = *reinterpret_cast<const f16x8*>(xb + 1024 + 16 * l);
-            float dl[16], dsv[16];
-            row_vals(prev, 128, dl);
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-              dsv[r] = (float)e0[r] * (dpt[r] - dl[r]);
-              dsv[8 + r] = (float)e1[r] * (dpt[8 + r] - dl[8 + r]);
-            }
-            const frag s0 = to_frag<T>(dsv), s1 = to_frag<T>(dsv + 8);
-            loads();
-            __builtin_amdgcn_s_setprio(1);
-            // as for dV above
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) acc[dt] = M::mma(frag_at(prev, OQT + 1024 * (2 * dt)), s0, acc[dt]);
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) acc[dt] = M::mma(frag_at(prev, OQT + 1024 * (2 * dt + 1)), s1, acc[dt]);
-          } else {
-            loads();
-          }
-          if (i < n_blk) {
-            dpt = f32x16{};
-#pragma unroll
-            for (int t = 0; t < NKS; ++t) dpt = M::mma(frag_at(cur, ODO + 1024 * t), kv[t], dpt);
-          }
+        for (int t = 0; t < NKS; ++t) {
+          frag z = {};
+          kv[t] = ok ? *reinterpret_cast<const frag*>(r + 8 * h + 16 * t) : z;
         }
-        __builtin_amdgcn_s_setprio(0);
-        if (i < n_blk) {  // the loads landed (each wavefront's own), P of block i written
-          __builtin_amdgcn_s_waitcnt(kWaitAll);
-          wg_barrier();
-        }
-        if (++cr == n_rb) cr = 0;
       }
-    };
-    // n MFMAs in program order, the LDS fragment of MFMA k read four MFMAs ahead into a
-    // register of its own (fenced MFMA by MFMA: left alone, the compiler reads each fragment
-    // just before its MFMA and waits for it)
-    auto chain = [&](auto n_c, auto rd, auto mm) __attribute__((always_inline)) {
-      constexpr int N = decltype(n_c)::value, RA = 4;
-      frag fr[N];
-#pragma unroll
-      for (int k = 0; k < RA && k < N; ++k) fr[k] = rd(k);
-#pragma unroll
-      for (int k = 0; k < N; ++k) {
-        __builtin_amdgcn_sched_barrier(0);
-        if (k + RA < N) fr[k + RA] = rd(k + RA);
-        mm(k, fr[k]);
+      const float c = p.scale * kLog2e;
+      // query rows that can see a key of this workgroup: from the first key on when causal
+      const int row_begin = max(sp.row_min, sp.causal ? kb0 : 0) / kBwdRows * kBwdRows;
+      const int n_rb = (L - row_begin + kBwdRows - 1) / kBwdRows;
+      // (query head, 32-row block) pairs, head-major: this workgroup's share of them, from `lo` on
+      int lo, hi;
+      if (kShares) {
+        if (!take_share(p, share, n_rb * p.group, lo, hi, shares)) continue;
+      } else {
+        lo = 0;
+        hi = n_rb * p.group;
       }
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    // up to head dim 128: whole stages, loaded two iterations ahead by the ninth wavefront
-    auto run_producer = [&]() __attribute__((always_inline)) {
-      // the next block to load (wave-uniform, advanced block by block: the blocks of one query
-      // head are consecutive, the next head's start n_pb blocks after the previous one's)
-      const char* gnext = reinterpret_cast<const char*>(
-          uniform_ptr(p.pk + ((int64_t)(kvh * p.group + lo / n_rb) * p.n_pb + blk0 + lo % n_rb) * BB));
-      const int64_t head_jump = (int64_t)(p.n_pb - n_rb) * BB;
-      int lr = lo % n_rb;
-      auto load_block = [&](char* st) __attribute__((always_inline)) {
-        const __amdgpu_buffer_rsrc_t rs = make_rsrc32(gnext, BB);
-        gnext += BB;
-        if (++lr == n_rb) {
-          lr = 0;
-          gnext += head_jump;
-        }
-#pragma unroll
-        for (int f = 0; f < 4 * NKS; ++f) dma16(rs, st + 1024 * f, 1024 * f + 16 * l);
-        dma4(rs, st + OVAL, 4 * R + 4 * l);
+      const int n_blk = hi - lo;
+      const int64_t blk0 = pstart + row_begin / kBwdRows;
+      // query head (within the group) and row block of the next block a load takes
+      struct Cursor {
+        int lh, lr;
       };
-      load_block(stage_of(0));
-      if (n_blk > 1) load_block(stage_of(1));
-      __builtin_amdgcn_s_waitcnt(kWaitAll);
-      wg_barrier();
-      for (int i = 0; i < n_blk; ++i) {
-        // block i + 1 (loaded an iteration ago) has landed before this iteration's barrier;
-        // block i + 2 goes into the stage of block i - 2, last read before the previous barrier
-        __builtin_amdgcn_s_waitcnt(kWaitAll);
-        if (i + 2 < n_blk) load_block(stage_of(i + 2));
-        wg_barrier();
-      }
-    };
-    auto run_whole = [&](auto role) {
-      constexpr bool PW = decltype(role)::value;
-      frag pb0, pb1;  // first wavefront: P of the previous block (operands of dV)
-      f32x16 dpt;     // second wavefront: dP of the previous block
-      int cr = lo % n_rb;  // row block (within the head) of block i
-      wg_barrier();
-      for (int i = 0; i <= n_blk; ++i) {
-        const char* cur = stage_of(i);       // block i: its row regions
-        const char* prev = stage_of(i + 3);  // block i - 1: its transposed regions and the values
-        if constexpr (PW) {
-          __builtin_amdgcn_s_setprio(1);
-          if (i > 0) {
-            chain(std::integral_constant<int, 2 * NDT>{}, [&](int k) { return frag_at(prev, ODOT + 1024 * k); },
-                  [&](int k, frag f) { acc[k >> 1] = M::mma(f, (k & 1) ? pb1 : pb0, acc[k >> 1]); });
-          }
-          if (i < n_blk) {
-            f32x16 st = {};
-            chain(std::integral_constant<int, NKS>{}, [&](int k) { return frag_at(cur, OQ + 1024 * k); },
-                  [&](int k, frag f) { st = M::mma(f, kv[k], st); });
-            __builtin_amdgcn_s_setprio(0);
-            float lse[16], pv[16];
-            row_vals(cur, 0, lse);
+      Cursor rc{lo / n_rb, lo % n_rb}, tc = rc;
+      // head dim 256: the half of the block at cursor cu made of regions r0 and r0 + 2 into
+      // half-stage st, then the per-row values
+      auto load = [&](Cursor& cu, char* st, int r0) {
+        const char* g = p.pk + ((int64_t)(kvh * p.group + cu.lh) * p.n_pb + blk0 + cu.lr) * BB;
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc32(uniform_ptr(g), BB);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) pv[r] = __builtin_amdgcn_exp2f(fmaf(st[r], c, -lse[r]));
-            const int row0 = row_begin + cr * kBwdRows;
-            const bool full = row0 >= sp.row_min && kg0 + kBwdRows <= sp.key_lim &&
-                              (!sp.causal || row0 >= kg0 + kBwdRows - 1);
-            if (!full) {
-#pragma unroll
-              for (int r = 0; r < 16; ++r) {
-                const int row = row0 + acc_pos(r, h);
-                const bool ok = row >= sp.row_min && key < sp.key_lim && (!sp.causal || key <= row);
-                pv[r] = ok ? pv[r] : 0.f;
-              }
-            }
-            pb0 = to_frag<T>(pv);
-            pb1 = to_frag<T>(pv + 8);
-            char* xb = xch + ((i & 1) * 4 + (w & 3)) * 2048;
-            *reinterpret_cast<f16x8*>(xb + 16 * l) = to_frag<_Float16>(pv);
-            *reinterpret_cast<f16x8*>(xb + 1024 + 16 * l) = to_frag<_Float16>(pv + 8);
-          }
-        } else {
-          if (i > 0) {
-            const char* xb = xch + (((i - 1) & 1) * 4 + (w & 3)) * 2048;
-            const f16x8 e0 = *reinterpret_cast<const f16x8*>(xb + 16 * l);
-            const f16x8 e1 = *reinterpret_cast<const f16x8*>(xb + 1024 + 16 * l);
-            float dl[16], dsv[16];
-            row_vals(prev, 128, dl);
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-              dsv[r] = (float)e0[r] * (dpt[r] - dl[r]);
-              dsv[8 + r] = (float)e1[r] * (dpt[8 + r] - dl[8 + r]);
-            }
-            const frag s0 = to_frag<T>(dsv), s1 = to_frag<T>(dsv + 8);
-            __builtin_amdgcn_s_setprio(1);
-            chain(std::integral_constant<int, 2 * NDT>{}, [&](int k) { return frag_at(prev, OQT + 1024 * k); },
-                  [&](int k, frag f) { acc[k >> 1] = M::mma(f, (k & 1) ? s1 : s0, acc[k >> 1]); });
-          }
-          if (i < n_blk) {
-            dpt = f32x16{};
-            chain(std::integral_constant<int, NKS>{}, [&](int k) { return frag_at(cur, ODO + 1024 * k); },
-                  [&](int k, frag f) { dpt = M::mma(f, kv[k], dpt); });
-          }
+        for (int j = 0; j < CPW; ++j) {
+          const int f = w + 8 * j;  // region r0 + 2 (f / NKS), fragment f % NKS
+          dma16(rs, st + 1024 * f, (r0 + 2 * (f / NKS)) * R + 1024 * (f % NKS) + 16 * l);
         }
-        __builtin_amdgcn_s_setprio(0);
-        if (i < n_blk) {  // P of block i written (the producer has waited for block i + 1)
+        dma4(rs, st + OVAL, 4 * R + 4 * l);  // every wavefront writes the same per-row values
+        if (++cu.lr == n_rb) {
+          cu.lr = 0;
+          ++cu.lh;
+        }
+      };
+      // lse * log2(e) (off 0) or delta (off 128) of the rows of accumulator registers 0..15
+      auto row_vals = [&](const char* st, int off, float (&v)[16]) {
+        const f32x4* s4 = reinterpret_cast<const f32x4*>(st + OVAL + off);
+        const f32x4 a = s4[2 * h], bq = s4[2 * h + 1], cq = s4[4 + 2 * h], dq = s4[5 + 2 * h];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v[j] = a[j];
+          v[4 + j] = bq[j];
+          v[8 + j] = cq[j];
+          v[12 + j] = dq[j];
+        }
+      };
+      auto frag_at = [&](const char* st, int off) { return *reinterpret_cast<const frag*>(st + off + 16 * l); };
+      // head dim 256: half-stages, loaded one iteration ahead
+      auto run_halves = [&](auto role) {
+        constexpr bool PW = decltype(role)::value;
+        frag pb0, pb1;  // first wavefront: P of the previous block (operands of dV)
+        f32x16 dpt;     // second wavefront: dP of the previous block
+        int cr = lo % n_rb;  // row block (within the head) of block i
+        load(rc, rows_of(0), 0);
+        __builtin_amdgcn_s_waitcnt(kWaitAll);
+        wg_barrier();
+        for (int i = 0; i <= n_blk; ++i) {
+          // this iteration's loads, issued in the VALU section of each wavefront (the first after
+          // writing P, the second after forming dS): 1.3 % faster than at the iteration start
+          auto loads = [&]() __attribute__((always_inline)) {
+            if (i + 1 < n_blk) load(rc, rows_of(i + 1), 0);
+            if (i < n_blk) load(tc, trans_of(i), 1);
+          };
+          const char* cur = rows_of(i);       // block i: its row regions
+          const char* prev = trans_of(i + 1);  // block i - 1: its transposed regions and the values
+          if constexpr (PW) {
+            __builtin_amdgcn_s_setprio(1);
+            if (i > 0) {
+              // the two 16-row halves in turn over the d tiles, so that consecutive MFMAs update
+              // different accumulators (each still sums its terms in the same order): 1.5-2 % off
+              // this kernel, where the same order made the head-dim-128 backward 1.2 % slower
+#pragma unroll
+              for (int dt = 0; dt < NDT; ++dt) acc[dt] = M::mma(frag_at(prev, ODOT + 1024 * (2 * dt)), pb0, acc[dt]);
+#pragma unroll
+              for (int dt = 0; dt < NDT; ++dt) acc[dt] = M::mma(frag_at(prev, ODOT + 1024 * (2 * dt + 1)), pb1, acc[dt]);
+            }
+            if (i < n_blk) {
+              f32x16 st = {};
+#pragma unroll
+              for (int t = 0; t < NKS; ++t) st = M::mma(frag_at(cur, OQ + 1024 * t), kv[t], st);
+              __builtin_amdgcn_s_setprio(0);
+              float lse[16], pv[16];
+              row_vals(cur, 0, lse);
+#pragma unroll
+              for (int r = 0; r < 16; ++r) pv[r] = __builtin_amdgcn_exp2f(fmaf(st[r], c, -lse[r]));
+              const int row0 = row_begin + cr * kBwdRows;
+              const bool full = row0 >= sp.row_min && kg0 + kBwdRows <= sp.key_lim &&
+                                (!sp.causal || row0 >= kg0 + kBwdRows - 1);
+              if (!full) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                  const int row = row0 + acc_pos(r, h);
+                  const bool ok = row >= sp.row_min && key < sp.key_lim && (!sp.causal || key <= row);
+                  pv[r] = ok ? pv[r] : 0.f;
+                }
+              }
+              pb0 = to_frag<T>(pv);
+              pb1 = to_frag<T>(pv + 8);
+              char* xb = xch + ((i & 1) * 4 + (w & 3)) * 2048;
+              *reinterpret_cast<f16x8*>(xb + 16 * l) = to_frag<_Float16>(pv);
+              *reinterpret_cast<f16x8*>(xb + 1024 + 16 * l) = to_frag<_Float16>(pv + 8);
+            }
+            loads();
+          } else {
+            if (i > 0) {
+              const char* xb = xch + (((i - 1) & 1) * 4 + (w & 3)) * 2048;
+              const f16x8 e0 = *reinterpret_cast<const f16x8*>(xb + 16 * l);
+              const f16x8 e1 = *reinterpret_cast<const f16x8*>(xb + 1024 + 16 * l);
+              float dl[16], dsv[16];
+              row_vals(prev, 128, dl);
+#pragma unroll
+              for (int r = 0; r < 8; ++r) {
+                dsv[r] = (float)e0[r] * (dpt[r] - dl[r]);
+                dsv[8 + r] = (float)e1[r] * (dpt[8 + r] - dl[8 + r]);
+              }
+              const frag s0 = to_frag<T>(dsv), s1 = to_frag<T>(dsv + 8);
+              loads();
+              __builtin_amdgcn_s_setprio(1);
+              // as for dV above
+#pragma unroll
+              for (int dt = 0; dt < NDT; ++dt) acc[dt] = M::mma(frag_at(prev, OQT + 1024 * (2 * dt)), s0, acc[dt]);
+#pragma unroll
+              for (int dt = 0; dt < NDT; ++dt) acc[dt] = M::mma(frag_at(prev, OQT + 1024 * (2 * dt + 1)), s1, acc[dt]);
+            } else {
+              loads();
+            }
+            if (i < n_blk) {
+              dpt = f32x16{};
+#pragma unroll
+              for (int t = 0; t < NKS; ++t) dpt = M::mma(frag_at(cur, ODO + 1024 * t), kv[t], dpt);
+            }
+          }
+          __builtin_amdgcn_s_setprio(0);
+          if (i < n_blk) {  // the loads landed (each wavefront's own), P of block i written
+            __builtin_amdgcn_s_waitcnt(kWaitAll);
+            wg_barrier();
+          }
+          if (++cr == n_rb) cr = 0;
+        }
+      };
+      // n MFMAs in program order, the LDS fragment of MFMA k read four MFMAs ahead into a
+      // register of its own (fenced MFMA by MFMA: left alone, the compiler reads each fragment
+      // just before its MFMA and waits for it)
+      auto chain = [&](auto n_c, auto rd, auto mm) __attribute__((always_inline)) {
+        constexpr int N = decltype(n_c)::value, RA = 4;
+        frag fr[N];
+#pragma unroll
+        for (int k = 0; k < RA && k < N; ++k) fr[k] = rd(k);
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (k + RA < N) fr[k + RA] = rd(k + RA);
+          mm(k, fr[k]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      // up to head dim 128: whole stages, loaded two iterations ahead by the ninth wavefront
+      auto run_producer = [&]() __attribute__((always_inline)) {
+        // the next block to load (wave-uniform, advanced block by block: the blocks of one query
+        // head are consecutive, the next head's start n_pb blocks after the previous one's)
+        const char* gnext = reinterpret_cast<const char*>(
+            uniform_ptr(p.pk + ((int64_t)(kvh * p.group + lo / n_rb) * p.n_pb + blk0 + lo % n_rb) * BB));
+        const int64_t head_jump = (int64_t)(p.n_pb - n_rb) * BB;
+        int lr = lo % n_rb;
+        auto load_block = [&](char* st) __attribute__((always_inline)) {
+          const __amdgpu_buffer_rsrc_t rs = make_rsrc32(gnext, BB);
+          gnext += BB;
+          if (++lr == n_rb) {
+            lr = 0;
+            gnext += head_jump;
+          }
+#pragma unroll
+          for (int f = 0; f < 4 * NKS; ++f) dma16(rs, st + 1024 * f, 1024 * f + 16 * l);
+          dma4(rs, st + OVAL, 4 * R + 4 * l);
+        };
+        load_block(stage_of(0));
+        if (n_blk > 1) load_block(stage_of(1));
+        __builtin_amdgcn_s_waitcnt(kWaitAll);
+        wg_barrier();
+        for (int i = 0; i < n_blk; ++i) {
+          // block i + 1 (loaded an iteration ago) has landed before this iteration's barrier;
+          // block i + 2 goes into the stage of block i - 2, last read before the previous barrier
           __builtin_amdgcn_s_waitcnt(kWaitAll);
+          if (i + 2 < n_blk) load_block(stage_of(i + 2));
           wg_barrier();
         }
-        if (++cr == n_rb) cr = 0;
-      }
-    };
-    if (n_blk > 0) {
-      if constexpr (HALVES) {
-        if (pwave) run_halves(std::true_type{});
-        else run_halves(std::false_type{});
-      } else {
-        if (producer) run_producer();
-        else if (pwave) run_whole(std::true_type{});
-        else run_whole(std::false_type{});
+      };
+      auto run_whole = [&](auto role) {
+        constexpr bool PW = decltype(role)::value;
+        frag pb0, pb1;  // first wavefront: P of the previous block (operands of dV)
+        f32x16 dpt;     // second wavefront: dP of the previous block
+        int cr = lo % n_rb;  // row block (within the head) of block i
+        wg_barrier();
+        for (int i = 0; i <= n_blk; ++i) {
+          const char* cur = stage_of(i);       // block i: its row regions
+          const char* prev = stage_of(i + 3);  // block i - 1: its transposed regions and the values
+          if constexpr (PW) {
+            __builtin_amdgcn_s_setprio(1);
+            if (i > 0) {
+              chain(std::integral_constant<int, 2 * NDT>{}, [&](int k) { return frag_at(prev, ODOT + 1024 * k); },
+                    [&](int k, frag f) { acc[k >> 1] = M::mma(f, (k & 1) ? pb1 : pb0, acc[k >> 1]); });
+            }
+            if (i < n_blk) {
+              f32x16 st = {};
+              chain(std::integral_constant<int, NKS>{}, [&](int k) { return frag_at(cur, OQ + 1024 * k); },
+                    [&](int k, frag f) { st = M::mma(f, kv[k], st); });
+              __builtin_amdgcn_s_setprio(0);
+              float lse[16], pv[16];
+              row_vals(cur, 0, lse);
+#pragma unroll
+              for (int r = 0; r < 16; ++r) pv[r] = __builtin_amdgcn_exp2f(fmaf(st[r], c, -lse[r]));
+              const int row0 = row_begin + cr * kBwdRows;
+              const bool full = row0 >= sp.row_min && kg0 + kBwdRows <= sp.key_lim &&
+                                (!sp.causal || row0 >= kg0 + kBwdRows - 1);
+              if (!full) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                  const int row = row0 + acc_pos(r, h);
+                  const bool ok = row >= sp.row_min && key < sp.key_lim && (!sp.causal || key <= row);
+                  pv[r] = ok ? pv[r] : 0.f;
+                }
+              }
+              pb0 = to_frag<T>(pv);
+              pb1 = to_frag<T>(pv + 8);
+              char* xb = xch + ((i & 1) * 4 + (w & 3)) * 2048;
+              *reinterpret_cast<f16x8*>(xb + 16 * l) = to_frag<_Float16>(pv);
+              *reinterpret_cast<f16x8*>(xb + 1024 + 16 * l) = to_frag<_Float16>(pv + 8);
+            }
+          } else {
+            if (i > 0) {
+              const char* xb = xch + (((i - 1) & 1) * 4 + (w & 3)) * 2048;
+              const f16x8 e0 = *reinterpret_cast<const f16x8*>(xb + 16 * l);
+              const f16x8 e1 = *reinterpret_cast<const f16x8*>(xb + 1024 + 16 * l);
+              float dl[16], dsv[16];
+              row_vals(prev, 128, dl);
+#pragma unroll
+              for (int r = 0; r < 8; ++r) {
+                dsv[r] = (float)e0[r] * (dpt[r] - dl[r]);
+                dsv[8 + r] = (float)e1[r] * (dpt[8 + r] - dl[8 + r]);
+              }
+              const frag s0 = to_frag<T>(dsv), s1 = to_frag<T>(dsv + 8);
+              __builtin_amdgcn_s_setprio(1);
+              chain(std::integral_constant<int, 2 * NDT>{}, [&](int k) { return frag_at(prev, OQT + 1024 * k); },
+                    [&](int k, frag f) { acc[k >> 1] = M::mma(f, (k & 1) ? s1 : s0, acc[k >> 1]); });
+            }
+            if (i < n_blk) {
+              dpt = f32x16{};
+              chain(std::integral_constant<int, NKS>{}, [&](int k) { return frag_at(cur, ODO + 1024 * k); },
+                    [&](int k, frag f) { dpt = M::mma(f, kv[k], dpt); });
+            }
+          }
+          __builtin_amdgcn_s_setprio(0);
+          if (i < n_blk) {  // P of block i written (the producer has waited for block i + 1)
+            __builtin_amdgcn_s_waitcnt(kWaitAll);
+            wg_barrier();
+          }
+          if (++cr == n_rb) cr = 0;
+        }
+      };
+      if (n_blk > 0) {
+        if constexpr (HALVES) {
+          if (pwave) run_halves(std::true_type{});
+          else run_halves(std::false_type{});
+        } else {
+          if (producer) run_producer();
+          else if (pwave) run_whole(std::true_type{});
+          else run_whole(std::false_type{});
+        }
       }
     }
-  }
-  if constexpr (kShares) {
-    if (share >= shares || !merge_shares<NDT>(p, tile, share, shares, 8, acc)) return;
-  }
-  // accumulator register r of lane l: head-dim element 32 dt + 8 (r / 4) + 4h + r % 4 of key
-  // `key`; keys no query of this rank attends (past key_lim) get zeros
-  if (producer || key >= L) return;
-  float* const base = pwave ? p.dv[src] : p.dk[src];
-  const int64_t at = ((int64_t)(qs + key) * p.h_kv + kvh) * D;
-  const float sc = pwave ? 1.f : p.scale;
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int d = 32 * dt + 8 * g + 4 * h;
-      f32x4 a = {acc[dt][4 * g] * sc, acc[dt][4 * g + 1] * sc, acc[dt][4 * g + 2] * sc, acc[dt][4 * g + 3] * sc};
-      if (p.grad16) {
-        typedef T t4 __attribute__((ext_vector_type(4)));
-        *reinterpret_cast<t4*>(reinterpret_cast<T*>(base) + at + d) = t4{(T)a[0], (T)a[1], (T)a[2], (T)a[3]};
-      } else {
-        float* const o = base + at + d;
-        if (p.accumulate) a += *reinterpret_cast<const f32x4*>(o);
-        *reinterpret_cast<f32x4*>(o) = a;
-      }
+    if constexpr (kShares) {
+      if (share >= shares || !merge_shares<NDT>(p, tile, share, shares, 8, acc)) continue;
     }
+    // accumulator register r of lane l: head-dim element 32 dt + 8 (r / 4) + 4h + r % 4 of key
+    // `key`; keys no query of this rank attends (past key_lim) get zeros
+    if (producer || key >= L) continue;
+    float* const base = pwave ? p.dv[src] : p.dk[src];
+    const int64_t at = ((int64_t)(qs + key) * p.h_kv + kvh) * D;
+    const float sc = pwave ? 1.f : p.scale;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int d = 32 * dt + 8 * g + 4 * h;
+        f32x4 a = {acc[dt][4 * g] * sc, acc[dt][4 * g + 1] * sc, acc[dt][4 * g + 2] * sc, acc[dt][4 * g + 3] * sc};
+        if (p.grad16) {
+          typedef T t4 __attribute__((ext_vector_type(4)));
+          *reinterpret_cast<t4*>(reinterpret_cast<T*>(base) + at + d) = t4{(T)a[0], (T)a[1], (T)a[2], (T)a[3]};
+        } else {
+          float* const o = base + at + d;
+          if (p.accumulate) a += *reinterpret_cast<const f32x4*>(o);
+          *reinterpret_cast<f32x4*>(o) = a;
+        }
+      }
+  } while (PAIR && another());
 }
-
 
 // Tiles of the two gradient kernels and the workgroups that share one.
 struct BwdPlan {
@@ -1387,9 +1406,14 @@ int launch_bwd(const BwdParams& base, const BwdPlan& pl, hipStream_t st) {
   p.n_tiles = (p.max_seqlen + kDkdvKeys - 1) / kDkdvKeys;
   use(pl.kv);
   if (shared) p.done += pl.dq_tiles;
-  const int64_t kv_blocks = pl.kv_tiles * p.ns;
+  // Pairs only where not all tiles run at once, and for one sequence: the short tiles of packed
+  // sequences fill the gaps that their uneven lengths leave (16 of 608-3072 tokens, cp 4: 744 us,
+  // in pairs 760).  At head dim 256 the loop over the tiles does not fit the registers.
+  const bool pair = D <= 128 && p.nseq == 1 && pl.kv_tiles > kCus;
+  const int64_t kv_blocks = pair ? pl.kv_tiles - (int64_t)(p.n_tiles / 2) * p.h_kv : pl.kv_tiles * p.ns;
   if (kv_blocks > 0x7fffffffLL) return set_error(FA4CP_EINVAL, "ring_sweep_bwd: too many key tiles");
-  hipLaunchKernelGGL((bwd_dkdv_kernel<T, D>), dim3((unsigned)kv_blocks), dim3(D > 128 ? 512 : 576), 0, st, p);
+  auto* const dkdv = pair ? bwd_dkdv_kernel<T, D, (D <= 128)> : bwd_dkdv_kernel<T, D, false>;
+  hipLaunchKernelGGL(dkdv, dim3((unsigned)kv_blocks), dim3(D > 128 ? 512 : 576), 0, st, p);
   return check_launch("ring_sweep_bwd");
 }
 
