@@ -59,6 +59,12 @@ KernelChoice pick16(int d, int hp, bool vt) {
   return k;
 }
 
+// The V^T kernel of head dim 64 with two workgroups per CU.
+template <typename T>
+auto pick_two(int hp) {
+  return hp == 4 ? attn_fwd_16bit_vt<T, 64, 4, 2> : hp == 2 ? attn_fwd_16bit_vt<T, 64, 2, 2> : attn_fwd_16bit_vt<T, 64, 1, 2>;
+}
+
 KernelChoice pick8(int d, int hp, bool vt) {
   KernelChoice k;
   if (vt && (d == 128 || d == 256)) {
@@ -236,6 +242,7 @@ extern "C" int fa4cp_attn_fwd(const fa4cp_attn_args* a, void* stream) {
     p.claim = claim_slot((hipStream_t)stream);
     if (p.claim != nullptr) grid = (unsigned)(blocks + 8 * spare);
   }
+  if (use_vt && two_per_cu(d, blocks)) kc.fn = a->dtype == FA4CP_BF16 ? pick_two<__bf16>(hp) : pick_two<_Float16>(hp);
   hipLaunchKernelGGL(kc.fn, dim3(grid), dim3(kc.threads), 0, (hipStream_t)stream, p);
   return check_launch("attn_fwd");
 }
@@ -340,10 +347,24 @@ static int ring_sweep_launch(const fa4cp_sweep_args* a, const fa4cp_sweep_kpages
   }
   void (*fn)(SweepParams) = nullptr;
   const bool pack = nseq > 1;  // several sequences: the gap-free row tile order
+  // (packed: about half a row tile per sequence more than total / rows)
+  const bool two = two_per_cu(d, pack ? (int64_t)p.n_hg * (a->total / rows + nseq / 2) : blocks);
 #define FA4CP_PICK_PK(KERNEL, H, ...)                                                       \
   {                                                                                         \
     if (paged) fn = pack ? KERNEL<__VA_ARGS__, H, true, true> : KERNEL<__VA_ARGS__, H, true, false>; \
     else fn = pack ? KERNEL<__VA_ARGS__, H, false, true> : KERNEL<__VA_ARGS__, H, false, false>;   \
+  }
+#define FA4CP_PICK_TWO(T, H)                                                                                     \
+  {                                                                                                              \
+    if (paged) fn = pack ? attn_fwd_16bit_sweep<T, 64, H, true, true, 2> : attn_fwd_16bit_sweep<T, 64, H, true, false, 2>; \
+    else fn = pack ? attn_fwd_16bit_sweep<T, 64, H, false, true, 2> : attn_fwd_16bit_sweep<T, 64, H, false, false, 2>;     \
+  }
+#define FA4CP_PICK_64(T)                                                   \
+  {                                                                        \
+    if (two && hp == 4) FA4CP_PICK_TWO(T, 4)                                \
+    else if (two && hp == 2) FA4CP_PICK_TWO(T, 2)                           \
+    else if (two) FA4CP_PICK_TWO(T, 1)                                      \
+    else FA4CP_PICK_HP(attn_fwd_16bit_sweep, T, 64)                         \
   }
 #define FA4CP_PICK_HP(KERNEL, ...)                      \
   {                                                     \
@@ -355,14 +376,16 @@ static int ring_sweep_launch(const fa4cp_sweep_args* a, const fa4cp_sweep_kpages
     if (d == 128) FA4CP_PICK_HP(attn_fwd_e4m3_sweep, 128)
     else FA4CP_PICK_HP(attn_fwd_e4m3_sweep, 256)
   } else if (a->dtype == FA4CP_BF16) {
-    if (d == 64) FA4CP_PICK_HP(attn_fwd_16bit_sweep, __bf16, 64)
+    if (d == 64) FA4CP_PICK_64(__bf16)
     else if (d == 128) FA4CP_PICK_HP(attn_fwd_16bit_sweep, __bf16, 128)
     else FA4CP_PICK_HP(attn_fwd_16bit_sweep, __bf16, 256)
   } else {
-    if (d == 64) FA4CP_PICK_HP(attn_fwd_16bit_sweep, _Float16, 64)
+    if (d == 64) FA4CP_PICK_64(_Float16)
     else if (d == 128) FA4CP_PICK_HP(attn_fwd_16bit_sweep, _Float16, 128)
     else FA4CP_PICK_HP(attn_fwd_16bit_sweep, _Float16, 256)
   }
+#undef FA4CP_PICK_64
+#undef FA4CP_PICK_TWO
 #undef FA4CP_PICK_HP
 #undef FA4CP_PICK_PK
   // dynamic hand-out of the lists' tails with a tenth more workgroups than row tiles (the

@@ -55,6 +55,15 @@ constexpr int kBN = 64;  // keys per tile
 template <int D>
 constexpr int vt_bn() { return D > 128 ? 32 : kBN; }
 
+// Workgroups per CU that the 16-bit pipeline's kernels are built for (their WGS).  At head dim 64 the
+// LDS tiles take 57 KB and the registers fit 128 without a spill, so two can run on a CU, one's loads,
+// softmax, start and end beside the other's MFMAs: 131072 tokens (H 32/8, cp 8, rank 3) 9180 -> 8460 us, 49152
+// (cp 4, rank 2) 2610 -> 2490, 24576 with 384 row tiles (cp 8, rank 5) 408 -> 383, 24 short sequences of 16
+// heads 57.6 -> 53.  With a CU for every workgroup that build is the slower one: two on one CU leave
+// another idle (256 row tiles, 8192 tokens, cp 4, rank 3: 105 -> 135 us), and kept apart they miss the
+// registers (110).
+inline bool two_per_cu(int d, int64_t workgroups) { return d == 64 && workgroups > 256; }
+
 struct AttnParams {
   const void* q;
   const void* k;
@@ -1551,8 +1560,8 @@ struct OneSegment {
   __device__ __forceinline__ const char* base(int, bool isk) const { return isk ? kb : vb; }
 };
 
-template <typename T, int D, int HP>
-__global__ __launch_bounds__(kPPThreads, 2) void attn_fwd_16bit_vt(AttnParams p) {
+template <typename T, int D, int HP, int WGS = 1>
+__global__ __launch_bounds__(kPPThreads, 2 * WGS) void attn_fwd_16bit_vt(AttnParams p) {
   constexpr int BN = vt_bn<D>();
   constexpr int RB = kPPWaves / HP;  // 32-row blocks per workgroup
   int hg, seq, rt;
@@ -1683,8 +1692,8 @@ struct RingSegments {
   __device__ __forceinline__ int num_pages() const { return p->num_pages; }
 };
 
-template <typename T, int D, int HP, bool PAGED, bool PACK>
-__global__ __launch_bounds__(kPPThreads, 2) void attn_fwd_16bit_sweep(SweepParams p) {
+template <typename T, int D, int HP, bool PAGED, bool PACK, int WGS = 1>
+__global__ __launch_bounds__(kPPThreads, 2 * WGS) void attn_fwd_16bit_sweep(SweepParams p) {
   constexpr int RB = kPPWaves / HP;
   int hg, seq, rt;
   int qs, L;

@@ -226,8 +226,8 @@ struct SplitWork {
   }
 };
 
-template <typename T, int D, int HP, bool PAGED>
-__global__ __launch_bounds__(kPPThreads, 2) void attn_fwd_16bit_sweep_split(SweepSplit sp) {
+template <typename T, int D, int HP, bool PAGED, int WGS = 1>
+__global__ __launch_bounds__(kPPThreads, 2 * WGS) void attn_fwd_16bit_sweep_split(SweepSplit sp) {
   const SweepParams& p = sp.p;
   SplitWork<D, HP, vt_bn<D>(), (int)sizeof(T), PAGED> w;
   if (!w.start(sp)) return;
@@ -353,15 +353,22 @@ int launch_split(const SweepParams& p, const SplitPlan& pl, void* ws, int dtype,
   sp.n_row = pl.n_row;
   sp.per_hg = pl.per_hg;
   void (*fn)(SweepSplit) = nullptr;
+  const int64_t slots = (int64_t)p.n_hg * ((pl.n_row - pl.n_front) * pl.ns_back + pl.n_front * pl.ns_front);
+  const bool two = two_per_cu(d, slots);
 #define FA4CP_PICK_HP(KERNEL, ...)                                                          \
   {                                                                                         \
     if (hp == 4) fn = paged ? KERNEL<__VA_ARGS__, 4, true> : KERNEL<__VA_ARGS__, 4, false>; \
     else if (hp == 2) fn = paged ? KERNEL<__VA_ARGS__, 2, true> : KERNEL<__VA_ARGS__, 2, false>; \
     else fn = paged ? KERNEL<__VA_ARGS__, 1, true> : KERNEL<__VA_ARGS__, 1, false>;         \
   }
+#define FA4CP_PICK_TWO(T, H) \
+  fn = paged ? attn_fwd_16bit_sweep_split<T, 64, H, true, 2> : attn_fwd_16bit_sweep_split<T, 64, H, false, 2>;
 #define FA4CP_PICK_16(T)                                               \
   {                                                                    \
-    if (d == 64) FA4CP_PICK_HP(attn_fwd_16bit_sweep_split, T, 64)        \
+    if (two && hp == 4) FA4CP_PICK_TWO(T, 4)                             \
+    else if (two && hp == 2) FA4CP_PICK_TWO(T, 2)                        \
+    else if (two) FA4CP_PICK_TWO(T, 1)                                   \
+    else if (d == 64) FA4CP_PICK_HP(attn_fwd_16bit_sweep_split, T, 64)   \
     else if (d == 128) FA4CP_PICK_HP(attn_fwd_16bit_sweep_split, T, 128) \
     else FA4CP_PICK_HP(attn_fwd_16bit_sweep_split, T, 256)               \
   }
@@ -374,6 +381,7 @@ int launch_split(const SweepParams& p, const SplitPlan& pl, void* ws, int dtype,
     FA4CP_PICK_16(_Float16)
   }
 #undef FA4CP_PICK_16
+#undef FA4CP_PICK_TWO
 #undef FA4CP_PICK_HP
   hipLaunchKernelGGL(fn, dim3((unsigned)(p.n_hg * pl.per_hg)), dim3(kPPThreads), 0, st, sp);
   return check_launch("ring_sweep_fwd_ws");
