@@ -896,7 +896,8 @@ __device__ __forceinline__ void dkdv_tile(const BwdParams& p, int b, int ns, int
 // each kind double-buffered by block parity: iteration i reads rows(i) and transposed(i - 1)
 // and loads rows(i + 1) and transposed(i) over those of blocks i - 1 and i - 2 (4 x 64.25 KB).
 // (The halves measured 7 % slower at 128, where whole stages fit.)
-template <typename T, int D, bool PAIR>
+// ALT: in pairs of own tiles (see dkdv_tile; up to head dim 128, one sequence), or at 256 in shares.
+template <typename T, int D, bool ALT>
 __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams p) {
   using M = BwdMfma<T>;
   typedef typename M::frag frag;
@@ -905,7 +906,9 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
   constexpr int R = pack_region_bytes<D>();
   constexpr int BB = pack_block_bytes<D>();
   constexpr bool HALVES = D > 128;
-  constexpr bool kShares = !HALVES;  // (at head dim 256 the kernel has no register to spare for them)
+  constexpr bool PAIR = ALT && !HALVES;
+  constexpr bool kParts = ALT && HALVES;  // the shares stay in their slots for bwd_dkdv_sum_kernel
+  constexpr bool kShares = !HALVES || ALT;
   constexpr int HB = 2 * R + 256;   // a half-stage: two regions and the per-row values
   // head dim 256: 1 KB fragments each wavefront loads per half-stage (below it the ninth
   // wavefront loads every fragment of a stage)
@@ -935,8 +938,8 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
   constexpr int OVAL = HALVES ? 2 * R : 4 * R;
 
   int share, tile, kt, seq, kvh, src;
-  dkdv_tile<PAIR>(p, blockIdx.x, kShares && !PAIR ? p.ns : 1, share, tile, kt, seq, kvh, src);
-  // PAIR (one sequence, see dkdv_tile): the distance to the second of the two own tiles
+  dkdv_tile<PAIR>(p, blockIdx.x, PAIR || !kShares ? 1 : p.ns, share, tile, kt, seq, kvh, src);
+  // the distance to the second of the two own tiles
   int next = PAIR && src == p.rank ? p.n_tiles - 1 - 2 * kt : 0;
   auto another = [&]() __attribute__((always_inline)) {
     if (next <= 0) return false;
@@ -1250,14 +1253,21 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
         }
       }
     }
-    if constexpr (kShares) {
-      if (share >= shares || !merge_shares<NDT>(p, tile, share, shares, 8, acc)) continue;
+    if (kShares && share >= shares) continue;
+    if constexpr (kShares && !kParts) {
+      if (!merge_shares<NDT>(p, tile, share, shares, 8, acc)) continue;
     }
     // accumulator register r of lane l: head-dim element 32 dt + 8 (r / 4) + 4h + r % 4 of key
     // `key`; keys no query of this rank attends (past key_lim) get zeros
     if (producer || key >= L) continue;
-    float* const base = pwave ? p.dv[src] : p.dk[src];
-    const int64_t at = ((int64_t)(qs + key) * p.h_kv + kvh) * D;
+    float* base = pwave ? p.dv[src] : p.dk[src];
+    int64_t at = ((int64_t)(qs + key) * p.h_kv + kvh) * D;
+    bool grad16 = p.grad16, add = p.accumulate;
+    if (kParts && shares > 1) {  // dV, then dK of the tile's keys
+      base = p.part + ((int64_t)(tile * p.ns + share) * 2 + (pwave ? 0 : 1)) * kDkdvKeys * D;
+      at = (key - kb0) * D;
+      grad16 = add = false;
+    }
     const float sc = pwave ? 1.f : p.scale;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
@@ -1265,16 +1275,52 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
       for (int g = 0; g < 4; ++g) {
         const int d = 32 * dt + 8 * g + 4 * h;
         f32x4 a = {acc[dt][4 * g] * sc, acc[dt][4 * g + 1] * sc, acc[dt][4 * g + 2] * sc, acc[dt][4 * g + 3] * sc};
-        if (p.grad16) {
+        if (grad16) {
           typedef T t4 __attribute__((ext_vector_type(4)));
           *reinterpret_cast<t4*>(reinterpret_cast<T*>(base) + at + d) = t4{(T)a[0], (T)a[1], (T)a[2], (T)a[3]};
         } else {
           float* const o = base + at + d;
-          if (p.accumulate) a += *reinterpret_cast<const f32x4*>(o);
+          if (add) a += *reinterpret_cast<const f32x4*>(o);
           *reinterpret_cast<f32x4*>(o) = a;
         }
       }
   } while (PAIR && another());
+}
+
+// dK / dV of the tiles whose shares are in their slots (head dim 256): eight workgroups per tile, 16 keys
+// each, add the shares in order.  HBM-bound, 256 KB a share.  In the kernel above, as below head dim 256, the
+// last share's summing costs registers that its loop does not have (250 of 256).  Backward, unshared and
+// shared: 8192 tokens (H 16/2, cp 4, rank 1, 128 key tiles) 1230 and 802 us, 16384 (H 8/1, cp 8, rank 7) 1259 and
+// 858, 2048 (H 8/2) 230 and 153.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void bwd_dkdv_sum_kernel(BwdParams p) {
+  constexpr int kKeys = kDkdvKeys / 8, kRow = D / 4;  // four-element chunks of a row
+  int share, tile, kt, seq, kvh, src, qs, L, lo, hi, shares;
+  dkdv_tile<false>(p, blockIdx.x >> 3, 1, share, tile, kt, seq, kvh, src);
+  seq_range(p.cu, seq, p.total, FA4CP_SEL_ALL, qs, L);
+  const int kb0 = kt * kDkdvKeys, key0 = (int)(blockIdx.x & 7) * kKeys;
+  const StepPairs sp = step_pairs(p.rank, p.S, src, L);
+  if (kb0 + key0 >= L || kb0 >= sp.key_lim) return;
+  const int row_begin = max(sp.row_min, sp.causal ? kb0 : 0) / kBwdRows * kBwdRows;
+  take_share(p, 0, (L - row_begin + kBwdRows - 1) / kBwdRows * p.group, lo, hi, shares);
+  if (shares == 1) return;  // (its workgroup wrote the gradient)
+  const int keys = min(kKeys, L - kb0 - key0);
+  for (int i = threadIdx.x; i < 2 * keys * kRow; i += 256) {
+    const int which = i / (keys * kRow), e = i - which * keys * kRow;  // dV, dK
+    const float* part = p.part + (((int64_t)tile * p.ns * 2 + which) * kDkdvKeys + key0) * D + 4 * e;
+    f32x4 a = *reinterpret_cast<const f32x4*>(part);
+    for (int j = 1; j < shares; ++j) a += *reinterpret_cast<const f32x4*>(part + (int64_t)j * 2 * kDkdvKeys * D);
+    float* const base = which ? p.dk[src] : p.dv[src];
+    const int64_t at = ((int64_t)(qs + kb0 + key0 + e / kRow) * p.h_kv + kvh) * D + e % kRow * 4;
+    if (p.grad16) {
+      typedef T t4 __attribute__((ext_vector_type(4)));
+      *reinterpret_cast<t4*>(reinterpret_cast<T*>(base) + at) = t4{(T)a[0], (T)a[1], (T)a[2], (T)a[3]};
+    } else {
+      float* const o = base + at;
+      if (p.accumulate) a += *reinterpret_cast<const f32x4*>(o);
+      *reinterpret_cast<f32x4*>(o) = a;
+    }
+  }
 }
 
 // Tiles of the two gradient kernels and the workgroups that share one.
@@ -1308,8 +1354,7 @@ BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
   const int L = nseq > 1 ? std::max(1, a.total / nseq) : longest;  // an average sequence when packed
   const int late = a.cp_size - 1 - a.cp_rank;
   auto blocks = [](int n) { return (n + kBwdRows - 1) / kBwdRows; };
-  if (a.d == 256) return pl;  // (its kernels have no register to spare for the shares)
-  if (pl.dq_tiles <= kMaxTiles) {
+  if (pl.dq_tiles <= kMaxTiles && a.d < 256) {  // (at 256 dq's kernel has no register to spare for shares)
     auto cost = [&](int len, int rt, bool back) {
       return blocks(std::min((rt + 1) * rows, len)) + a.cp_rank * blocks(len / 2) + (back ? late * blocks(len) : 0);
     };
@@ -1412,8 +1457,10 @@ int launch_bwd(const BwdParams& base, const BwdPlan& pl, hipStream_t st) {
   const bool pair = D <= 128 && p.nseq == 1 && pl.kv_tiles > kCus;
   const int64_t kv_blocks = pair ? pl.kv_tiles - (int64_t)(p.n_tiles / 2) * p.h_kv : pl.kv_tiles * p.ns;
   if (kv_blocks > 0x7fffffffLL) return set_error(FA4CP_EINVAL, "ring_sweep_bwd: too many key tiles");
-  auto* const dkdv = pair ? bwd_dkdv_kernel<T, D, (D <= 128)> : bwd_dkdv_kernel<T, D, false>;
+  auto* const dkdv = pair || (D > 128 && p.ns > 1) ? bwd_dkdv_kernel<T, D, true> : bwd_dkdv_kernel<T, D, false>;
   hipLaunchKernelGGL(dkdv, dim3((unsigned)kv_blocks), dim3(D > 128 ? 512 : 576), 0, st, p);
+  if (D > 128 && p.ns > 1)
+    hipLaunchKernelGGL((bwd_dkdv_sum_kernel<T, D>), dim3((unsigned)(8 * pl.kv_tiles)), dim3(256), 0, st, p);
   return check_launch("ring_sweep_bwd");
 }
 
