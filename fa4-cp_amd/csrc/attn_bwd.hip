@@ -193,6 +193,18 @@ __device__ __forceinline__ void put_grad(const BwdParams& p, float* base, int64_
   else base[at] = p.accumulate ? base[at] + x : x;
 }
 
+template <typename T>
+__device__ __forceinline__ void put_grad4(const BwdParams& p, float* base, int64_t at, f32x4 a) {
+  if (p.grad16) {
+    typedef T t4 __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<t4*>(reinterpret_cast<T*>(base) + at) = t4{(T)a[0], (T)a[1], (T)a[2], (T)a[3]};
+  } else {
+    float* const o = base + at;
+    if (p.accumulate) a += *reinterpret_cast<const f32x4*>(o);
+    *reinterpret_cast<f32x4*>(o) = a;
+  }
+}
+
 // Which local rows attend which keys of source `src` (one sequence of L rows): keys
 // [0, key_lim), rows [row_min, L), and key <= row when causal.
 struct StepPairs {
@@ -206,6 +218,19 @@ __device__ __forceinline__ StepPairs step_pairs(int rank, int S, int src, int L)
   sp.key_lim = (s != 0 && s <= rank) ? (L >> 1) : L;
   sp.row_min = s > rank ? (L >> 1) : 0;
   return sp;
+}
+
+// Keys of step s that the 32 rows from r0 on of a sequence of L see (0: none), and the 32-key blocks of
+// all steps.
+__device__ __forceinline__ int row_block_keys(const BwdParams& p, int s, int L, int r0) {
+  const StepPairs sp = step_pairs(p.rank, p.S, p.rank - s < 0 ? p.rank - s + p.S : p.rank - s, L);
+  if (r0 + kBwdRows <= sp.row_min) return 0;
+  return sp.causal ? min(sp.key_lim, r0 + kBwdRows) : sp.key_lim;
+}
+__device__ __forceinline__ int row_block_blocks(const BwdParams& p, int L, int r0) {
+  int n = 0;
+  for (int s = 0; s < p.S; ++s) n += (row_block_keys(p, s, L, r0) + kBwdRows - 1) / kBwdRows;
+  return n;
 }
 
 template <typename T>
@@ -365,7 +390,7 @@ __global__ __launch_bounds__(256) void bwd_pack_kv_kernel(BwdParams p) {
 // of block i and dQ of block i - 1, so neither wavefront of a pair waits for the other within
 // an iteration.  One barrier per iteration: block i + 1 has landed, P^T of block i is in LDS,
 // and the stage of block i - 1 is free for block i + 2.
-template <typename T, int D, int HP>
+template <typename T, int D, int HP, bool SHARES>
 __global__ __launch_bounds__(128 * HP) void bwd_dq_pair_kernel(BwdParams p) {
   using M = BwdMfma<T>;
   typedef typename M::frag frag;
@@ -391,7 +416,10 @@ __global__ __launch_bounds__(128 * HP) void bwd_dq_pair_kernel(BwdParams p) {
   int b = blockIdx.x;
   const int hg = b % n_hg;
   b /= n_hg;
-  const int rt = b % p.n_tiles;
+  const int share = SHARES ? b % p.ns : 0;
+  if (SHARES) b /= p.ns;
+  const int tile = b * n_hg + hg;
+  const int rt = p.n_tiles - 1 - b % p.n_tiles;  // longest first
   const int seq = b / p.n_tiles;
   const int64_t pstart = vt_seq_start(p.cu, seq, p.total, FA4CP_SEL_ALL) / kBwdRows;
   int qs, L;
@@ -428,13 +456,13 @@ __global__ __launch_bounds__(128 * HP) void bwd_dq_pair_kernel(BwdParams p) {
 
   // the key blocks of every step the row block attends, in order: (step, first key)
   auto src_of = [&](int s) { return p.rank - s < 0 ? p.rank - s + p.S : p.rank - s; };
-  auto key_end_of = [&](int s) {  // keys of step s the rows see (0: no row attends it)
-    const StepPairs sp = step_pairs(p.rank, p.S, src_of(s), L);
-    if (r0 + kBwdRows <= sp.row_min) return 0;
-    return sp.causal ? min(sp.key_lim, r0 + kBwdRows) : sp.key_lim;
-  };
-  int n_blk = 0;
-  for (int s = 0; s < p.S; ++s) n_blk += (key_end_of(s) + kBwdRows - 1) / kBwdRows;
+  auto key_end_of = [&](int s) { return row_block_keys(p, s, L, r0); };
+  int n_blk = row_block_blocks(p, L, r0), lo = 0, shares = 1;
+  if (SHARES) {
+    int hi;
+    if (!take_share(p, share, n_blk, lo, hi, shares)) return;
+    n_blk = hi - lo;
+  }
   struct Cursor {
     int s, k0, kend;
   };
@@ -445,8 +473,20 @@ __global__ __launch_bounds__(128 * HP) void bwd_dq_pair_kernel(BwdParams p) {
       if (cu.s < p.S) cu.kend = key_end_of(cu.s);
     }
   };
-  Cursor lc{0, 0, key_end_of(0)};  // the next block to load
-  settle(lc);
+  auto seek = [&]() {  // block lo
+    Cursor cu{0, 0, key_end_of(0)};
+    settle(cu);
+    if (SHARES) {
+      for (int x = lo; x > 0;) {
+        const int m = min(x, (cu.kend - cu.k0 + kBwdRows - 1) / kBwdRows);
+        cu.k0 += m * kBwdRows;
+        x -= m;
+        settle(cu);
+      }
+    }
+    return cu;
+  };
+  Cursor lc = seek();  // the next block to load
   auto load = [&](int bi) {
     const char* g = p.pkv + (((int64_t)src_of(lc.s) * p.h_kv + kvh) * p.n_pb + pstart + lc.k0 / kBwdRows) * KB;
     const __amdgpu_buffer_rsrc_t rs = make_rsrc32(uniform_ptr(g), KB);
@@ -460,8 +500,7 @@ __global__ __launch_bounds__(128 * HP) void bwd_dq_pair_kernel(BwdParams p) {
   auto run = [&](auto role) {
     constexpr bool SW = decltype(role)::value;
     f32x16 dpt;                       // second wavefront: dP^T of the previous block
-    Cursor cc{0, 0, key_end_of(0)};  // first wavefront: the block of the MFMA phase
-    settle(cc);
+    Cursor cc = seek();  // first wavefront: the block of the MFMA phase
     load(0);
     __builtin_amdgcn_s_waitcnt(kWaitAll);
     wg_barrier();
@@ -537,6 +576,14 @@ __global__ __launch_bounds__(128 * HP) void bwd_dq_pair_kernel(BwdParams p) {
     else run(std::false_type{});
   }
   if (swave) return;
+  if (SHARES && shares > 1) {  // left for bwd_dq_sum_kernel
+    float* const part = p.part + (((int64_t)tile * p.ns + share) * HP + w % HP) * kBwdRows * D + lq;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) part[(8 * (r >> 2) + 4 * h + (r & 3)) * D + 32 * dt] = acc[dt][r] * p.scale;
+    return;
+  }
   // accumulator register r of lane l: query row 8 (r / 4) + 4h + r % 4, column 32 dt + lq
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
@@ -545,6 +592,30 @@ __global__ __launch_bounds__(128 * HP) void bwd_dq_pair_kernel(BwdParams p) {
     const int64_t at = ((int64_t)(qs + row) * p.h_q + head) * D + lq;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) put_grad<T>(p, p.dq, at + 32 * dt, acc[dt][r] * p.scale);
+  }
+}
+
+// dQ of the row tiles whose shares are in their slots (head dim 256): one workgroup per tile and query
+// head adds them in order.  HBM-bound, 32 KB a share and head.  Backward, unshared (longest tiles last) and
+// shared: 16384 tokens (H 16/2, cp 8, rank 3: 256 row tiles, those of the back half 3.6 times as long) 1454 and 1333
+// us, 8192 (H 16/2, cp 4, rank 1) 802 and 726, 2048 (H 8/2) 153 and 111.  Where they are not shared the longest
+// first alone gives 2-3 % (49152 tokens, H 32/8, cp 4: 34.6 -> 34.0 ms).
+template <typename T, int D, int HP>
+__global__ __launch_bounds__(256) void bwd_dq_sum_kernel(BwdParams p) {
+  const int n_hg = p.h_q / HP, tile = blockIdx.x / HP, j = blockIdx.x % HP;
+  const int rt = p.n_tiles - 1 - tile / n_hg % p.n_tiles, seq = tile / n_hg / p.n_tiles;
+  int qs, L, lo, hi, shares;
+  seq_range(p.cu, seq, p.total, FA4CP_SEL_ALL, qs, L);
+  const int r0 = rt * kBwdRows;
+  if (r0 >= L) return;
+  take_share(p, 0, row_block_blocks(p, L, r0), lo, hi, shares);
+  if (shares == 1) return;  // (its workgroup wrote the gradient)
+  const float* part = p.part + ((int64_t)tile * p.ns * HP + j) * kBwdRows * D;
+  const int n = min(kBwdRows, L - r0) * (D / 4);  // four-element chunks
+  for (int e = threadIdx.x; e < n; e += 256) {
+    f32x4 a = *reinterpret_cast<const f32x4*>(part + 4 * e);
+    for (int i = 1; i < shares; ++i) a += *reinterpret_cast<const f32x4*>(part + (int64_t)i * HP * kBwdRows * D + 4 * e);
+    put_grad4<T>(p, p.dq, ((int64_t)(qs + r0 + e / (D / 4)) * p.h_q + tile % n_hg * HP + j) * D + e % (D / 4) * 4, a);
   }
 }
 
@@ -1312,14 +1383,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_sum_kernel(BwdParams p) {
     for (int j = 1; j < shares; ++j) a += *reinterpret_cast<const f32x4*>(part + (int64_t)j * 2 * kDkdvKeys * D);
     float* const base = which ? p.dk[src] : p.dv[src];
     const int64_t at = ((int64_t)(qs + kb0 + key0 + e / kRow) * p.h_kv + kvh) * D + e % kRow * 4;
-    if (p.grad16) {
-      typedef T t4 __attribute__((ext_vector_type(4)));
-      *reinterpret_cast<t4*>(reinterpret_cast<T*>(base) + at) = t4{(T)a[0], (T)a[1], (T)a[2], (T)a[3]};
-    } else {
-      float* const o = base + at;
-      if (p.accumulate) a += *reinterpret_cast<const f32x4*>(o);
-      *reinterpret_cast<f32x4*>(o) = a;
-    }
+    put_grad4<T>(p, base, at, a);
   }
 }
 
@@ -1331,7 +1395,7 @@ struct BwdPlan {
 };
 
 // A 32-key block of dq takes 1.2 us and a 32-row block of dk / dv 1.02 (measured, head dim 128, the
-// chip full).  dq's row tiles are shared wherever best_shares finds it faster (backward, GPU time in
+// chip full; dq at 256, half the rows, 1.7).  dq's row tiles are shared wherever best_shares finds it faster (backward, GPU time in
 // us, shares of the back-half / other row tiles: 8192 tokens, H 32/8, cp 4, rank 1: none 622, 2/1 584,
 // 2/2 564 (chosen), 3/2 589; 16384, cp 8, rank 3: 1098, 1046, 1000 (chosen), 1054; rank 7, equal row
 // tiles: 985 (chosen), 1071, 992, 1050).  dk / dv's key tiles only where all shares run at once: the
@@ -1354,7 +1418,7 @@ BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
   const int L = nseq > 1 ? std::max(1, a.total / nseq) : longest;  // an average sequence when packed
   const int late = a.cp_size - 1 - a.cp_rank;
   auto blocks = [](int n) { return (n + kBwdRows - 1) / kBwdRows; };
-  if (pl.dq_tiles <= kMaxTiles && a.d < 256) {  // (at 256 dq's kernel has no register to spare for shares)
+  if (pl.dq_tiles <= kMaxTiles) {
     auto cost = [&](int len, int rt, bool back) {
       return blocks(std::min((rt + 1) * rows, len)) + a.cp_rank * blocks(len / 2) + (back ? late * blocks(len) : 0);
     };
@@ -1366,7 +1430,7 @@ BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
     w.top2 = fronts ? cost(L, fronts - 1, false) : 0;
     w.avg2 = fronts ? 0.5f * (w.top2 + cost(L, 0, false)) : 0.f;
     w.n2 = (a.h_q / hp) * fronts * nseq;
-    w.us = 1.2f * a.d / 128.f;
+    w.us = a.d == 256 ? 1.7f : 1.2f * a.d / 128.f;
     w.merge = 5.f;
     w.read = 1.25f * a.d / 128.f;
     w.packed = nseq > 1;
@@ -1404,6 +1468,18 @@ int64_t share_bytes(const BwdPlan& pl, int d) {
   return share_count_bytes(pl) + std::max(dq, kv) * 8 * 32 * d * 4;
 }
 
+// dq at head dim 256, and the sum of its shares.
+template <typename T, int D, int HP>
+void launch_dq_pair(const BwdParams& p, int64_t blocks, hipStream_t st) {
+  const dim3 grid((unsigned)blocks), block(128 * HP);
+  if (p.ns == 1) {
+    hipLaunchKernelGGL((bwd_dq_pair_kernel<T, D, HP, false>), grid, block, 0, st, p);
+  } else {
+    hipLaunchKernelGGL((bwd_dq_pair_kernel<T, D, HP, true>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((bwd_dq_sum_kernel<T, D, HP>), dim3((unsigned)(blocks / p.ns * HP)), dim3(256), 0, st, p);
+  }
+}
+
 template <typename T, int D>
 int launch_bwd(const BwdParams& base, const BwdPlan& pl, hipStream_t st) {
   BwdParams p = base;
@@ -1431,9 +1507,9 @@ int launch_bwd(const BwdParams& base, const BwdPlan& pl, hipStream_t st) {
     if (kv_pack_blocks > 0x7fffffffLL) return set_error(FA4CP_EINVAL, "ring_sweep_bwd: too many key blocks");
     hipLaunchKernelGGL((bwd_pack_kv_kernel<T, D>), dim3((unsigned)kv_pack_blocks), dim3(256), 0, st, p);
     switch (hp) {
-      case 4: hipLaunchKernelGGL((bwd_dq_pair_kernel<T, D, 4>), dim3((unsigned)dq_blocks), dim3(512), 0, st, p); break;
-      case 2: hipLaunchKernelGGL((bwd_dq_pair_kernel<T, D, 2>), dim3((unsigned)dq_blocks), dim3(256), 0, st, p); break;
-      default: hipLaunchKernelGGL((bwd_dq_pair_kernel<T, D, 1>), dim3((unsigned)dq_blocks), dim3(128), 0, st, p); break;
+      case 4: launch_dq_pair<T, D, 4>(p, dq_blocks, st); break;
+      case 2: launch_dq_pair<T, D, 2>(p, dq_blocks, st); break;
+      default: launch_dq_pair<T, D, 1>(p, dq_blocks, st); break;
     }
   } else {  // the packed K / V blocks, then four wavefronts over 4 / hp row blocks
     const int64_t kv_pack_blocks = (int64_t)p.S * p.h_kv * p.nseq * p.n_tiles;
