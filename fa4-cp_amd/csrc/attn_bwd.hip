@@ -1402,7 +1402,11 @@ struct BwdPlan {
 // workgroups stream the query blocks in step, and shares at other blocks cost more in L2
 // misses than the even split gains (8192 tokens: none 622, two shares 628-651, three 634-650; 24576
 // tokens, H 16/2: 1311, 1337-1389), but 32 key tiles leave the chip idle (2048 tokens, H 8/2: 138,
-// 120, 113; four 112).
+// 120, 113; four 112).  At head dim 256 a block takes the MFMAs twice as long and the even split wins up to
+// 256 tiles, of up to four times as many shares as CUs (backward: 16384 tokens, H 16/2, cp 8, rank 3, 256 tiles
+// 1333 and 1165; 8192, cp 4, 128 tiles: two shares 727, up to eight 610; four sequences, H 8/2, 273 and 205),
+// not beyond (32768 tokens, cp 4, 512 tiles 8450 and 8559).  There a share costs 0.08 us for its 256 KB (without
+// that, 3072 tokens, H 24/8, cp 8, rank 6, short tiles: unshared 266, shared 281).
 BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
   constexpr int kMaxTiles = 1024, kMaxSlots = 2048;  // slots of 128 KB at head dim 128
   BwdPlan pl;
@@ -1437,7 +1441,8 @@ BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
     w.free2 = true;
     pl.dq = best_shares(w, std::min<int64_t>(kMaxShares, kMaxSlots / pl.dq_tiles));
   }
-  if (2 * pl.kv_tiles <= kCus) {
+  const bool wide = a.d == 256;
+  if (2 * pl.kv_tiles <= (wide ? 2 : 1) * kCus) {
     // earlier sources: every row, the front half of the keys; own: half of the rows on average, the
     // first half of the tiles three quarters; later sources: the back-half rows
     const int kts = (L + kDkdvKeys - 1) / kDkdvKeys, own1 = (kts + 1) / 2;
@@ -1450,12 +1455,13 @@ BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
     w.top2 = (int)(0.5f * all);
     w.n2 = a.h_kv * nseq * (late * kts + kts - own1);
     w.avg2 = w.n2 ? all * (0.5f * late * kts + 0.25f * (kts - own1)) / (late * kts + kts - own1) : 0.f;
-    w.us = 1.02f * a.d / 128.f;
-    w.merge = 5.f;
-    w.read = 1.25f * a.d / 128.f;
+    w.us = wide ? 1.75f : 1.02f * a.d / 128.f;
+    w.merge = wide ? 6.f : 5.f;
+    w.read = wide ? 0.f : 1.25f * a.d / 128.f;
+    w.slot = wide ? 0.08f : 0.f;  // 256 KB each
     w.packed = nseq > 1;
     w.free2 = true;
-    pl.kv = best_shares(w, std::min<int64_t>(kMaxShares, kCus / pl.kv_tiles));
+    pl.kv = best_shares(w, std::min<int64_t>(kMaxShares, (wide ? 4 : 1) * kCus / pl.kv_tiles));
   }
   return pl;
 }

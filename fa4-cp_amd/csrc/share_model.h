@@ -19,7 +19,8 @@ struct ShareLoad {
   float avg2;
   int n2;
   float us;           // microseconds per step
-  float merge, read;  // merging k shares takes merge + k read microseconds
+  float merge, read;  // merging k shares takes merge + k read microseconds,
+  float slot = 0.f;   // and `slot` more for every share of the launch (written out and read by another)
   bool packed;        // tiles of several sequences, whose lengths only the device knows: the classes are guesses
   bool free2;         // the second class's shares are chosen apart (false: chunks as long as the first one's)
 };
@@ -56,7 +57,7 @@ inline Shares best_shares(const ShareLoad& w, int most = kMaxShares) {
                          : std::max(longs, (n1 * c1 + n2 * c2) / kCus + 0.5f * c2);
       }
       t = std::max(t, (float)w.top / k + over);
-      if (k > 1) t += (w.merge + w.read * k) / w.us;
+      if (k > 1) t += (w.merge + w.read * k + w.slot * (n1 + n2)) / w.us;
       if (k == 1) one = least = t;
       else if (t < least) {
         least = t;

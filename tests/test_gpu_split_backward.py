@@ -27,7 +27,7 @@ CASES = [  # (local lens, H, H_kv, D, cp, rank, dtype, shared)
     ([512], 8, 2, 256, 4, 1, torch.bfloat16, True),    # head dim 256: dk / dv, summed by a kernel of its own
     ([386], 8, 1, 256, 8, 5, torch.float16, True),     # a partial key tile, tiles no row attends
     ([300, 0, 70, 2], 4, 1, 256, 4, 3, torch.bfloat16, True),  # packed
-    ([2048], 8, 8, 256, 2, 0, torch.bfloat16, False),  # more key tiles than the chip can share
+    ([2048], 16, 16, 256, 2, 0, torch.bfloat16, False),  # more tiles than are shared
     ([2], 4, 2, 128, 4, 2, torch.bfloat16, False),
 ]
 
