@@ -18,7 +18,8 @@
 // source's gradient (a multi-GPU ring sends them back to their owners).
 //
 // Where the tiles of the last two kernels are few, several workgroups share one's blocks
-// (take_share) and the last of them sums the parts (merge_shares).
+// (take_share) and the last of them sums the parts (merge_shares); at head dim 256 the parts are
+// left to one more launch each (bwd_dq_sum_kernel, bwd_dkdv_sum_kernel).
 //
 // Four launches:
 // * bwd_pack_kernel (HBM-bound): delta, and every 32-row block of Q and dO copied into the
@@ -1471,7 +1472,8 @@ int64_t share_count_bytes(const BwdPlan& pl) { return (share_words(pl) * 4 + 255
 int64_t share_bytes(const BwdPlan& pl, int d) {
   if (share_words(pl) == 0) return 0;
   const int64_t dq = pl.dq.k > 1 ? pl.dq_tiles * pl.dq.k : 0, kv = pl.kv.k > 1 ? pl.kv_tiles * pl.kv.k : 0;
-  return share_count_bytes(pl) + std::max(dq, kv) * 8 * 32 * d * 4;
+  const int64_t dq_blocks = d == 256 ? 4 : 8;  // 32-row blocks of a dq slot, at most
+  return share_count_bytes(pl) + std::max(dq * dq_blocks, kv * 8) * 32 * d * 4;
 }
 
 // dq at head dim 256, and the sum of its shares.

@@ -314,7 +314,8 @@ int64_t fa4cp_ring_sweep_workspace_bytes(const fa4cp_sweep_args* args, int32_t* 
  * per source) there; it holds nothing across calls.  With accumulate != 0 the results are
  * added to dq / dk / dv instead of stored (summing the contributions of several ranks, as a
  * ring's backward does).  q, dout and out may have any row and head stride; k / v shards
- * share strides and the cu layout of fa4cp_ring_sweep_fwd.  Four launches on `stream`.
+ * share strides and the cu layout of fa4cp_ring_sweep_fwd.  Four launches on `stream` (head dim 256 with
+ * shares: up to six).
  */
 typedef struct fa4cp_sweep_bwd_args {
   const void* q;    /* [total] x h_q x d */
