@@ -57,6 +57,10 @@ inline Shares best_shares(const ShareLoad& w, int most = kMaxShares) {
                          : std::max(longs, (n1 * c1 + n2 * c2) / kCus + 0.5f * c2);
       }
       t = std::max(t, (float)w.top / k + over);
+      // The forward's tiles of both classes cut up, in more workgroups than CUs: 10-20 % over the estimate
+      // (their parts go to memory while the next workgroups start).  13664 tokens (H 32/8, cp 8, rank 5):
+      // unshared 244 us, in halves 258; 16384: 287, 298; with a larger gain ahead, 12288: 200, in 3 and 2 181.
+      if (!w.free2 && !w.packed && k2 > 1 && n1 + n2 > kCus) t *= 1.2f;
       if (k > 1) t += (w.merge + w.read * k + w.slot * (n1 + n2)) / w.us;
       if (k == 1) one = least = t;
       else if (t < least) {
