@@ -320,12 +320,15 @@ def ring_sweep(local_q: torch.Tensor, local_k: torch.Tensor, local_v: torch.Tens
     h_kv = ks[0].shape[1]
     shape, k_stride, v_stride, v_dtype = (total, h_kv, d), ks[0].stride(), vs[0].stride(), vs[0].dtype
     for k, v in zip(ks, vs):
-        assert k.shape == shape and v.shape == shape and k.dtype == dtype
+        assert k.shape == shape and k.dtype == dtype
         assert k.stride() == k_stride, "all K shards must share strides"
-        assert v.stride() == v_stride and v.dtype == v_dtype, "all V shards must share strides and dtype"
+        # (raised and not asserted, as every check of what the V^T launch reads: also under python -O)
+        if v.shape != shape or v.stride() != v_stride or v.dtype != v_dtype:
+            raise AssertionError(f"V shards must be [{total}, {h_kv}, {d}] and share strides and dtype")
     # the sweep's arguments carry K's row and head strides only: D must be contiguous
-    assert k_stride[2] == 1 and v_stride[2] == 1, "K and V shards must be contiguous in D"
-    assert vs[0].device == local_q.device, f"V must be on {local_q.device}"
+    assert k_stride[2] == 1, "K shards must be contiguous in D"
+    if v_stride[2] != 1 or not vs[0].is_cuda or vs[0].device != local_q.device:
+        raise AssertionError(f"V shards must be contiguous in D and on {local_q.device}")
 
     def transpose(*args):
         transpose_v_into(vs, *args)
@@ -396,9 +399,11 @@ def _sweep_launch(local_q: torch.Tensor, q_stride: Tuple[int, ...], k_ptrs: List
             f"lse must be [{total}, {h_q}] float32 on {dev} with unit head stride"
     nseq, longest = 1, total
     if cu_seqlens is not None:
-        assert cu_seqlens.dtype == torch.int32 and cu_seqlens.device == dev and cu_seqlens.is_contiguous() \
-            and cu_seqlens.dim() == 1 and cu_seqlens.shape[0] >= 2, "cu_seqlens must be contiguous int32 [num_seq + 1] on the device"
-        assert max_seqlen is not None, "max_seqlen required when cu_seqlens is given"
+        if cu_seqlens.dtype != torch.int32 or cu_seqlens.device != dev or not cu_seqlens.is_contiguous() \
+                or cu_seqlens.dim() != 1 or cu_seqlens.shape[0] < 2:
+            raise AssertionError("cu_seqlens must be contiguous int32 [num_seq + 1] on the device")
+        if max_seqlen is None:
+            raise AssertionError("max_seqlen required when cu_seqlens is given")
         nseq, longest = cu_seqlens.shape[0] - 1, int(max_seqlen)
     stride = lib.fa4cp_vt_min_d_stride(total, nseq)
     o_stride = out.stride()

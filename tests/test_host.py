@@ -6,6 +6,7 @@ import ctypes
 import os
 import re
 import subprocess
+import sys
 import tempfile
 
 import pytest
@@ -311,6 +312,67 @@ def test_ring_sweep_workspace_contract():
     for ws, n in ((fake, need - 1), (fake + 8, need)):
         rc = lib.fa4cp_ring_sweep_fwd_ws(ctypes.byref(args()), None, ws, n, None)
         assert rc != 0 and b"workspace" in lib.fa4cp_last_error()
+
+
+_CHECKED_CODE = """
+import sys, torch
+sys.path.insert(0, sys.argv[1])
+from fa4_ring import RingConfig, LocalKVRing, ring_attention as RA
+
+assert False, "python -O strips this"
+
+class Device(torch.Tensor):  # a host tensor that says it is on a GPU
+    is_cuda = property(lambda self: True)
+
+class Library:  # nothing may be queued
+    def __getattr__(self, name):
+        if name == "fa4cp_vt_min_d_stride":
+            return lambda t, n: (t + 128 * n + 127) // 128 * 128
+        if name == "fa4cp_ring_sweep_workspace_bytes":
+            return lambda a, w: 0
+        raise SystemError("reached " + name)
+
+RA._lib.load = lambda: Library()
+dev = lambda x: x.as_subclass(Device)
+bf = torch.bfloat16
+t = lambda *s, dtype=bf: dev(torch.zeros(*s, dtype=dtype))
+q, k, v, cu = t(64, 4, 128), t(64, 2, 128), t(64, 2, 128), dev(torch.tensor([0, 32, 64], dtype=torch.int32))
+vs = lambda x: [v, x, v]
+cases = {
+    "good": (vs(v), cu, 32),
+    "v on the host": ([torch.zeros(64, 2, 128, dtype=bf)] * 3, cu, 32),
+    "v shape": (vs(t(62, 2, 128)), cu, 32),
+    "v strides": (vs(t(2, 64, 128).transpose(0, 1)), cu, 32),
+    "v dtype": (vs(t(64, 2, 128, dtype=torch.float16)), cu, 32),
+    "v in d": ([t(64, 128, 2).transpose(1, 2)] * 3, cu, 32),
+    "cu dtype": (vs(v), cu.long(), 32),
+    "cu device": (vs(v), torch.empty(3, dtype=torch.int32, device="meta"), 32),
+    "cu strided": (vs(v), dev(torch.zeros(6, dtype=torch.int32))[::2], 32),
+    "cu dims": (vs(v), cu.view(1, 3), 32),
+    "cu empty": (vs(v), cu[:1], 32),
+    "max_seqlen": (vs(v), cu, None),
+}
+for name, (v_shards, cu_, longest) in cases.items():
+    ring = LocalKVRing([k] * 3, [v] * 3)
+    ring.v = v_shards
+    try:
+        RA.ring_sweep(q, k, v_shards[0], RingConfig(cp_size=3, cp_rank=0), ring, cu_, longest)
+        print(name, "ran")
+    except AssertionError:
+        print(name, "refused")
+    except Exception as e:
+        print(name, e)
+"""
+
+
+def test_sweep_checks_hold_without_assert_statements():
+    """What the V^T launch reads through the shards and cu_seqlens is checked by code that python -O
+    keeps: a bad one is refused before anything is queued."""
+    out = subprocess.run([sys.executable, "-O", "-c", _CHECKED_CODE, os.path.join(ROOT, "fa4-cp_amd")], check=True,
+                         capture_output=True, text=True, env={**os.environ, "HIP_VISIBLE_DEVICES": ""}).stdout
+    lines = out.split("\n")[:-1]
+    assert lines[0] == "good reached fa4cp_transpose_v_ring"
+    assert len(lines) == 12 and all(x.endswith(" refused") for x in lines[1:]), out
 
 
 @pytest.mark.parametrize("struct,cname", [(_lib.AttnArgs, "fa4cp_attn_args"),
