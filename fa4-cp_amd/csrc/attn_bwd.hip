@@ -44,14 +44,11 @@
 // fragment of a packed block: no transposing LDS read is left.
 #include <type_traits>
 
+#include "attn_plan.h"
 #include "common.h"
-#include "share_model.h"
 
 namespace fa4cp {
 namespace {
-
-constexpr int kBwdRows = 32;  // query rows (dq) or keys (dk/dv) per wavefront
-constexpr int kDkdvKeys = 4 * kBwdRows;  // keys per dk/dv workgroup
 
 // A packed block: rows [32 b, 32 b + 32) of one sequence and one query head in four regions of
 // D / 16 MFMA operand fragments of 1 KB (lane l's 16 bytes at 16 l), then 256 bytes of
@@ -1388,85 +1385,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_sum_kernel(BwdParams p) {
   }
 }
 
-// Tiles of the two gradient kernels and the workgroups that share one.
-struct BwdPlan {
-  int64_t dq_tiles = 0, kv_tiles = 0;
-  int dq_rows = 0;  // rows of a dq tile
-  Shares dq, kv;
-};
-
-// A 32-key block of dq takes 1.2 us and a 32-row block of dk / dv 1.02 (measured, head dim 128, the
-// chip full; dq at 256, half the rows, 1.7).  dq's row tiles are shared wherever best_shares finds it faster (backward, GPU time in
-// us, shares of the back-half / other row tiles: 8192 tokens, H 32/8, cp 4, rank 1: none 622, 2/1 584,
-// 2/2 564 (chosen), 3/2 589; 16384, cp 8, rank 3: 1098, 1046, 1000 (chosen), 1054; rank 7, equal row
-// tiles: 985 (chosen), 1071, 992, 1050).  dk / dv's key tiles only where all shares run at once: the
-// workgroups stream the query blocks in step, and shares at other blocks cost more in L2
-// misses than the even split gains (8192 tokens: none 622, two shares 628-651, three 634-650; 24576
-// tokens, H 16/2: 1311, 1337-1389), but 32 key tiles leave the chip idle (2048 tokens, H 8/2: 138,
-// 120, 113; four 112).  At head dim 256 a block takes the MFMAs twice as long and the even split wins up to
-// 256 tiles, of up to four times as many shares as CUs (backward: 16384 tokens, H 16/2, cp 8, rank 3, 256 tiles
-// 1333 and 1165; 8192, cp 4, 128 tiles: two shares 727, up to eight 610; four sequences, H 8/2, 273 and 205),
-// not beyond (32768 tokens, cp 4, 512 tiles 8450 and 8559).  There a share costs 0.08 us for its 256 KB (without
-// that, 3072 tokens, H 24/8, cp 8, rank 6, short tiles: unshared 266, shared 281).
-BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
-  constexpr int kMaxTiles = 1024, kMaxSlots = 2048;  // slots of 128 KB at head dim 128
-  BwdPlan pl;
-  const int group = a.h_q / a.h_kv, nseq = a.cu ? a.nseq : 1;
-  const int hp = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-  const int longest = a.cu ? std::min(a.max_seqlen, a.total) : a.total;
-  const int rows = a.d == 256 ? kBwdRows : kBwdRows * 2 * (4 / hp);
-  const int64_t row_tiles = (longest + rows - 1) / rows, key_tiles = (longest + kDkdvKeys - 1) / kDkdvKeys;
-  pl.dq_rows = rows;
-  pl.dq_tiles = nseq * row_tiles * (a.h_q / hp);
-  pl.kv_tiles = (int64_t)a.cp_size * a.h_kv * nseq * key_tiles;
-  if (longest <= 0) return pl;
-  const int L = nseq > 1 ? std::max(1, a.total / nseq) : longest;  // an average sequence when packed
-  const int late = a.cp_size - 1 - a.cp_rank;
-  auto blocks = [](int n) { return (n + kBwdRows - 1) / kBwdRows; };
-  if (pl.dq_tiles <= kMaxTiles) {
-    auto cost = [&](int len, int rt, bool back) {
-      return blocks(std::min((rt + 1) * rows, len)) + a.cp_rank * blocks(len / 2) + (back ? late * blocks(len) : 0);
-    };
-    const int rts = (L + rows - 1) / rows, fronts = late > 0 ? L / 2 / rows : 0;
-    ShareLoad w;
-    w.top = cost(longest, (int)row_tiles - 1, true);
-    w.avg = 0.5f * (cost(L, rts - 1, true) + cost(L, fronts, true));
-    w.n = (a.h_q / hp) * (rts - fronts) * nseq;
-    w.top2 = fronts ? cost(L, fronts - 1, false) : 0;
-    w.avg2 = fronts ? 0.5f * (w.top2 + cost(L, 0, false)) : 0.f;
-    w.n2 = (a.h_q / hp) * fronts * nseq;
-    w.us = a.d == 256 ? 1.7f : 1.2f * a.d / 128.f;
-    w.merge = 5.f;
-    w.read = 1.25f * a.d / 128.f;
-    w.packed = nseq > 1;
-    w.free2 = true;
-    pl.dq = best_shares(w, std::min<int64_t>(kMaxShares, kMaxSlots / pl.dq_tiles));
-  }
-  const bool wide = a.d == 256;
-  if (2 * pl.kv_tiles <= (wide ? 2 : 1) * kCus) {
-    // earlier sources: every row, the front half of the keys; own: half of the rows on average, the
-    // first half of the tiles three quarters; later sources: the back-half rows
-    const int kts = (L + kDkdvKeys - 1) / kDkdvKeys, own1 = (kts + 1) / 2;
-    const int early = a.cp_rank * ((L / 2 + kDkdvKeys - 1) / kDkdvKeys);
-    ShareLoad w;
-    w.top = blocks(longest) * group;
-    const float all = (float)(blocks(L) * group);
-    w.n = a.h_kv * nseq * (early + own1);
-    w.avg = all * (early + 0.75f * own1) / (early + own1);
-    w.top2 = (int)(0.5f * all);
-    w.n2 = a.h_kv * nseq * (late * kts + kts - own1);
-    w.avg2 = w.n2 ? all * (0.5f * late * kts + 0.25f * (kts - own1)) / (late * kts + kts - own1) : 0.f;
-    w.us = wide ? 1.75f : 1.02f * a.d / 128.f;
-    w.merge = wide ? 6.f : 5.f;
-    w.read = wide ? 0.f : 1.25f * a.d / 128.f;
-    w.slot = wide ? 0.08f : 0.f;  // 256 KB each
-    w.packed = nseq > 1;
-    w.free2 = true;
-    pl.kv = best_shares(w, std::min<int64_t>(kMaxShares, (wide ? 4 : 1) * kCus / pl.kv_tiles));
-  }
-  return pl;
-}
-// Their workspace: the counters (dq's tiles, then dk / dv's), then the slots of one kernel at a time.
+// Workspace of a plan's shared tiles: the counters (dq's tiles, then dk / dv's), then the slots of one kernel at a time.
 int64_t share_words(const BwdPlan& pl) { return (pl.dq.k > 1 || pl.kv.k > 1) ? pl.dq_tiles + pl.kv_tiles : 0; }
 int64_t share_count_bytes(const BwdPlan& pl) { return (share_words(pl) * 4 + 255) / 256 * 256; }
 int64_t share_bytes(const BwdPlan& pl, int d) {

@@ -42,6 +42,7 @@
 #include <cfloat>
 #include <type_traits>
 
+#include "attn_plan.h"
 #include "common.h"
 
 namespace fa4cp {
@@ -54,15 +55,6 @@ constexpr int kBN = 64;  // keys per tile
 // 32 x 256 fp32 output already takes 128 VGPRs and its Q fragments 64.
 template <int D>
 constexpr int vt_bn() { return D > 128 ? 32 : kBN; }
-
-// Workgroups per CU that the 16-bit pipeline's kernels are built for (their WGS).  At head dim 64 the
-// LDS tiles take 57 KB and the registers fit 128 without a spill, so two can run on a CU, one's loads,
-// softmax, start and end beside the other's MFMAs: 131072 tokens (H 32/8, cp 8, rank 3) 9180 -> 8460 us, 49152
-// (cp 4, rank 2) 2610 -> 2490, 24576 with 384 row tiles (cp 8, rank 5) 408 -> 383, 24 short sequences of 16
-// heads 57.6 -> 53.  With a CU for every workgroup that build is the slower one: two on one CU leave
-// another idle (256 row tiles, 8192 tokens, cp 4, rank 3: 105 -> 135 us), and kept apart they miss the
-// registers (110).
-inline bool two_per_cu(int d, int64_t workgroups) { return d == 64 && workgroups > 256; }
 
 struct AttnParams {
   const void* q;
@@ -773,7 +765,6 @@ __global__ __launch_bounds__(kThreads, (D >= 256 ? 1 : 2)) void attn_fwd_16bit(A
 // off the MFMA phases.  Each wavefront waits for its own LDS-DMA at the end of its next
 // phase, so data is published by that phase's barrier, at least one phase before use.
 //--------------------------------------------------------------------------------------
-constexpr int kPPWaves = 8;
 constexpr int kPPThreads = kPPWaves * 64;
 constexpr int kPPReadAhead = 4;  // LDS fragment reads issued ahead of the MFMA chain
 
@@ -2959,13 +2950,6 @@ __global__ __launch_bounds__(kPPThreads, 2) void attn_fwd_e4m3_sweep(SweepParams
   } else {
     e8_pipeline<D, HP, 2>(lds, geo, q, p.q_rs, qv, out, p.o_rs, lse, p.lse_rs, r0, L, k_rsb, vt_rsb, c_q);
   }
-}
-
-// Heads of one kv-head group that a workgroup takes (HP of the kernels).
-inline int heads_per_wg(int group) {
-  if (group % 4 == 0) return 4;
-  if (group % 2 == 0) return 2;
-  return 1;
 }
 
 }  // namespace

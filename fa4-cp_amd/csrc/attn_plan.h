@@ -1,0 +1,185 @@
+// Plans of the attention launches: which build of a kernel runs and how many workgroups share a
+// tile.  Host code without HIP, so that a plan can be looked at where there is no GPU.
+#pragma once
+
+#include <stdint.h>
+
+#include <algorithm>
+
+#include "../../include/fa4cp.h"
+#include "share_model.h"
+
+namespace fa4cp {
+
+// Heads of one kv-head group that a workgroup takes (HP of the kernels).
+inline int heads_per_wg(int group) {
+  if (group % 4 == 0) return 4;
+  if (group % 2 == 0) return 2;
+  return 1;
+}
+
+constexpr int kPPWaves = 8;  // wavefronts of a ping-pong kernel's workgroup, 32 (row, head) pairs each
+
+// Workgroups per CU that the 16-bit pipeline's kernels are built for (their WGS).  At head dim 64 the
+// LDS tiles take 57 KB and the registers fit 128 without a spill, so two can run on a CU, one's loads,
+// softmax, start and end beside the other's MFMAs: 131072 tokens (H 32/8, cp 8, rank 3) 9180 -> 8460 us, 49152
+// (cp 4, rank 2) 2610 -> 2490, 24576 with 384 row tiles (cp 8, rank 5) 408 -> 383, 24 short sequences of 16
+// heads 57.6 -> 53.  With a CU for every workgroup that build is the slower one: two on one CU leave
+// another idle (256 row tiles, 8192 tokens, cp 4, rank 3: 105 -> 135 us), and kept apart they miss the
+// registers (110).
+inline bool two_per_cu(int d, int64_t workgroups) { return d == 64 && workgroups > 256; }
+
+// How a sweep is split (see SweepSplit in attn_split.hip).
+struct SplitPlan {
+  Shares shares;
+  int ns_back = 1, ns_front = 1, n_front = 0, n_row = 0, per_hg = 0;
+  bool split() const { return shares.k > 1; }
+};
+
+// The plan for a sweep's shape (no pointer of `a` is followed).
+// The number of shares comes from best_shares' estimate: the row tiles that meet the later sources
+// (about `avg` key tiles each) before the others, 1.65 us a key tile (1 us at head dim 64), a merge
+// of 5 us plus 1.25 us per share and 128 columns.  It orders the measured times of 15 shapes
+// (one and four rings, D 64 / 128 / 256, 16 to 512 row tiles; GPU time, us):
+//   shares                                1     2     3     4     6     8
+//   2048 tokens, H 8/2, cp 4, rank 1     52    42    39    38    38    40   (chosen: 5)
+//   8192, H 32/8, cp 8, rank 3          144    96    88   107   103   116   (3)
+//   16384, rank 3                       298   282   270   298   298   313   (3)
+//   16384, rank 7 (equal row tiles)     264   267   277   291   319   344   (1)
+//   24576, rank 3                       555   573   560   623   594   626   (1)
+//   8192, e4m3, rank 3                  113    80    69    85    84   100   (3)
+//   16384, H 16/2, D 256, rank 3        476   301   278   353   335   400   (3)
+inline SplitPlan split_plan(const fa4cp_sweep_args* a) {
+  constexpr int kMaxRowTiles = 1024, kMaxSlots = 2048;  // slots of 128 KB at head dim 128
+  SplitPlan pl;
+  const bool fp8 = a->dtype == FA4CP_E4M3;
+  const int bn = fp8 ? (a->d == 256 ? 64 : 128) : (a->d == 256 ? 32 : 64);
+  const int hp = heads_per_wg(a->h_q / a->h_kv), rows = 32 * kPPWaves / hp;
+  const int n_hg = a->h_q / hp;
+  const int nseq = a->cu ? a->nseq : 1;
+  const int longest = a->cu ? std::min(a->max_seqlen, a->total) : a->total;
+  if (longest <= 0) return pl;
+  const int64_t n_rt = (longest + rows - 1) / rows;
+  // packed: at most one row tile per sequence beyond total / rows
+  const int64_t n_row = nseq > 1 ? std::min(nseq * n_rt, (int64_t)a->total / rows + nseq) : n_rt;
+  if (n_hg * n_row > kMaxRowTiles) return pl;
+  auto tiles = [&](int keys) { return (keys + bn - 1) / bn; };
+  const int late_steps = a->cp_size - 1 - a->cp_rank;
+  // key tiles of row tile rt of a sequence of L rows
+  auto cost = [&](int L, int rt, bool back) {
+    return (std::min((rt + 1) * rows, L) - 1) / bn + 1 + a->cp_rank * tiles(L / 2) + (back ? late_steps * tiles(L) : 0);
+  };
+  // the classes of row tiles, of a sequence of average length when packed
+  const int L = nseq > 1 ? std::max(1, a->total / nseq) : longest;
+  const int rts = (L + rows - 1) / rows;
+  const int fronts = late_steps > 0 ? (L / 2) / rows : 0;
+  const int top = cost(longest, (int)n_rt - 1, true);
+  if (top > 1 << 20) return pl;
+  const int front_top = fronts ? cost(L, fronts - 1, false) : 0;
+  ShareLoad w;
+  w.top = top;
+  w.avg = 0.5f * (cost(L, rts - 1, true) + cost(L, fronts, true));
+  w.n = n_hg * (rts - fronts) * nseq;
+  w.top2 = front_top;
+  w.avg2 = fronts ? 0.5f * (front_top + cost(L, 0, false)) : 0.f;
+  w.n2 = n_hg * fronts * nseq;
+  w.us = a->d == 64 ? 1.f : 1.65f;
+  w.merge = 5.f;
+  w.read = 1.25f * a->d / 128.f;
+  w.packed = nseq > 1;
+  w.free2 = false;
+  pl.shares = best_shares(w, std::min(kMaxShares, kMaxSlots / (int)(n_hg * n_row)));
+  if (pl.shares.k == 1) return pl;
+  pl.n_row = (int)n_row;
+  pl.ns_back = pl.shares.k;
+  if (nseq == 1 && fronts > 0) {
+    pl.n_front = fronts;
+    pl.ns_front = pl.shares.k2;
+  }
+  pl.per_hg = ((pl.n_row - pl.n_front) * pl.ns_back + pl.n_front * pl.ns_front + 7) / 8 * 8;
+  return pl;
+}
+
+constexpr int kBwdRows = 32;  // query rows (dq) or keys (dk/dv) per wavefront
+constexpr int kDkdvKeys = 4 * kBwdRows;  // keys per dk/dv workgroup
+
+// Tiles of the two gradient kernels and the workgroups that share one.
+struct BwdPlan {
+  int64_t dq_tiles = 0, kv_tiles = 0;
+  int dq_rows = 0;  // rows of a dq tile
+  Shares dq, kv;
+};
+
+// A 32-key block of dq takes 1.2 us and a 32-row block of dk / dv 1.02 (measured, head dim 128, the
+// chip full; dq at 256, half the rows, 1.7).  dq's row tiles are shared wherever best_shares finds it faster (backward, GPU time in
+// us, shares of the back-half / other row tiles: 8192 tokens, H 32/8, cp 4, rank 1: none 622, 2/1 584,
+// 2/2 564 (chosen), 3/2 589; 16384, cp 8, rank 3: 1098, 1046, 1000 (chosen), 1054; rank 7, equal row
+// tiles: 985 (chosen), 1071, 992, 1050).  dk / dv's key tiles only where all shares run at once: the
+// workgroups stream the query blocks in step, and shares at other blocks cost more in L2
+// misses than the even split gains (8192 tokens: none 622, two shares 628-651, three 634-650; 24576
+// tokens, H 16/2: 1311, 1337-1389), but 32 key tiles leave the chip idle (2048 tokens, H 8/2: 138,
+// 120, 113; four 112).  At head dim 256 a block takes the MFMAs twice as long and the even split wins up to
+// 256 tiles, of up to four times as many shares as CUs (backward: 16384 tokens, H 16/2, cp 8, rank 3, 256 tiles
+// 1333 and 1165; 8192, cp 4, 128 tiles: two shares 727, up to eight 610; four sequences, H 8/2, 273 and 205),
+// not beyond (32768 tokens, cp 4, 512 tiles 8450 and 8559).  There a share costs 0.08 us for its 256 KB (without
+// that, 3072 tokens, H 24/8, cp 8, rank 6, short tiles: unshared 266, shared 281).
+inline BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
+  constexpr int kMaxTiles = 1024, kMaxSlots = 2048;  // slots of 128 KB at head dim 128
+  BwdPlan pl;
+  const int group = a.h_q / a.h_kv, nseq = a.cu ? a.nseq : 1;
+  const int hp = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+  const int longest = a.cu ? std::min(a.max_seqlen, a.total) : a.total;
+  const int rows = a.d == 256 ? kBwdRows : kBwdRows * 2 * (4 / hp);
+  const int64_t row_tiles = (longest + rows - 1) / rows, key_tiles = (longest + kDkdvKeys - 1) / kDkdvKeys;
+  pl.dq_rows = rows;
+  pl.dq_tiles = nseq * row_tiles * (a.h_q / hp);
+  pl.kv_tiles = (int64_t)a.cp_size * a.h_kv * nseq * key_tiles;
+  if (longest <= 0) return pl;
+  const int L = nseq > 1 ? std::max(1, a.total / nseq) : longest;  // an average sequence when packed
+  const int late = a.cp_size - 1 - a.cp_rank;
+  auto blocks = [](int n) { return (n + kBwdRows - 1) / kBwdRows; };
+  if (pl.dq_tiles <= kMaxTiles) {
+    auto cost = [&](int len, int rt, bool back) {
+      return blocks(std::min((rt + 1) * rows, len)) + a.cp_rank * blocks(len / 2) + (back ? late * blocks(len) : 0);
+    };
+    const int rts = (L + rows - 1) / rows, fronts = late > 0 ? L / 2 / rows : 0;
+    ShareLoad w;
+    w.top = cost(longest, (int)row_tiles - 1, true);
+    w.avg = 0.5f * (cost(L, rts - 1, true) + cost(L, fronts, true));
+    w.n = (a.h_q / hp) * (rts - fronts) * nseq;
+    w.top2 = fronts ? cost(L, fronts - 1, false) : 0;
+    w.avg2 = fronts ? 0.5f * (w.top2 + cost(L, 0, false)) : 0.f;
+    w.n2 = (a.h_q / hp) * fronts * nseq;
+    w.us = a.d == 256 ? 1.7f : 1.2f * a.d / 128.f;
+    w.merge = 5.f;
+    w.read = 1.25f * a.d / 128.f;
+    w.packed = nseq > 1;
+    w.free2 = true;
+    pl.dq = best_shares(w, std::min<int64_t>(kMaxShares, kMaxSlots / pl.dq_tiles));
+  }
+  const bool wide = a.d == 256;
+  if (2 * pl.kv_tiles <= (wide ? 2 : 1) * kCus) {
+    // earlier sources: every row, the front half of the keys; own: half of the rows on average, the
+    // first half of the tiles three quarters; later sources: the back-half rows
+    const int kts = (L + kDkdvKeys - 1) / kDkdvKeys, own1 = (kts + 1) / 2;
+    const int early = a.cp_rank * ((L / 2 + kDkdvKeys - 1) / kDkdvKeys);
+    ShareLoad w;
+    w.top = blocks(longest) * group;
+    const float all = (float)(blocks(L) * group);
+    w.n = a.h_kv * nseq * (early + own1);
+    w.avg = all * (early + 0.75f * own1) / (early + own1);
+    w.top2 = (int)(0.5f * all);
+    w.n2 = a.h_kv * nseq * (late * kts + kts - own1);
+    w.avg2 = w.n2 ? all * (0.5f * late * kts + 0.25f * (kts - own1)) / (late * kts + kts - own1) : 0.f;
+    w.us = wide ? 1.75f : 1.02f * a.d / 128.f;
+    w.merge = wide ? 6.f : 5.f;
+    w.read = wide ? 0.f : 1.25f * a.d / 128.f;
+    w.slot = wide ? 0.08f : 0.f;  // 256 KB each
+    w.packed = nseq > 1;
+    w.free2 = true;
+    pl.kv = best_shares(w, std::min<int64_t>(kMaxShares, (wide ? 4 : 1) * kCus / pl.kv_tiles));
+  }
+  return pl;
+}
+
+}  // namespace fa4cp

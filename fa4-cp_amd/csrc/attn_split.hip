@@ -9,11 +9,8 @@
 // slots.  Shares are cut at tile
 // granularity from the flattened segment list, alike for contiguous and paged K, so the two
 // stay bit-identical.
-#include <algorithm>
-
 #include "attn_kernels.h"
 #include "attn_split.h"
-#include "share_model.h"
 
 namespace fa4cp {
 namespace {
@@ -269,69 +266,6 @@ int64_t split_rows(const SplitPlan& pl, int n_hg) { return (int64_t)n_hg * pl.pe
 int64_t done_bytes(int64_t words) { return (words * 4 + 255) / 256 * 256; }
 
 }  // namespace
-
-// The number of shares comes from best_shares' estimate: the row tiles that meet the later sources
-// (about `avg` key tiles each) before the others, 1.65 us a key tile (1 us at head dim 64), a merge
-// of 5 us plus 1.25 us per share and 128 columns.  It orders the measured times of 15 shapes
-// (one and four rings, D 64 / 128 / 256, 16 to 512 row tiles; GPU time, us):
-//   shares                                1     2     3     4     6     8
-//   2048 tokens, H 8/2, cp 4, rank 1     52    42    39    38    38    40   (chosen: 5)
-//   8192, H 32/8, cp 8, rank 3          144    96    88   107   103   116   (3)
-//   16384, rank 3                       298   282   270   298   298   313   (3)
-//   16384, rank 7 (equal row tiles)     264   267   277   291   319   344   (1)
-//   24576, rank 3                       555   573   560   623   594   626   (1)
-//   8192, e4m3, rank 3                  113    80    69    85    84   100   (3)
-//   16384, H 16/2, D 256, rank 3        476   301   278   353   335   400   (3)
-SplitPlan split_plan(const fa4cp_sweep_args* a) {
-  constexpr int kMaxRowTiles = 1024, kMaxSlots = 2048;  // slots of 128 KB at head dim 128
-  SplitPlan pl;
-  const bool fp8 = a->dtype == FA4CP_E4M3;
-  const int bn = fp8 ? (a->d == 256 ? 64 : 128) : (a->d == 256 ? 32 : 64);
-  const int hp = heads_per_wg(a->h_q / a->h_kv), rows = 32 * kPPWaves / hp;
-  const int n_hg = a->h_q / hp;
-  const int nseq = a->cu ? a->nseq : 1;
-  const int longest = a->cu ? std::min(a->max_seqlen, a->total) : a->total;
-  if (longest <= 0) return pl;
-  const int64_t n_rt = (longest + rows - 1) / rows;
-  // packed: at most one row tile per sequence beyond total / rows
-  const int64_t n_row = nseq > 1 ? std::min(nseq * n_rt, (int64_t)a->total / rows + nseq) : n_rt;
-  if (n_hg * n_row > kMaxRowTiles) return pl;
-  auto tiles = [&](int keys) { return (keys + bn - 1) / bn; };
-  const int late_steps = a->cp_size - 1 - a->cp_rank;
-  // key tiles of row tile rt of a sequence of L rows
-  auto cost = [&](int L, int rt, bool back) {
-    return (std::min((rt + 1) * rows, L) - 1) / bn + 1 + a->cp_rank * tiles(L / 2) + (back ? late_steps * tiles(L) : 0);
-  };
-  // the classes of row tiles, of a sequence of average length when packed
-  const int L = nseq > 1 ? std::max(1, a->total / nseq) : longest;
-  const int rts = (L + rows - 1) / rows;
-  const int fronts = late_steps > 0 ? (L / 2) / rows : 0;
-  const int top = cost(longest, (int)n_rt - 1, true);
-  if (top > 1 << 20) return pl;
-  const int front_top = fronts ? cost(L, fronts - 1, false) : 0;
-  ShareLoad w;
-  w.top = top;
-  w.avg = 0.5f * (cost(L, rts - 1, true) + cost(L, fronts, true));
-  w.n = n_hg * (rts - fronts) * nseq;
-  w.top2 = front_top;
-  w.avg2 = fronts ? 0.5f * (front_top + cost(L, 0, false)) : 0.f;
-  w.n2 = n_hg * fronts * nseq;
-  w.us = a->d == 64 ? 1.f : 1.65f;
-  w.merge = 5.f;
-  w.read = 1.25f * a->d / 128.f;
-  w.packed = nseq > 1;
-  w.free2 = false;
-  pl.shares = best_shares(w, std::min(kMaxShares, kMaxSlots / (int)(n_hg * n_row)));
-  if (pl.shares.k == 1) return pl;
-  pl.n_row = (int)n_row;
-  pl.ns_back = pl.shares.k;
-  if (nseq == 1 && fronts > 0) {
-    pl.n_front = fronts;
-    pl.ns_front = pl.shares.k2;
-  }
-  pl.per_hg = ((pl.n_row - pl.n_front) * pl.ns_back + pl.n_front * pl.ns_front + 7) / 8 * 8;
-  return pl;
-}
 
 int64_t split_words(const SplitPlan& pl, int n_hg) { return (int64_t)n_hg * pl.n_row; }
 int64_t split_bytes(const SplitPlan& pl, int n_hg, int d) {

@@ -11,24 +11,27 @@ import ctypes
 import pytest
 import torch
 
+import plans
 from fa4_ring import LocalKVRing, RingConfig, _lib, ring_flash_attn, ring_flash_attn_backward, ring_flash_attn_func
 from fa4_ring.backward import _backward
 from gpu_helpers import DEV, say
 
 pytestmark = pytest.mark.gpu
 
-CASES = [  # (local lens, H, H_kv, D, cp, rank, dtype, shared)
-    ([512], 8, 2, 128, 4, 1, torch.bfloat16, True),    # dq and dk / dv shared
-    ([386], 4, 4, 64, 8, 2, torch.float16, True),      # one query head per kv head, partial blocks
-    ([1024], 8, 2, 128, 2, 0, torch.bfloat16, True),   # no earlier source
-    ([640], 16, 2, 128, 8, 7, torch.float16, True),    # no later source
-    ([1024, 66, 0, 514], 4, 1, 128, 8, 3, torch.bfloat16, True),  # packed
-    ([2048], 16, 4, 64, 4, 1, torch.bfloat16, True),   # dq alone
-    ([512], 8, 2, 256, 4, 1, torch.bfloat16, True),    # head dim 256: dk / dv, summed by a kernel of its own
-    ([386], 8, 1, 256, 8, 5, torch.float16, True),     # a partial key tile, tiles no row attends
-    ([300, 0, 70, 2], 4, 1, 256, 4, 3, torch.bfloat16, True),  # packed
-    ([2048], 16, 16, 256, 2, 0, torch.bfloat16, False),  # more tiles than are shared
-    ([2], 4, 2, 128, 4, 2, torch.bfloat16, False),
+CASES = [  # (local lens, H, H_kv, D, cp, rank, dtype, what is shared: dq's and dk / dv's tiles)
+    ([512], 8, 2, 128, 4, 1, torch.bfloat16, "dq kv"),
+    ([386], 4, 4, 64, 8, 2, torch.float16, "dq"),         # one query head per kv head, partial blocks
+    ([1024], 8, 2, 128, 2, 0, torch.bfloat16, "dq kv"),   # no earlier source
+    ([640], 16, 2, 128, 8, 7, torch.float16, "dq kv"),    # no later source
+    ([1024, 66, 0, 514], 4, 1, 128, 8, 3, torch.bfloat16, "dq"),  # packed
+    ([2048], 16, 4, 64, 4, 1, torch.bfloat16, "dq"),
+    ([512], 8, 2, 256, 4, 1, torch.bfloat16, "dq kv"),    # head dim 256: the shares summed by kernels of their own
+    ([386], 8, 1, 256, 8, 5, torch.float16, "dq kv"),     # a partial key tile, tiles no row attends
+    ([300, 0, 70, 2], 4, 1, 256, 4, 3, torch.bfloat16, "dq kv"),  # packed
+    ([256], 8, 1, 256, 4, 0, torch.bfloat16, "dq kv"),    # the shorter row tiles whole beside shared ones
+    ([4096], 16, 2, 256, 4, 1, torch.bfloat16, "kv"),
+    ([2048], 16, 16, 256, 2, 0, torch.bfloat16, ""),      # more tiles than are shared
+    ([2], 4, 2, 128, 4, 2, torch.bfloat16, ""),
 ]
 
 
@@ -46,13 +49,9 @@ def test_shared_backward(lens, h, h_kv, d, cp, rank, dtype, shared, monkeypatch)
     lk, lv = ring.kv(rank)
     out, lse = ring_flash_attn(q, lk, lv, cfg, group=ring, return_lse=True, **kw)
 
-    a = _lib.SweepBwdArgs()
-    a.total, a.h_q, a.h_kv, a.d, a.cp_rank, a.cp_size = total, h, h_kv, d, rank, cp
-    if packed:
-        a.cu, a.nseq, a.max_seqlen = cu.data_ptr(), len(lens), max(lens)
     lib = _lib.load()
-    need = lib.fa4cp_ring_sweep_bwd_share_bytes(ctypes.byref(a))
-    assert (need > 0) == shared
+    need = lib.fa4cp_ring_sweep_bwd_share_bytes(ctypes.byref(plans.backward_args(lens, h, h_kv, d, cp, rank)))
+    assert (need > 0) == bool(shared)
 
     def grads(dt=torch.float32):
         r = _backward(dout, q, lk, lv, out, lse, cfg, ring, cu, kw["max_seqlen"], None, None, None, False, dt)
