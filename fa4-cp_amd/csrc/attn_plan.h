@@ -49,6 +49,16 @@ struct SplitPlan {
 //   24576, rank 3                       555   573   560   623   594   626   (1)
 //   8192, e4m3, rank 3                  113    80    69    85    84   100   (3)
 //   16384, H 16/2, D 256, rank 3        476   301   278   353   335   400   (3)
+// At head dim 256 a share costs more: the merging workgroup takes 8 us for each (its 256 KB come one load
+// at a time: beside the 128 registers of the output there is room for no more), and the launch 0.1 us for
+// each (256 KB written and read at the copy rate).  At 2.5 us and nothing, shapes were split that are
+// faster whole or in fewer shares (us unsplit, in the shares chosen then, and now):
+//   1024 tokens, H 8/2, fp16, cp 2, rank 1        52   72 (4)   52 (1)
+//   8000, H 32/8, bf16, cp 4, rank 3             261  292 (2)  261 (1)
+//   8772, H 32/8, e4m3, cp 2, rank 1             340  449 (2)  340 (1)
+//   1456, H 16/2, fp16, cp 8, rank 3              69   82 (5)   70 (3)
+//   2368, H 8/2, bf16, cp 8, rank 5               85   98 (7)   77 (3)
+//   nine sequences, 7888, H 16/2, cp 8, rank 6    84  108 (6)   77 (2)
 inline SplitPlan split_plan(const fa4cp_sweep_args* a) {
   constexpr int kMaxRowTiles = 1024, kMaxSlots = 2048;  // slots of 128 KB at head dim 128
   SplitPlan pl;
@@ -84,8 +94,10 @@ inline SplitPlan split_plan(const fa4cp_sweep_args* a) {
   w.avg2 = fronts ? 0.5f * (front_top + cost(L, 0, false)) : 0.f;
   w.n2 = n_hg * fronts * nseq;
   w.us = a->d == 64 ? 1.f : 1.65f;
+  const bool wide = a->d == 256;
   w.merge = 5.f;
-  w.read = 1.25f * a->d / 128.f;
+  w.read = wide ? 8.f : 1.25f * a->d / 128.f;
+  w.slot = wide ? 0.1f : 0.f;
   w.packed = nseq > 1;
   w.free2 = false;
   pl.shares = best_shares(w, std::min(kMaxShares, kMaxSlots / (int)(n_hg * n_row)));

@@ -1,6 +1,7 @@
 """How the attention launches are laid out (csrc/attn_plan.h), without a GPU."""
 
 import pytest
+import torch
 
 import plans
 from test_gpu_split_backward import CASES as BACKWARD
@@ -20,3 +21,23 @@ def test_backward_cases_reach_every_form():
         for shares in (dq, kv):
             assert any(s.k > 1 and s.k2 > 1 for s in shares), (wide, shares)
         assert any(s.k > 1 and s.top2 and s.k2 == 1 for s in dq + kv), (wide, dq, kv)
+
+
+BF16, FP16, E4M3 = torch.bfloat16, torch.float16, torch.float8_e4m3fn
+NINE = [260, 216, 144, 112, 96, 64, 46, 32, 16]
+
+
+@pytest.mark.parametrize("lens,h,h_kv,cp,rank,dtype,least,most", [
+    # (the times beside split_plan: within 2 % of the fastest share count are least..most)
+    ([512], 8, 2, 2, 1, FP16, 1, 1),
+    ([2000], 32, 8, 4, 3, BF16, 1, 1),
+    ([4386], 32, 8, 2, 1, E4M3, 1, 1),
+    ([290], 8, 2, 8, 7, E4M3, 1, 1),
+    ([182], 16, 2, 8, 3, FP16, 1, 3),
+    ([296], 8, 2, 8, 5, BF16, 2, 3),
+    ([2048], 16, 2, 8, 3, BF16, 3, 3),   # still shared where that is 1.7 times as fast
+    (NINE, 16, 2, 8, 6, BF16, 1, 3),
+])
+def test_wide_sweeps_are_not_split_at_a_loss(lens, h, h_kv, cp, rank, dtype, least, most):
+    """Head dim 256: the merge and the slots' traffic are charged."""
+    assert least <= plans.split_plan(lens, h, h_kv, 256, cp, rank, dtype).back <= most
