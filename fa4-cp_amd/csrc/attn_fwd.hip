@@ -242,7 +242,7 @@ extern "C" int fa4cp_attn_fwd(const fa4cp_attn_args* a, void* stream) {
     p.claim = claim_slot((hipStream_t)stream);
     if (p.claim != nullptr) grid = (unsigned)(blocks + 8 * spare);
   }
-  if (use_vt && two_per_cu(d, blocks)) kc.fn = a->dtype == FA4CP_BF16 ? pick_two<__bf16>(hp) : pick_two<_Float16>(hp);
+  if (use_vt && attn_two_per_cu(a)) kc.fn = a->dtype == FA4CP_BF16 ? pick_two<__bf16>(hp) : pick_two<_Float16>(hp);
   hipLaunchKernelGGL(kc.fn, dim3(grid), dim3(kc.threads), 0, (hipStream_t)stream, p);
   return check_launch("attn_fwd");
 }
@@ -347,8 +347,7 @@ static int ring_sweep_launch(const fa4cp_sweep_args* a, const fa4cp_sweep_kpages
   }
   void (*fn)(SweepParams) = nullptr;
   const bool pack = nseq > 1;  // several sequences: the gap-free row tile order
-  // (packed: about half a row tile per sequence more than total / rows)
-  const bool two = two_per_cu(d, pack ? (int64_t)p.n_hg * (a->total / rows + nseq / 2) : blocks);
+  const bool two = sweep_two_per_cu(a);
 #define FA4CP_PICK_PK(KERNEL, H, ...)                                                       \
   {                                                                                         \
     if (paged) fn = pack ? KERNEL<__VA_ARGS__, H, true, true> : KERNEL<__VA_ARGS__, H, true, false>; \

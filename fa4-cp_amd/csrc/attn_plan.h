@@ -29,6 +29,37 @@ constexpr int kPPWaves = 8;  // wavefronts of a ping-pong kernel's workgroup, 32
 // registers (110).
 inline bool two_per_cu(int d, int64_t workgroups) { return d == 64 && workgroups > 256; }
 
+// Row tiles of `rows` rows, at most n_rt in a sequence, that nseq sequences of `total` rows in all make.
+// Only the device knows the lengths of packed ones: about half a tile per sequence more than
+// total / rows.  (A grid of n_rt tiles for each of nine sequences of 1024 rows in all, the longest 350, H
+// 32/8, has 432 workgroups, 160 of them with rows.)
+inline int64_t working_row_tiles(int64_t total, int rows, int nseq, int64_t n_rt) {
+  return nseq > 1 ? std::min(nseq * n_rt, total / rows + nseq / 2) : n_rt;
+}
+
+// The build of the unsplit sweep, whose workgroups without rows come last.
+inline bool sweep_two_per_cu(const fa4cp_sweep_args* a) {
+  const int hp = heads_per_wg(a->h_q / a->h_kv), rows = 32 * kPPWaves / hp;
+  const int n_rt = ((a->cu ? a->max_seqlen : a->total) + rows - 1) / rows;
+  return two_per_cu(a->d, a->h_q / hp * working_row_tiles(a->total, rows, a->cu ? a->nseq : 1, n_rt));
+}
+
+// The build of the V^T kernel for one attention call.  Its workgroups without rows stand among the others
+// and hold up their start: where all row tiles are short, that counts for more than a CU for each
+// with rows.  Attention of two steps, the grid above 256 workgroups, those with rows below: with five row tiles or more in
+// the longest sequence, or over 512 rows, the one-per-CU build takes 0.95 of the other's time in the mean of 42
+// shapes (0.81-1.09; the nine sequences above 47.4 -> 43.1 us, 7596 rows in three, H 8/1, 147 -> 130), below that
+// 1.07 in the mean of 18 (nine of 784 rows, H 32/8, 38 and 44 us).
+inline bool attn_two_per_cu(const fa4cp_attn_args* a) {
+  const int hp = heads_per_wg(a->h_q / a->h_kv), rows = 32 * kPPWaves / hp, nseq = a->cu_q ? a->nseq : 1;
+  const bool all = a->q_sel == FA4CP_SEL_ALL;
+  auto selected = [&](int n) { return all ? n : (n + 1) / 2; };
+  const int longest = selected(a->cu_q ? a->max_seqlen_q : a->total_q);
+  const int64_t n_rt = (longest + rows - 1) / rows;
+  const bool by_rows = n_rt >= 5 || longest > 512;
+  return two_per_cu(a->d, a->h_q / hp * (by_rows ? working_row_tiles(selected(a->total_q), rows, nseq, n_rt) : nseq * n_rt));
+}
+
 // How a sweep is split (see SweepSplit in attn_split.hip).
 struct SplitPlan {
   Shares shares;

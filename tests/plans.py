@@ -8,6 +8,8 @@ import subprocess
 import tempfile
 from collections import namedtuple
 
+import torch
+
 from fa4_ring import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -20,6 +22,8 @@ extern "C" void split(const fa4cp_sweep_args* a, int* o) {
   const SplitPlan pl = split_plan(a);
   o[0] = pl.ns_back; o[1] = pl.ns_front; o[2] = pl.shares.chunk; o[3] = pl.n_front; o[4] = pl.n_row;
 }
+extern "C" int sweep_two(const fa4cp_sweep_args* a) { return sweep_two_per_cu(a); }
+extern "C" int attn_two(const fa4cp_attn_args* a) { return attn_two_per_cu(a); }
 extern "C" void backward(const fa4cp_sweep_bwd_args* a, int* o) {
   const BwdPlan pl = bwd_plan(*a);
   put(pl.dq, o);
@@ -58,6 +62,22 @@ def split_plan(lens, h, h_kv, d, cp, rank, dtype):
     out = (ctypes.c_int * 5)()
     _probe().split(ctypes.byref(sweep_args(lens, h, h_kv, d, cp, rank, dtype)), out)
     return Split(*out)
+
+
+def heads_per_wg(group):
+    return 4 if group % 4 == 0 else 2 if group % 2 == 0 else 1
+
+
+def sweep_two_per_cu(lens, h, h_kv, d):
+    return bool(_probe().sweep_two(ctypes.byref(sweep_args(lens, h, h_kv, d, 4, 1, torch.bfloat16))))
+
+
+def attn_two_per_cu(lens, h, h_kv, d, q_sel=0):
+    a = _lib.AttnArgs()
+    a.total_q, a.h_q, a.h_kv, a.d, a.nseq, a.q_sel = sum(lens), h, h_kv, d, 1, q_sel
+    if len(lens) > 1:
+        a.cu_q, a.nseq, a.max_seqlen_q = 1 << 20, len(lens), max(lens)
+    return bool(_probe().attn_two(ctypes.byref(a)))
 
 
 def backward_args(lens, h, h_kv, d, cp, rank):

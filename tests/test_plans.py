@@ -41,3 +41,40 @@ NINE = [260, 216, 144, 112, 96, 64, 46, 32, 16]
 def test_wide_sweeps_are_not_split_at_a_loss(lens, h, h_kv, cp, rank, dtype, least, most):
     """Head dim 256: the merge and the slots' traffic are charged."""
     assert least <= plans.split_plan(lens, h, h_kv, 256, cp, rank, dtype).back <= most
+
+
+@pytest.mark.parametrize("lens,h,h_kv", [
+    ([350, 150, 124, 100, 100, 80, 60, 40, 20], 32, 8),  # 432 workgroups with the longest one's tiles for each
+    ([2048] + [64] * 31, 8, 2),
+    ([256] * 8, 32, 8),                                  # whole tiles: 256 workgroups, none to spare
+    ([322] * 8, 32, 8),
+    ([1024] * 8, 32, 8),
+    ([2050], 32, 8),
+    ([2048], 32, 8),
+    ([1300] * 12, 16, 16),
+    ([600] * 9, 6, 3),
+])
+@pytest.mark.parametrize("q_sel", [0, 1])
+def test_two_per_cu_counts_the_workgroups_with_rows(lens, h, h_kv, q_sel):
+    """Two workgroups per CU (head dim 64) only where more than 256 have rows; half a tile per sequence
+    off at most, as the host doesn't know the lengths."""
+    hp = plans.heads_per_wg(h // h_kv)
+
+    def workgroups(ns):
+        return h // hp * sum(-(-n * hp // 256) for n in ns)
+
+    slack = h // hp * len(lens) // 2 if len(lens) > 1 else 0
+    for two, ns in ((plans.attn_two_per_cu(lens, h, h_kv, 64, q_sel), [n if q_sel == 0 else n // 2 for n in lens]),
+                    (plans.sweep_two_per_cu(lens, h, h_kv, 64), lens)):
+        n = workgroups(ns)
+        assert two == (n > 256) or abs(n - 256) <= slack, (two, n)
+    assert not plans.attn_two_per_cu(lens, h, h_kv, 128, q_sel)
+
+
+def test_two_per_cu_of_packed_sequences():
+    nine = [350, 150, 124, 100, 100, 80, 60, 40, 20]
+    assert not plans.attn_two_per_cu(nine, 32, 8, 64) and not plans.sweep_two_per_cu(nine, 32, 8, 64)
+    assert not plans.attn_two_per_cu([256] * 8, 32, 8, 64) and not plans.sweep_two_per_cu([256] * 8, 32, 8, 64)
+    assert plans.attn_two_per_cu([322] * 8, 32, 8, 64)
+    # short row tiles: by the grid, empty workgroups and all
+    assert plans.attn_two_per_cu([222] + [70] * 8, 32, 8, 64) and not plans.sweep_two_per_cu([222] + [70] * 8, 32, 8, 64)
