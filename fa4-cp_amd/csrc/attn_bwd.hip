@@ -130,8 +130,7 @@ constexpr int kAgent = 16;
 // The share of a tile's n blocks that workgroup i of the launch's ns takes: [lo, hi), of `shares`;
 // false: the tile has fewer shares.
 __device__ __forceinline__ bool take_share(const BwdParams& p, int i, int n, int& lo, int& hi, int& shares) {
-  const int chunk = n > p.top2 ? p.chunk : p.chunk2;
-  shares = max(1, min(p.ns, (n + chunk - 1) / chunk));
+  shares = shares_of(p.ns, p.chunk, p.top2, p.chunk2, n);
   lo = n * i / shares;
   hi = n * (i + 1) / shares;
   return i < shares;
@@ -1053,8 +1052,8 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
       }
       const float c = p.scale * kLog2e;
       // query rows that can see a key of this workgroup: from the first key on when causal
-      const int row_begin = max(sp.row_min, sp.causal ? kb0 : 0) / kBwdRows * kBwdRows;
-      const int n_rb = (L - row_begin + kBwdRows - 1) / kBwdRows;
+      const int row_begin = first_block_row(max(sp.row_min, sp.causal ? kb0 : 0));
+      const int n_rb = row_blocks(L, row_begin);
       // (query head, 32-row block) pairs, head-major: this workgroup's share of them, from `lo` on
       int lo, hi;
       if (kShares) {
@@ -1370,8 +1369,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_sum_kernel(BwdParams p) {
   const int kb0 = kt * kDkdvKeys, key0 = (int)(blockIdx.x & 7) * kKeys;
   const StepPairs sp = step_pairs(p.rank, p.S, src, L);
   if (kb0 + key0 >= L || kb0 >= sp.key_lim) return;
-  const int row_begin = max(sp.row_min, sp.causal ? kb0 : 0) / kBwdRows * kBwdRows;
-  take_share(p, 0, (L - row_begin + kBwdRows - 1) / kBwdRows * p.group, lo, hi, shares);
+  take_share(p, 0, row_blocks(L, max(sp.row_min, sp.causal ? kb0 : 0)) * p.group, lo, hi, shares);
   if (shares == 1) return;  // (its workgroup wrote the gradient)
   const int keys = min(kKeys, L - kb0 - key0);
   for (int i = threadIdx.x; i < 2 * keys * kRow; i += 256) {

@@ -146,6 +146,11 @@ inline SplitPlan split_plan(const fa4cp_sweep_args* a) {
 constexpr int kBwdRows = 32;  // query rows (dq) or keys (dk/dv) per wavefront
 constexpr int kDkdvKeys = 4 * kBwdRows;  // keys per dk/dv workgroup
 
+// The 32-row blocks that hold rows [row, L) of a sequence of L: the first one's first row, and how many.
+// A key tile walks them, with row the first of its keys' causal rows, or the back half's first.
+constexpr int first_block_row(int row) { return row / kBwdRows * kBwdRows; }
+constexpr int row_blocks(int L, int row) { return (L - first_block_row(row) + kBwdRows - 1) / kBwdRows; }
+
 // Tiles of the two gradient kernels and the workgroups that share one.
 struct BwdPlan {
   int64_t dq_tiles = 0, kv_tiles = 0;
@@ -202,18 +207,27 @@ inline BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
   }
   const bool wide = a.d == 256;
   if (2 * pl.kv_tiles <= (wide ? 2 : 1) * kCus) {
-    // earlier sources: every row, the front half of the keys; own: half of the rows on average, the
-    // first half of the tiles three quarters; later sources: the back-half rows
-    const int kts = (L + kDkdvKeys - 1) / kDkdvKeys, own1 = (kts + 1) / 2;
-    const int early = a.cp_rank * ((L / 2 + kDkdvKeys - 1) / kDkdvKeys);
+    // earlier sources: every row, the front half of the keys; own: half of the rows on average; later
+    // sources: the back-half rows.  The own tiles of more blocks than a later source's are of the first
+    // class (about three quarters of the rows; the first half of the tiles, short of a middle one as long as a later source's).
+    const int all = row_blocks(L, 0) * group, back = row_blocks(L, L / 2) * group;
+    const int kts = (L + kDkdvKeys - 1) / kDkdvKeys, early = a.cp_rank * ((L / 2 + kDkdvKeys - 1) / kDkdvKeys);
+    int own1 = 0;
+    while (own1 < kts && row_blocks(L, own1 * kDkdvKeys) * group > back) ++own1;
     ShareLoad w;
     w.top = blocks(longest) * group;
-    const float all = (float)(blocks(L) * group);
-    w.n = a.h_kv * nseq * (early + own1);
-    w.avg = all * (early + 0.75f * own1) / (early + own1);
-    w.top2 = (int)(0.5f * all);
-    w.n2 = a.h_kv * nseq * (late * kts + kts - own1);
-    w.avg2 = w.n2 ? all * (0.5f * late * kts + 0.25f * (kts - own1)) / (late * kts + kts - own1) : 0.f;
+    if (back < all) {
+      w.n = a.h_kv * nseq * (early + own1);
+      w.avg = all * (early + 0.75f * own1) / (early + own1);
+      w.top2 = back;
+      w.n2 = a.h_kv * nseq * (late * kts + kts - own1);
+      w.avg2 = w.n2 ? ((float)back * late * kts + 0.25f * all * (kts - own1)) / (late * kts + kts - own1) : 0.f;
+    } else {  // a single key tile of few rows: all alike
+      w.n = a.h_kv * nseq * (early + kts + late * kts);
+      w.avg = all;
+      w.top2 = w.n2 = 0;
+      w.avg2 = 0.f;
+    }
     w.us = wide ? 1.75f : 1.02f * a.d / 128.f;
     w.merge = wide ? 6.f : 5.f;
     w.read = wide ? 0.f : 1.25f * a.d / 128.f;

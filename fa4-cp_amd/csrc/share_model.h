@@ -31,6 +31,12 @@ struct Shares {
   int k = 1, k2 = 1, chunk = 1, top2 = 0, chunk2 = 1;
 };
 
+// Workgroups that share a tile of n steps: the plan's rule and the kernels'.
+constexpr int shares_of(int k, int chunk, int top2, int chunk2, int n) {
+  const int c = n > top2 ? chunk : chunk2, m = (n + c - 1) / c;
+  return m < 1 ? 1 : m > k ? k : m;
+}
+
 // The shares with the least estimated time, none unless they are 7 % faster (15 % for packed
 // sequences).  A workgroup costs its steps plus 11.5 us for its start and end.
 inline Shares best_shares(const ShareLoad& w, int most = kMaxShares) {

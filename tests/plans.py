@@ -24,6 +24,7 @@ extern "C" void split(const fa4cp_sweep_args* a, int* o) {
 }
 extern "C" int sweep_two(const fa4cp_sweep_args* a) { return sweep_two_per_cu(a); }
 extern "C" int attn_two(const fa4cp_attn_args* a) { return attn_two_per_cu(a); }
+extern "C" int shares(const int* s, int n) { return shares_of(s[0], s[2], s[3], s[4], n); }
 extern "C" void backward(const fa4cp_sweep_bwd_args* a, int* o) {
   const BwdPlan pl = bwd_plan(*a);
   put(pl.dq, o);
@@ -89,3 +90,8 @@ def backward_plan(lens, h, h_kv, d, cp, rank):
     out = (ctypes.c_int * 10)()
     _probe().backward(ctypes.byref(backward_args(lens, h, h_kv, d, cp, rank)), out)
     return Shares(*out[:5]), Shares(*out[5:])
+
+
+def shares_of(plan, n):
+    """Workgroups that share a tile of n steps under a Shares plan."""
+    return _probe().shares((ctypes.c_int * 5)(*plan), n)

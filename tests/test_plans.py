@@ -78,3 +78,28 @@ def test_two_per_cu_of_packed_sequences():
     assert plans.attn_two_per_cu([322] * 8, 32, 8, 64)
     # short row tiles: by the grid, empty workgroups and all
     assert plans.attn_two_per_cu([222] + [70] * 8, 32, 8, 64) and not plans.sweep_two_per_cu([222] + [70] * 8, 32, 8, 64)
+
+
+@pytest.mark.parametrize("h,h_kv,d,cp,rank", [(16, 2, 256, 4, 1), (8, 1, 256, 4, 0), (16, 2, 256, 4, 3), (8, 2, 256, 8, 5),
+                                              (8, 2, 128, 4, 1), (8, 1, 64, 8, 3), (2, 1, 128, 2, 0)])
+def test_key_tiles_take_their_classes_shares(h, h_kv, d, cp, rank):
+    """dk / dv: a tile walks the 32-row blocks that hold a row of its own, of every query head.  A
+    later source's tiles (the back-half rows, from the middle of a block on where half the length
+    is no multiple of 32) are the second class's longest, an earlier source's of the first."""
+    group, seen = h // h_kv, 0
+    for length in list(range(2, 900, 2)) + [1022, 1024, 1534, 2046, 2048, 3070, 3072, 4094, 4096]:
+        kv = plans.backward_plan([length], h, h_kv, d, cp, rank)[1]
+        if kv.k == 1:
+            continue
+
+        def blocks(first):
+            return group * len({row // 32 for row in range(first, length)})
+
+        late, early = blocks(length // 2), blocks(0)
+        own = [blocks(first) for first in range(0, length, 128)]
+        assert kv.top2 == (late if late < early and (rank < cp - 1 or min(own) <= late) else 0), length
+        if kv.top2:
+            seen += 1
+            assert plans.shares_of(kv, late) == min(kv.k, -(-kv.top2 // kv.chunk2)) <= kv.k2, length
+            assert plans.shares_of(kv, early) == min(kv.k, -(-early // kv.chunk)), length
+    assert seen
