@@ -413,8 +413,9 @@ __global__ __launch_bounds__(128 * HP) void bwd_dq_pair_kernel(BwdParams p) {
   int b = blockIdx.x;
   const int hg = b % n_hg;
   b /= n_hg;
-  const int share = SHARES ? b % p.ns : 0;
+  int share = SHARES ? b % p.ns : 0;
   if (SHARES) b /= p.ns;
+  if (SHARES && p.nseq > 1) share = turned_share(share, b, p.ns);
   const int tile = b * n_hg + hg;
   const int rt = p.n_tiles - 1 - b % p.n_tiles;  // longest first
   const int seq = b / p.n_tiles;
@@ -660,8 +661,9 @@ __global__ __launch_bounds__(512) void bwd_dq_pp_kernel(BwdParams p) {
   int b = blockIdx.x;
   const int hg = b % n_hg;
   b /= n_hg;
-  const int share = b % p.ns;
+  int share = b % p.ns;
   b /= p.ns;
+  if (p.nseq > 1) share = turned_share(share, b, p.ns);
   const int tile = b * n_hg + hg;
   const int rt = p.n_tiles - 1 - b % p.n_tiles;
   const int seq = b / p.n_tiles;

@@ -219,7 +219,7 @@ struct SplitWork {
     geo.po = sp.po + row * D;
     geo.pl = sp.pl + row;
     geo.done = sp.done + (int64_t)hg * sp.n_row + ri;
-    return geo.cut(sp, r - first, ns);
+    return geo.cut(sp, p.nseq > 1 ? turned_share(r - first, ri, ns) : r - first, ns);
   }
 };
 

@@ -25,6 +25,7 @@ extern "C" void split(const fa4cp_sweep_args* a, int* o) {
 extern "C" int sweep_two(const fa4cp_sweep_args* a) { return sweep_two_per_cu(a); }
 extern "C" int attn_two(const fa4cp_attn_args* a) { return attn_two_per_cu(a); }
 extern "C" int shares(const int* s, int n) { return shares_of(s[0], s[2], s[3], s[4], n); }
+extern "C" int turned(int i, int tile, int ns) { return turned_share(i, tile, ns); }
 extern "C" void backward(const fa4cp_sweep_bwd_args* a, int* o) {
   const BwdPlan pl = bwd_plan(*a);
   put(pl.dq, o);
@@ -95,3 +96,7 @@ def backward_plan(lens, h, h_kv, d, cp, rank):
 def shares_of(plan, n):
     """Workgroups that share a tile of n steps under a Shares plan."""
     return _probe().shares((ctypes.c_int * 5)(*plan), n)
+
+
+def turned_share(i, tile, ns):
+    return _probe().turned(i, tile, ns)

@@ -103,3 +103,16 @@ def test_key_tiles_take_their_classes_shares(h, h_kv, d, cp, rank):
             assert plans.shares_of(kv, late) == min(kv.k, -(-kv.top2 // kv.chunk2)) <= kv.k2, length
             assert plans.shares_of(kv, early) == min(kv.k, -(-early // kv.chunk)), length
     assert seen
+
+
+def test_turned_shares():
+    """Packed sequences: every tile's workgroups take its shares once each, and over the tiles share 0 comes
+    to each XCD and, within it, to each shader engine (workgroups in turn) about as often."""
+    for ns in range(2, 9):
+        for k in (1, 2, 4, 8):  # XCDs that a head group's workgroups go to in turn
+            seen = [0] * (4 * k)
+            for tile in range(128):
+                shares = [plans.turned_share(i, tile, ns) for i in range(ns)]
+                assert sorted(shares) == list(range(ns))
+                seen[(tile * ns + shares.index(0)) % (4 * k)] += 1
+            assert max(seen) <= 1.6 * 128 / (4 * k), (ns, k, seen)
