@@ -67,19 +67,30 @@ struct SplitPlan {
   bool split() const { return shares.k > 1; }
 };
 
+// The length whose tiles stand for those of packed sequences of `total` rows in all: the longer ones
+// hold more of the rows than their number says.
+inline int mixed_len(int total, int nseq, int longest) { return (std::max(1, total / nseq) + 2 * longest) / 3; }
+
+constexpr float kSlotUs = 0.035f;  // a slot of 128 KB written and read while the chip is full of workgroups
+
 // The plan for a sweep's shape (no pointer of `a` is followed).
 // The number of shares comes from best_shares' estimate: the row tiles that meet the later sources
 // (about `avg` key tiles each) before the others, 1.65 us a key tile (1 us at head dim 64), a merge
-// of 5 us plus 1.25 us per share and 128 columns.  It orders the measured times of 15 shapes
-// (one and four rings, D 64 / 128 / 256, 16 to 512 row tiles; GPU time, us):
+// of 5 us plus 1.25 us per share and 128 columns.  Some of the shapes it was set by (one and four rings, D 64 /
+// 128 / 256, 16 to 512 row tiles; GPU time, us):
 //   shares                                1     2     3     4     6     8
-//   2048 tokens, H 8/2, cp 4, rank 1     52    42    39    38    38    40   (chosen: 5)
+//   2048 tokens, H 8/2, cp 4, rank 1     52    42    39    38    38    40   (chosen: 6)
 //   8192, H 32/8, cp 8, rank 3          144    96    88   107   103   116   (3)
 //   16384, rank 3                       298   282   270   298   298   313   (3)
 //   16384, rank 7 (equal row tiles)     264   267   277   291   319   344   (1)
 //   24576, rank 3                       555   573   560   623   594   626   (1)
 //   8192, e4m3, rank 3                  113    80    69    85    84   100   (3)
 //   16384, H 16/2, D 256, rank 3        476   301   278   353   335   400   (3)
+// Packed sequences go by packed_shares.  By best_shares, with two classes of row tiles from an average
+// sequence, 27 of 210 drawn shapes at head dim 128 were more than 5 % slower than unsplit (30 sequences of 7708 rows, H
+// 8/1, e4m3, cp 4, rank 1: 74 us, in four 129).  Time by the unsplit one's, mean and worst of 90 shapes that either
+// splits, and with packed_shares and turned_share: head dim 128 0.89 (1.32), 0.84 (1.06); 64 0.76 (1.25), 0.76 (1.12);
+// 256 0.94 (1.48), 0.82 (1.09).
 // At head dim 256 a share costs more: the merging workgroup takes 8 us for each (its 256 KB come one load
 // at a time: beside the 128 registers of the output there is room for no more), and the launch 0.1 us for
 // each (256 KB written and read at the copy rate).  At 2.5 us and nothing, shapes were split that are
@@ -110,8 +121,8 @@ inline SplitPlan split_plan(const fa4cp_sweep_args* a) {
   auto cost = [&](int L, int rt, bool back) {
     return (std::min((rt + 1) * rows, L) - 1) / bn + 1 + a->cp_rank * tiles(L / 2) + (back ? late_steps * tiles(L) : 0);
   };
-  // the classes of row tiles, of a sequence of average length when packed
-  const int L = nseq > 1 ? std::max(1, a->total / nseq) : longest;
+  // the classes of row tiles, of one sequence for all when packed
+  const int L = nseq > 1 ? mixed_len(a->total, nseq, longest) : longest;
   const int rts = (L + rows - 1) / rows;
   const int fronts = late_steps > 0 ? (L / 2) / rows : 0;
   const int top = cost(longest, (int)n_rt - 1, true);
@@ -120,18 +131,25 @@ inline SplitPlan split_plan(const fa4cp_sweep_args* a) {
   ShareLoad w;
   w.top = top;
   w.avg = 0.5f * (cost(L, rts - 1, true) + cost(L, fronts, true));
-  w.n = n_hg * (rts - fronts) * nseq;
+  w.n = n_hg * (rts - fronts);
   w.top2 = front_top;
   w.avg2 = fronts ? 0.5f * (front_top + cost(L, 0, false)) : 0.f;
-  w.n2 = n_hg * fronts * nseq;
+  w.n2 = n_hg * fronts;
   w.us = a->d == 64 ? 1.f : 1.65f;
   const bool wide = a->d == 256;
   w.merge = 5.f;
   w.read = wide ? 8.f : 1.25f * a->d / 128.f;
-  w.slot = wide ? 0.1f : 0.f;
-  w.packed = nseq > 1;
+  w.slot = wide ? 0.1f : nseq > 1 && a->d == 128 ? kSlotUs : 0.f;
   w.free2 = false;
-  pl.shares = best_shares(w, std::min(kMaxShares, kMaxSlots / (int)(n_hg * n_row)));
+  const int most = std::min(kMaxShares, kMaxSlots / (int)(n_hg * n_row));
+  if (nseq > 1) {
+    w.avg = ((rts - fronts) * w.avg + fronts * w.avg2) / rts;
+    w.n = n_hg * (int)std::max<int64_t>(1, working_row_tiles(a->total, rows, nseq, n_rt));
+    if (a->d == 64) w.over = kOverUs64;
+    pl.shares = packed_shares(w, most);
+  } else {
+    pl.shares = best_shares(w, most);
+  }
   if (pl.shares.k == 1) return pl;
   pl.n_row = (int)n_row;
   pl.ns_back = pl.shares.k;
@@ -183,7 +201,7 @@ inline BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
   pl.dq_tiles = nseq * row_tiles * (a.h_q / hp);
   pl.kv_tiles = (int64_t)a.cp_size * a.h_kv * nseq * key_tiles;
   if (longest <= 0) return pl;
-  const int L = nseq > 1 ? std::max(1, a.total / nseq) : longest;  // an average sequence when packed
+  const int L = nseq > 1 ? mixed_len(a.total, nseq, longest) : longest;
   const int late = a.cp_size - 1 - a.cp_rank;
   auto blocks = [](int n) { return (n + kBwdRows - 1) / kBwdRows; };
   if (pl.dq_tiles <= kMaxTiles) {
@@ -194,16 +212,24 @@ inline BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
     ShareLoad w;
     w.top = cost(longest, (int)row_tiles - 1, true);
     w.avg = 0.5f * (cost(L, rts - 1, true) + cost(L, fronts, true));
-    w.n = (a.h_q / hp) * (rts - fronts) * nseq;
+    w.n = (a.h_q / hp) * (rts - fronts);
     w.top2 = fronts ? cost(L, fronts - 1, false) : 0;
     w.avg2 = fronts ? 0.5f * (w.top2 + cost(L, 0, false)) : 0.f;
-    w.n2 = (a.h_q / hp) * fronts * nseq;
+    w.n2 = (a.h_q / hp) * fronts;
     w.us = a.d == 256 ? 1.7f : 1.2f * a.d / 128.f;
     w.merge = 5.f;
     w.read = 1.25f * a.d / 128.f;
-    w.packed = nseq > 1;
     w.free2 = true;
-    pl.dq = best_shares(w, std::min<int64_t>(kMaxShares, kMaxSlots / pl.dq_tiles));
+    const int most = std::min<int64_t>(kMaxShares, kMaxSlots / pl.dq_tiles);
+    if (nseq > 1) {
+      w.avg = ((rts - fronts) * w.avg + fronts * w.avg2) / rts;
+      w.n = a.h_q / hp * (int)std::max<int64_t>(1, working_row_tiles(a.total, rows, nseq, row_tiles));
+      w.slot = a.d == 64 ? 0.f : kSlotUs;  // (128 KB at head dim 256 too)
+      if (a.d == 64) w.over = kOverUs64;
+      pl.dq = packed_shares(w, most);
+    } else {
+      pl.dq = best_shares(w, most);
+    }
   }
   const bool wide = a.d == 256;
   if (2 * pl.kv_tiles <= (wide ? 2 : 1) * kCus) {
@@ -217,13 +243,13 @@ inline BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
     ShareLoad w;
     w.top = blocks(longest) * group;
     if (back < all) {
-      w.n = a.h_kv * nseq * (early + own1);
+      w.n = a.h_kv * (early + own1);
       w.avg = all * (early + 0.75f * own1) / (early + own1);
       w.top2 = back;
-      w.n2 = a.h_kv * nseq * (late * kts + kts - own1);
+      w.n2 = a.h_kv * (late * kts + kts - own1);
       w.avg2 = w.n2 ? ((float)back * late * kts + 0.25f * all * (kts - own1)) / (late * kts + kts - own1) : 0.f;
     } else {  // a single key tile of few rows: all alike
-      w.n = a.h_kv * nseq * (early + kts + late * kts);
+      w.n = a.h_kv * (early + kts + late * kts);
       w.avg = all;
       w.top2 = w.n2 = 0;
       w.avg2 = 0.f;
@@ -232,9 +258,16 @@ inline BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
     w.merge = wide ? 6.f : 5.f;
     w.read = wide ? 0.f : 1.25f * a.d / 128.f;
     w.slot = wide ? 0.08f : 0.f;  // 256 KB each
-    w.packed = nseq > 1;
     w.free2 = true;
-    pl.kv = best_shares(w, std::min<int64_t>(kMaxShares, (wide ? 4 : 1) * kCus / pl.kv_tiles));
+    const int most = std::min<int64_t>(kMaxShares, (wide ? 4 : 1) * kCus / pl.kv_tiles);
+    if (nseq > 1) {
+      w.avg = (w.n * w.avg + w.n2 * w.avg2) / (w.n + w.n2);
+      w.n = std::max(1, (int)((float)a.total / L * (w.n + w.n2)));
+      if (a.d == 128) w.slot = kSlotUs;
+      pl.kv = packed_shares(w, most);
+    } else {
+      pl.kv = best_shares(w, most);
+    }
   }
   return pl;
 }

@@ -8,6 +8,8 @@ namespace fa4cp {
 
 constexpr int kCus = 256;     // workgroups the chip runs at a time (one per CU)
 constexpr int kMaxShares = 8;
+constexpr float kOverUs = 11.5f;  // start and end of a workgroup
+constexpr float kOverUs64 = 6.f;  // at head dim 64, beside another on the same CU
 
 // Two classes of tiles, the long ones handed out first.  Work is counted in steps (key tiles,
 // 32-row blocks) of `us` microseconds.
@@ -19,9 +21,9 @@ struct ShareLoad {
   float avg2;
   int n2;
   float us;           // microseconds per step
+  float over = kOverUs;  // for the start and end of a workgroup
   float merge, read;  // merging k shares takes merge + k read microseconds,
   float slot = 0.f;   // and `slot` more for every share of the launch (written out and read by another)
-  bool packed;        // tiles of several sequences, whose lengths only the device knows: the classes are guesses
   bool free2;         // the second class's shares are chosen apart (false: chunks as long as the first one's)
 };
 
@@ -37,19 +39,18 @@ constexpr int shares_of(int k, int chunk, int top2, int chunk2, int n) {
   return m < 1 ? 1 : m > k ? k : m;
 }
 
-// The shares with the least estimated time, none unless they are 7 % faster (15 % for packed
-// sequences).  A workgroup costs its steps plus 11.5 us for its start and end.
-inline Shares best_shares(const ShareLoad& w, int most = kMaxShares) {
-  const float over = 11.5f / w.us;
+// The shares with the least estimated time, none unless they are 7 % faster.  A workgroup costs its steps
+// plus `over`.
+inline Shares best_shares(const ShareLoad& w, int most) {
+  const float over = w.over / w.us;
   float one = 0.f, least = 0.f;
   Shares best;
   for (int k = 1; k <= most; ++k) {
     const int chunk = (w.top + k - 1) / k;
-    const int k1 = w.packed ? std::max(1, std::min(k, ((int)w.avg + chunk - 1) / chunk)) : k;
     const int tied = w.n2 ? std::max(1, std::min(k, (w.top2 + chunk - 1) / chunk)) : 1;
     for (int k2 = w.free2 ? 1 : tied; k2 <= (w.free2 && w.n2 ? k : tied); ++k2) {
-      const float c1 = w.avg / k1 + over, c2 = w.avg2 / k2 + over;
-      const int n1 = w.n * k1, n2 = w.n2 * k2;
+      const float c1 = w.avg / k + over, c2 = w.avg2 / k2 + over;
+      const int n1 = w.n * k, n2 = w.n2 * k2;
       const int q = n1 / kCus, r = n1 % kCus;
       const float longs = (q + (r > 0)) * c1;
       float t;
@@ -63,10 +64,10 @@ inline Shares best_shares(const ShareLoad& w, int most = kMaxShares) {
                          : std::max(longs, (n1 * c1 + n2 * c2) / kCus + 0.5f * c2);
       }
       t = std::max(t, (float)w.top / k + over);
-      // The forward's tiles of both classes cut up, in more workgroups than CUs: 10-20 % over the estimate
-      // (their parts go to memory while the next workgroups start).  13664 tokens (H 32/8, cp 8, rank 5):
-      // unshared 244 us, in halves 258; 16384: 287, 298; with a larger gain ahead, 12288: 200, in 3 and 2 181.
-      if (!w.free2 && !w.packed && k2 > 1 && n1 + n2 > kCus) t *= 1.2f;
+      // The forward's tiles of both classes cut up, in more workgroups than CUs: 10-20 % over the estimate.
+      // 13664 tokens (H 32/8, cp 8, rank 5): unshared 244 us, in halves 258; 16384: 287, 298; with a larger gain
+      // ahead, 12288: 200, in 3 and 2 181.
+      if (!w.free2 && k2 > 1 && n1 + n2 > kCus) t *= 1.2f;
       if (k > 1) t += (w.merge + w.read * k + w.slot * (n1 + n2)) / w.us;
       if (k == 1) one = least = t;
       else if (t < least) {
@@ -76,10 +77,38 @@ inline Shares best_shares(const ShareLoad& w, int most = kMaxShares) {
       }
     }
   }
-  if (least > (w.packed ? 0.85f : 0.93f) * one) return Shares{};
+  if (least > 0.93f * one) return Shares{};
   best.chunk = (w.top + best.k - 1) / best.k;
   best.top2 = w.free2 && w.n2 ? w.top2 : 0;
   best.chunk2 = std::max(1, (w.top2 + best.k2 - 1) / best.k2);
+  return best;
+}
+
+// The shares for the tiles of packed sequences, of one class: w.n tiles of w.avg steps on average and w.top
+// the longest.  Their lengths differ and every CU takes the next one as it comes free, so the launch
+// takes the chip's share of all steps and then about half a workgroup more, or one of the longest tile's.  (Above
+// 0.8 workgroups a CU: some shader engines run out of CUs before others.)  None
+// unless they are 7 % faster, nor where there are tiles enough to even out by themselves: 1.5 for a CU, 2 where
+// two share one (15648 rows in three, H 8/2, cp 8, rank 6, 490 row tiles: 1425 us, in four 1540).
+inline Shares packed_shares(const ShareLoad& w, int most) {
+  if (2 * w.n > (w.over < kOverUs ? 4 : 3) * kCus) return Shares{};
+  float one = 0.f, least = 0.f;
+  Shares best;
+  for (int k = 1; k <= most; ++k) {
+    best.chunk = (w.top + k - 1) / k;
+    const float k1 = k == 1 ? 1.f : std::max(1.f, std::min((float)k, w.avg / best.chunk + 0.5f));  // on average
+    const float wgs = w.n * k1, each = w.avg / k1 * w.us + w.over;
+    float t = wgs > 0.8f * kCus ? (w.n * w.avg * w.us + wgs * w.over) / kCus + 0.5f * each : each;
+    t = std::max(t, w.top * w.us / k + w.over);
+    if (k > 1) t += w.merge + w.read * k + w.slot * wgs;
+    if (k == 1) one = least = t;
+    else if (t < least) {
+      least = t;
+      best.k = k;
+    }
+  }
+  if (least > 0.93f * one) return Shares{};
+  best.chunk = (w.top + best.k - 1) / best.k;
   return best;
 }
 

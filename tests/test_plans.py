@@ -43,6 +43,22 @@ def test_wide_sweeps_are_not_split_at_a_loss(lens, h, h_kv, cp, rank, dtype, lea
     assert least <= plans.split_plan(lens, h, h_kv, 256, cp, rank, dtype).back <= most
 
 
+@pytest.mark.parametrize("lens,h,h_kv,cp,rank,dtype,least,most", [
+    # (as above; unsplit, and in the shares that an average sequence's two classes of row tiles gave, us)
+    ([216, 78, 252, 314, 82, 340, 166, 102, 924], 32, 8, 2, 0, BF16, 1, 1),  # 64, 80
+    ([1024, 4608, 662], 16, 16, 4, 2, E4M3, 1, 1),                           # 252, 304
+    ([360, 2034, 334], 32, 8, 2, 0, E4M3, 1, 1),                             # 84, 102
+    ([344, 414], 32, 8, 4, 2, BF16, 2, 3),                                   # 50, 60 (4; now 44)
+    ([308, 56, 40, 60, 24, 76, 82, 230, 104], 24, 8, 4, 3, FP16, 1, 1),      # 44, 55
+    ([8410, 4742, 2496], 8, 2, 8, 6, BF16, 1, 1),                            # 1425, 1540 (4)
+    ([706, 730], 16, 2, 2, 0, BF16, 1, 3),                                   # 48, 54 (4)
+    ([968, 598, 574], 8, 1, 8, 4, FP16, 3, 6),                               # 140, 75
+])
+def test_packed_sweeps_are_not_split_at_a_loss(lens, h, h_kv, cp, rank, dtype, least, most):
+    """Head dim 128: packed sequences' tiles of many lengths fill the chip unsplit, and slots cost bandwidth."""
+    assert least <= plans.split_plan(lens, h, h_kv, 128, cp, rank, dtype).back <= most
+
+
 @pytest.mark.parametrize("lens,h,h_kv", [
     ([350, 150, 124, 100, 100, 80, 60, 40, 20], 32, 8),  # 432 workgroups with the longest one's tiles for each
     ([2048] + [64] * 31, 8, 2),
