@@ -76,14 +76,16 @@ constexpr float kSlotUs = 0.035f;  // a slot of 128 KB written and read while th
 // The plan for a sweep's shape (no pointer of `a` is followed).
 // The number of shares comes from best_shares' estimate: the row tiles that meet the later sources
 // (about `avg` key tiles each) before the others, 1.65 us a key tile (1 us at head dim 64), a merge
-// of 5 us plus 1.25 us per share and 128 columns.  Some of the shapes it was set by (one and four rings, D 64 /
-// 128 / 256, 16 to 512 row tiles; GPU time, us):
+// of 5 us plus 1.25 us per share and 128 columns, and at head dim 128 kSlotUs for every share of the launch (at
+// 64, half the bytes and two workgroups on a CU, it hides).  Some of the shapes it was set by (one
+// and four rings, D 64 / 128 / 256, 16 to 512 row tiles; GPU time, us):
 //   shares                                1     2     3     4     6     8
 //   2048 tokens, H 8/2, cp 4, rank 1     52    42    39    38    38    40   (chosen: 6)
 //   8192, H 32/8, cp 8, rank 3          144    96    88   107   103   116   (3)
 //   16384, rank 3                       298   282   270   298   298   313   (3)
 //   16384, rank 7 (equal row tiles)     264   267   277   291   319   344   (1)
 //   24576, rank 3                       555   573   560   623   594   626   (1)
+//   8832, fp16, cp 2, rank 1            340   387                            (1)
 //   8192, e4m3, rank 3                  113    80    69    85    84   100   (3)
 //   16384, H 16/2, D 256, rank 3        476   301   278   353   335   400   (3)
 // Packed sequences go by packed_shares.  By best_shares, with two classes of row tiles from an average
@@ -91,7 +93,7 @@ constexpr float kSlotUs = 0.035f;  // a slot of 128 KB written and read while th
 // 8/1, e4m3, cp 4, rank 1: 74 us, in four 129).  Time by the unsplit one's, mean and worst of 90 shapes that either
 // splits, and with packed_shares and turned_share: head dim 128 0.89 (1.32), 0.84 (1.06); 64 0.76 (1.25), 0.76 (1.12);
 // 256 0.94 (1.48), 0.82 (1.09).
-// At head dim 256 a share costs more: the merging workgroup takes 8 us for each (its 256 KB come one load
+// At head dim 256 a share costs more: the merging workgroup takes 10 us and 8 for each (its 256 KB come one load
 // at a time: beside the 128 registers of the output there is room for no more), and the launch 0.1 us for
 // each (256 KB written and read at the copy rate).  At 2.5 us and nothing, shapes were split that are
 // faster whole or in fewer shares (us unsplit, in the shares chosen then, and now):
@@ -137,9 +139,9 @@ inline SplitPlan split_plan(const fa4cp_sweep_args* a) {
   w.n2 = n_hg * fronts;
   w.us = a->d == 64 ? 1.f : 1.65f;
   const bool wide = a->d == 256;
-  w.merge = 5.f;
+  w.merge = wide ? 10.f : 5.f;
   w.read = wide ? 8.f : 1.25f * a->d / 128.f;
-  w.slot = wide ? 0.1f : nseq > 1 && a->d == 128 ? kSlotUs : 0.f;
+  w.slot = wide ? 0.1f : a->d == 128 ? kSlotUs : 0.f;
   w.free2 = false;
   const int most = std::min(kMaxShares, kMaxSlots / (int)(n_hg * n_row));
   if (nseq > 1) {

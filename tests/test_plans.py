@@ -43,6 +43,18 @@ def test_wide_sweeps_are_not_split_at_a_loss(lens, h, h_kv, cp, rank, dtype, lea
     assert least <= plans.split_plan(lens, h, h_kv, 256, cp, rank, dtype).back <= most
 
 
+@pytest.mark.parametrize("lens,h,h_kv,d,least,most", [
+    ([4416], 32, 8, 128, 1, 1),   # 340 us, in halves 387
+    ([10440], 8, 2, 128, 1, 1),   # 425, 470
+    ([8824], 16, 2, 64, 1, 1),    # 383, 420
+    ([5360], 16, 16, 256, 1, 1),  # 453, 545
+    ([2054], 8, 2, 128, 2, 6),    # 77, in three 51
+])
+def test_sweeps_of_uneven_row_tiles_are_not_split_at_a_loss(lens, h, h_kv, d, least, most):
+    """Rank 1 of 2: one class of row tiles, the longest of three times the shortest's keys."""
+    assert least <= plans.split_plan(lens, h, h_kv, d, 2, 1, FP16).back <= most
+
+
 @pytest.mark.parametrize("lens,h,h_kv,cp,rank,dtype,least,most", [
     # (as above; unsplit, and in the shares that an average sequence's two classes of row tiles gave, us)
     ([216, 78, 252, 314, 82, 340, 166, 102, 924], 32, 8, 2, 0, BF16, 1, 1),  # 64, 80
