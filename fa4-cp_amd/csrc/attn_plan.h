@@ -69,8 +69,15 @@ struct SplitPlan {
 
 // The length whose tiles stand for those of packed sequences of `total` rows in all: the longer ones
 // hold more of the rows than their number says.
-inline int mixed_len(int total, int nseq, int longest) { return (std::max(1, total / nseq) + 2 * longest) / 3; }
+inline int mixed_len(int total, int nseq, int longest) {
+  return (int)((std::max(1, total / nseq) + 2 * (int64_t)longest) / 3);
+}
 
+// Slots of one launch: of a sweep 256 rows of float32 outputs and their LSEs each (129 KB at head dim 128, 257 at
+// 256: 514 MB at most), of the backward 128 KB (dq; 256 MB).  Half as many would take the gain from long
+// sweeps of few heads at head dim 256 (74752 tokens, H 8/2, cp 8, rank 7: 3242 us unsplit, in four 2554 with 299
+// MB; 143008 tokens: 9941, in three 8705 with 431).
+constexpr int kMaxSlots = 2048;
 constexpr float kSlotUs = 0.035f;  // a slot of 128 KB written and read while the chip is full of workgroups
 
 // The plan for a sweep's shape (no pointer of `a` is followed).
@@ -104,7 +111,7 @@ constexpr float kSlotUs = 0.035f;  // a slot of 128 KB written and read while th
 //   2368, H 8/2, bf16, cp 8, rank 5               85   98 (7)   77 (3)
 //   nine sequences, 7888, H 16/2, cp 8, rank 6    84  108 (6)   77 (2)
 inline SplitPlan split_plan(const fa4cp_sweep_args* a) {
-  constexpr int kMaxRowTiles = 1024, kMaxSlots = 2048;  // slots of 128 KB at head dim 128
+  constexpr int kMaxRowTiles = 1024;
   SplitPlan pl;
   const bool fp8 = a->dtype == FA4CP_E4M3;
   const int bn = fp8 ? (a->d == 256 ? 64 : 128) : (a->d == 256 ? 32 : 64);
@@ -143,7 +150,9 @@ inline SplitPlan split_plan(const fa4cp_sweep_args* a) {
   w.read = wide ? 8.f : 1.25f * a->d / 128.f;
   w.slot = wide ? 0.1f : a->d == 128 ? kSlotUs : 0.f;
   w.free2 = false;
-  const int most = std::min(kMaxShares, kMaxSlots / (int)(n_hg * n_row));
+  // (per_hg, the slots of a head group, is rounded up to 8)
+  int most = std::min(kMaxShares, kMaxSlots / (int)(n_hg * n_row));
+  while (most > 1 && n_hg * ((n_row * most + 7) / 8 * 8) > kMaxSlots) --most;
   if (nseq > 1) {
     w.avg = ((rts - fronts) * w.avg + fronts * w.avg2) / rts;
     w.n = n_hg * (int)std::max<int64_t>(1, working_row_tiles(a->total, rows, nseq, n_rt));
@@ -192,7 +201,7 @@ struct BwdPlan {
 // not beyond (32768 tokens, cp 4, 512 tiles 8450 and 8559).  There a share costs 0.08 us for its 256 KB (without
 // that, 3072 tokens, H 24/8, cp 8, rank 6, short tiles: unshared 266, shared 281).
 inline BwdPlan bwd_plan(const fa4cp_sweep_bwd_args& a) {
-  constexpr int kMaxTiles = 1024, kMaxSlots = 2048;  // slots of 128 KB at head dim 128
+  constexpr int kMaxTiles = 1024;
   BwdPlan pl;
   const int group = a.h_q / a.h_kv, nseq = a.cu ? a.nseq : 1;
   const int hp = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;

@@ -289,8 +289,9 @@ int fa4cp_ring_sweep_fwd_paged(const fa4cp_sweep_args* args, const fa4cp_sweep_k
  * partial result in the workspace, and the last of a row tile merges them.  The workspace's
  * first *clear_words 32-bit words (counters) must be zero when the sweep starts
  * (fa4cp_transpose_v_ring can clear them); they are zero again when it has ended, and nothing
- * else is kept across calls.  With a NULL workspace, and where 0 bytes are asked for, the call
- * is the unsplit sweep.
+ * else is kept across calls.  They are at most 2048 parts of 256 rows: 257 MiB at head dim 128, 514 MiB
+ * at 256.  With a NULL workspace, and where 0 bytes are asked for, the call is the unsplit
+ * sweep.
  */
 int fa4cp_ring_sweep_fwd_ws(const fa4cp_sweep_args* args, const fa4cp_sweep_kpages* k_pages, void* workspace,
                             int64_t workspace_bytes, void* stream);
@@ -351,7 +352,7 @@ int64_t fa4cp_ring_sweep_bwd_workspace_bytes(const fa4cp_sweep_bwd_args* args);
  * with a second workspace of fa4cp_ring_sweep_bwd_share_bytes(args) bytes, 16-byte aligned (NULL:
  * none): where the gradient kernels' tiles are too few to fill the chip, that is above 0 and
  * several workgroups share a tile, their float32 parts summed there in a fixed order.  It
- * holds nothing across calls.
+ * holds nothing across calls and is at most 257 MiB.
  */
 int fa4cp_ring_sweep_bwd_shared(const fa4cp_sweep_bwd_args* args, int32_t grad_dtype, void* shares,
                                 int64_t share_bytes, void* stream);

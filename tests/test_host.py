@@ -3,7 +3,9 @@ entry point, the ctypes struct mirror matches the C layout, and the Python inter
 the reference's argument checking and error behaviour."""
 
 import ctypes
+import math
 import os
+import random
 import re
 import subprocess
 import sys
@@ -312,6 +314,28 @@ def test_ring_sweep_workspace_contract():
     for ws, n in ((fake, need - 1), (fake + 8, need)):
         rc = lib.fa4cp_ring_sweep_fwd_ws(ctypes.byref(args()), None, ws, n, None)
         assert rc != 0 and b"workspace" in lib.fa4cp_last_error()
+
+
+def test_shared_workspaces_are_bounded():
+    """At most 2048 slots: 256 rows of float32 outputs and an LSE each for the sweep, 128 KB for
+    the backward (and, up to 16 KB, the counters)."""
+    lib, rng, most = _lib.load(), random.Random(0), {}
+    for _ in range(6000):
+        h_kv, group, d = rng.choice([1, 2, 3, 8, 16, 128, 144, 509]), rng.choice([1, 2, 4, 8, 16]), rng.choice([64, 128, 256])
+        cp, nseq = rng.choice([1, 2, 4, 8, 16]), rng.choice([1, 1, 3, 9, 30])
+        total = int(math.exp(rng.uniform(math.log(2), math.log(65536))))
+        fwd, bwd = _lib.SweepArgs(), _lib.SweepBwdArgs()
+        for a in (fwd, bwd):
+            a.h_q, a.h_kv, a.d, a.total, a.nseq = h_kv * group, h_kv, d, total, nseq
+            a.cp_size, a.cp_rank = cp, rng.choice([0, cp - 1, rng.randrange(cp)])
+            if nseq > 1:
+                a.cu, a.max_seqlen = 1 << 20, min(total, int(total / nseq * rng.uniform(1, 3)) + 1)
+            a.dtype = _lib.dtype_code(torch.bfloat16)
+        for what, n, slot in (("fwd", lib.fa4cp_ring_sweep_workspace_bytes(ctypes.byref(fwd), None), 1024 * (d + 1)),
+                              ("bwd", lib.fa4cp_ring_sweep_bwd_share_bytes(ctypes.byref(bwd)), 131072)):
+            assert 0 <= n <= 2048 * slot + 16384, (what, n, h_kv, group, d, cp, nseq, total)
+            most[what, d] = max(most.get((what, d), 0), n)
+    assert most["fwd", 256] > 300 << 20 and most["bwd", 256] > 128 << 20
 
 
 _CHECKED_CODE = """
