@@ -93,27 +93,31 @@ def test_autograd_gradients_are_the_rounded_ones():
     assert all(torch.equal(x, y.to(torch.bfloat16)) for x, y in zip(got, [dq, *dk, *dv]))
 
 
-@pytest.mark.parametrize("n,longest,h,h_kv,d,cp,rank", [
-    (126, None, 32, 32, 64, 16, 3),   # one key tile: no pair
-    (130, None, 32, 16, 128, 16, 5),  # one pair
-    (386, None, 16, 16, 128, 8, 0),   # no earlier source, the last tile partial
-    (640, None, 16, 8, 64, 8, 7),     # no later source, a tile without a partner
-    (386, 900, 16, 16, 64, 8, 4),     # tiles past the sequence's end
+@pytest.mark.parametrize("n,rows,h,h_kv,d,cp,rank", [
+    (126, 126, 32, 32, 64, 16, 3),   # one key tile: no pair
+    (130, 130, 32, 16, 128, 16, 5),  # one pair
+    (386, 386, 16, 16, 128, 8, 0),   # no earlier source, the last tile partial
+    (640, 640, 16, 8, 64, 8, 7),     # no later source, a tile without a partner
+    (386, 900, 16, 16, 64, 8, 4),    # a shorter sequence than the tensors hold: the second tiles past its end,
+    (130, 900, 16, 16, 128, 8, 4),   # and both
 ])
-def test_paired_key_tiles(n, longest, h, h_kv, d, cp, rank):
+def test_paired_key_tiles(n, rows, h, h_kv, d, cp, rank):
     """One sequence (its own key tiles taken in pairs) against the same one packed with an empty one (never
     in pairs): each tile sums the same terms in the same order, so the bits are equal."""
-    say(f"paired key tiles n={n} h={h}/{h_kv} d={d} cp={cp} rank={rank}")
+    say(f"paired key tiles n={n} rows={rows} h={h}/{h_kv} d={d} cp={cp} rank={rank}")
+    assert cp * h_kv * -(-rows // 128) > 256  # (else no tile is paired)
     g = torch.Generator(device="cuda").manual_seed(41)
-    mk = lambda hh: torch.randn(n, hh, d, generator=g, device=DEV).to(torch.bfloat16)  # noqa: E731
+    mk = lambda hh: torch.randn(rows, hh, d, generator=g, device=DEV).to(torch.bfloat16)  # noqa: E731
     q, dout = mk(h), mk(h)
     ring = LocalKVRing([mk(h_kv) for _ in range(cp)], [mk(h_kv) for _ in range(cp)])
     cfg = RingConfig(cp_size=cp, cp_rank=rank)
     lk, lv = ring.kv(rank)
-    out, lse = ring_flash_attn(q, lk, lv, cfg, group=ring, return_lse=True)
-    one = dict(cu_seqlens=torch.tensor([0, n], dtype=torch.int32, device=DEV), max_seqlen=longest) if longest else {}
+    out, lse = torch.zeros_like(q), torch.zeros(rows, h, device=DEV)
+    part = LocalKVRing([k[:n] for k in ring.k], [v[:n] for v in ring.v])
+    out[:n], lse[:n] = ring_flash_attn(q[:n], *part.kv(rank), cfg, group=part, return_lse=True)
+    one = dict(cu_seqlens=torch.tensor([0, n], dtype=torch.int32, device=DEV), max_seqlen=rows) if rows > n else {}
     two = dict(cu_seqlens=torch.tensor([0, n, n], dtype=torch.int32, device=DEV), max_seqlen=n)
     got = ring_flash_attn_backward(dout, q, lk, lv, out, lse, cfg, group=ring, **one)
     ref = ring_flash_attn_backward(dout, q, lk, lv, out, lse, cfg, group=ring, **two)
     for x, y in zip([*got[1], *got[2]], [*ref[1], *ref[2]]):
-        assert torch.equal(x, y)
+        assert torch.equal(x[:n], y[:n])
