@@ -5,9 +5,9 @@
 A step is one rank's full ring sweep over inputs already resident in HBM, at the bf16
 benchmark configuration: N = 131072 tokens, cp_size = 8 (local Q, K, V of 16384 tokens
 each), H_q = 32, H_kv = 8, D = 128, causal, rank 3 (all source ranks' KV shards in HBM).
-The default sweep transposes every source shard's V once (fa4cp_transpose_v) and runs one
-fused kernel over all cp_size sources (fa4cp_ring_sweep_fwd); both are inside the timed
-step.  The reference's per-step form (one attention launch plus one LSE merge per step) is
+The default sweep transposes every source shard's V as the rank reads it (fa4cp_transpose_v_ring)
+and runs one fused kernel over all cp_size sources (fa4cp_ring_sweep_fwd_ws); both are inside the
+timed step.  The reference's per-step form (one attention launch plus one LSE merge per step) is
 timed beside it as `per_step_bf16`.
 
 Prints one JSON line.  `value` is causal-adjusted attention TFLOP/s of the sweep:

@@ -22,9 +22,9 @@ constexpr int kPPWaves = 8;  // wavefronts of a ping-pong kernel's workgroup, 32
 
 // Workgroups per CU that the 16-bit pipeline's kernels are built for (their WGS).  At head dim 64 the
 // LDS tiles take 57 KB and the registers fit 128 without a spill, so two can run on a CU, one's loads,
-// softmax, start and end beside the other's MFMAs: 131072 tokens (H 32/8, cp 8, rank 3) 9180 -> 8460 us, 49152
-// (cp 4, rank 2) 2610 -> 2490, 24576 with 384 row tiles (cp 8, rank 5) 408 -> 383, 24 short sequences of 16
-// heads 57.6 -> 53.  With a CU for every workgroup that build is the slower one: two on one CU leave
+// softmax, start and end beside the other's MFMAs.  Sweeps (GPU time, the V^T launch with them): 131072 tokens (H
+// 32/8, cp 8, rank 3) 9000 -> 8325 us, 49152 (cp 4, rank 2) 2555 -> 2390, 24576 with 384 row tiles (cp 8, rank 5) 401
+// -> 370, 24 short sequences of 16 heads 58.4 -> 52.6.  With a CU for every workgroup that build is the slower one: two on one CU leave
 // another idle (256 row tiles, 8192 tokens, cp 4, rank 3: 105 -> 135 us), and kept apart they miss the
 // registers (110).
 inline bool two_per_cu(int d, int64_t workgroups) { return d == 64 && workgroups > 256; }

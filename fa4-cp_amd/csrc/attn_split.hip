@@ -6,9 +6,8 @@
 // front-half ones.  The split form hands a row tile's key tiles to up to ns_back / ns_front
 // workgroups (about `chunk` tiles each, equal shares); each writes its rows' normalised fp32
 // output and LSE to a slot of the workspace, and the last of a row tile's to finish merges its
-// slots.  Shares are cut at tile
-// granularity from the flattened segment list, alike for contiguous and paged K, so the two
-// stay bit-identical.
+// slots.  Shares are cut at tile granularity from the flattened segment list, alike for contiguous
+// and paged K, so the two stay bit-identical.  split_plan (attn_plan.h) says how many.
 #include "attn_kernels.h"
 #include "attn_split.h"
 

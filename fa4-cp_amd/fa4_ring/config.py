@@ -15,7 +15,8 @@ class RingConfig:
     cp_size / cp_rank: ring size and this rank's position.  causal must stay True (the
     zig-zag schedule is the causal one).  softmax_scale None means 1/sqrt(head_dim).
     deterministic is accepted for interface compatibility; every kernel here is
-    deterministic (fixed reduction order, no atomics)."""
+    deterministic: sums are taken in a fixed order (where several workgroups share a tile, an
+    atomic counter finds the last to finish, which adds all parts in order)."""
 
     cp_size: int
     cp_rank: int

@@ -302,10 +302,11 @@ def ring_sweep(local_q: torch.Tensor, local_k: torch.Tensor, local_v: torch.Tens
                group: "LocalKVRing", cu_seqlens: Optional[torch.Tensor] = None,
                max_seqlen: Optional[int] = None, out: Optional[torch.Tensor] = None,
                lse: Optional[torch.Tensor] = None, descales: Optional[Descales] = None) -> torch.Tensor:
-    """The whole sweep of ring_flash_attn (fa4_ring/ring_attention.py:61-174) in one
-    fa4cp_ring_sweep_fwd launch: every source's V is transposed (one fa4cp_transpose_v_many
-    launch), then one kernel carries each row tile's online softmax through the causal local keys, the front
-    halves of the earlier sources and, for the back-half rows, all keys of the later ones.
+    """The whole sweep of ring_flash_attn (fa4_ring/ring_attention.py:61-174) in two launches: every
+    source's V is transposed as this rank reads it (fa4cp_transpose_v_ring), then one kernel
+    (fa4cp_ring_sweep_fwd_ws) carries each row tile's online softmax through the causal local keys, the front
+    halves of the earlier sources and, for the back-half rows, all keys of the later ones; where few
+    row tiles leave the chip idle, several workgroups share one's keys.
     e4m3 inputs take ``descales`` (the k / v descales per source rank, as ring_flash_attn)
     and give a bf16 out.  Returns out [T, H, D] (``lse`` [T, H], if given, receives the
     natural-log LSE)."""
