@@ -23,11 +23,19 @@ constexpr int kPPWaves = 8;  // wavefronts of a ping-pong kernel's workgroup, 32
 // Workgroups per CU that the 16-bit pipeline's kernels are built for (their WGS).  At head dim 64 the
 // LDS tiles take 57 KB and the registers fit 128 without a spill, so two can run on a CU, one's loads,
 // softmax, start and end beside the other's MFMAs.  Sweeps (GPU time, the V^T launch with them): 131072 tokens (H
-// 32/8, cp 8, rank 3) 9000 -> 8325 us, 49152 (cp 4, rank 2) 2555 -> 2390, 24576 with 384 row tiles (cp 8, rank 5) 401
-// -> 370, 24 short sequences of 16 heads 58.4 -> 52.6.  With a CU for every workgroup that build is the slower one: two on one CU leave
-// another idle (256 row tiles, 8192 tokens, cp 4, rank 3: 105 -> 135 us), and kept apart they miss the
-// registers (110).
-inline bool two_per_cu(int d, int64_t workgroups) { return d == 64 && workgroups > 256; }
+// 32/8, cp 8, rank 3) 9000 -> 8325 us, 49152 (cp 4, rank 2) 2555 -> 2390, 24 short sequences of 16 heads 58.4 ->
+// 52.6.  Either of two on a CU takes 1.85 times as long, so there must be more than that:
+// * more than two for each CU: with fewer all start at once, the longest two to a CU while others fall idle (432 row
+//   tiles, H 24/8, 4504 rows, cp 8, rank 0: 800 us one per CU, 1170 two).  Two by one per CU, in the mean of drawn
+//   shapes of 257-512 row tiles and of more: one sequence 1.14 (34), 0.97 (62); packed 1.07 (20), 0.97 (51); per-step
+//   1.06 (20), 0.96 (25);
+// * in a sweep of fewer than four head groups, whose row tiles several XCDs share, four for each (512-1024 row
+//   tiles 1.03 (12; 27782 rows of H 8/1, cp 4, rank 2: 3650 and 4130 us), packed 1.10 (4), more 0.96 (3));
+// * more than one for each where all row tiles are short (few_rows) and their start and end count for more: 0.93 (63;
+//   H 144/144, cp 2, 296 rows, 288 row tiles: 52 and 45 us), with fewer 1.03 (12);
+// * or where the sweep is split, in workgroups of about equal length: 0.91-0.94 (39).
+inline bool two_per_cu(int d, int64_t workgroups, int most_alone) { return d == 64 && workgroups > most_alone; }
+inline bool few_rows(int64_t longest, int rows) { return longest <= std::min(4 * rows, 512); }
 
 // Row tiles of `rows` rows, at most n_rt in a sequence, that nseq sequences of `total` rows in all make.
 // Only the device knows the lengths of packed ones: about half a tile per sequence more than
@@ -40,24 +48,27 @@ inline int64_t working_row_tiles(int64_t total, int rows, int nseq, int64_t n_rt
 // The build of the unsplit sweep, whose workgroups without rows come last.
 inline bool sweep_two_per_cu(const fa4cp_sweep_args* a) {
   const int hp = heads_per_wg(a->h_q / a->h_kv), rows = 32 * kPPWaves / hp;
-  const int n_rt = ((a->cu ? a->max_seqlen : a->total) + rows - 1) / rows;
-  return two_per_cu(a->d, a->h_q / hp * working_row_tiles(a->total, rows, a->cu ? a->nseq : 1, n_rt));
+  const int longest = a->cu ? a->max_seqlen : a->total;
+  const int64_t n_rt = ((int64_t)longest + rows - 1) / rows;
+  const int n_hg = a->h_q / hp;
+  return two_per_cu(a->d, n_hg * working_row_tiles(a->total, rows, a->cu ? a->nseq : 1, n_rt),
+                    few_rows(longest, rows) ? kCus : n_hg < 4 ? 4 * kCus : 2 * kCus);
 }
 
 // The build of the V^T kernel for one attention call.  Its workgroups without rows stand among the others
-// and hold up their start: where all row tiles are short, that counts for more than a CU for each
-// with rows.  Attention of two steps, the grid above 256 workgroups, those with rows below: with five row tiles or more in
-// the longest sequence, or over 512 rows, the one-per-CU build takes 0.95 of the other's time in the mean of 42
-// shapes (0.81-1.09; the nine sequences above 47.4 -> 43.1 us, 7596 rows in three, H 8/1, 147 -> 130), below that
-// 1.07 in the mean of 18 (nine of 784 rows, H 32/8, 38 and 44 us).
+// and hold up their start: where all row tiles are short the grid counts (attention of two steps, the grid above
+// 256 workgroups, those with rows below: two per CU 0.93 of the time in the mean of 18 shapes; nine sequences of 784
+// rows, H 32/8, 44 and 38 us), elsewhere the workgroups with rows (1.05 in the mean of 42; the nine sequences above
+// 43.1 and 47.4 us, 7652 rows in three, H 8/1, 130 and 147).
 inline bool attn_two_per_cu(const fa4cp_attn_args* a) {
   const int hp = heads_per_wg(a->h_q / a->h_kv), rows = 32 * kPPWaves / hp, nseq = a->cu_q ? a->nseq : 1;
   const bool all = a->q_sel == FA4CP_SEL_ALL;
   auto selected = [&](int n) { return all ? n : (n + 1) / 2; };
   const int longest = selected(a->cu_q ? a->max_seqlen_q : a->total_q);
-  const int64_t n_rt = (longest + rows - 1) / rows;
-  const bool by_rows = n_rt >= 5 || longest > 512;
-  return two_per_cu(a->d, a->h_q / hp * (by_rows ? working_row_tiles(selected(a->total_q), rows, nseq, n_rt) : nseq * n_rt));
+  const int64_t n_rt = ((int64_t)longest + rows - 1) / rows;
+  const bool few = few_rows(longest, rows);
+  const int64_t tiles = few ? nseq * n_rt : working_row_tiles(selected(a->total_q), rows, nseq, n_rt);
+  return two_per_cu(a->d, a->h_q / hp * tiles, few ? kCus : 2 * kCus);
 }
 
 // How a sweep is split (see SweepSplit in attn_split.hip).

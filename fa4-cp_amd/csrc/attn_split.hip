@@ -287,7 +287,7 @@ int launch_split(const SweepParams& p, const SplitPlan& pl, void* ws, int dtype,
   sp.per_hg = pl.per_hg;
   void (*fn)(SweepSplit) = nullptr;
   const int64_t slots = (int64_t)p.n_hg * ((pl.n_row - pl.n_front) * pl.ns_back + pl.n_front * pl.ns_front);
-  const bool two = two_per_cu(d, slots);
+  const bool two = two_per_cu(d, slots, kCus);
 #define FA4CP_PICK_HP(KERNEL, ...)                                                          \
   {                                                                                         \
     if (hp == 4) fn = paged ? KERNEL<__VA_ARGS__, 4, true> : KERNEL<__VA_ARGS__, 4, false>; \

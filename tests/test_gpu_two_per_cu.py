@@ -1,5 +1,5 @@
-"""Head dim 64 launches of more workgroups than the chip has CUs run two on a CU, in kernels built
-for half the registers.
+"""Head dim 64 launches of many workgroups (more than the chip has CUs, or two for each) run two on a CU, in
+kernels built for half the registers.
 
 Every case has enough heads for them; a slice of its heads alone has not, and goes to the kernels that
 the other tests hold against the oracle.  Both forms round the same probabilities and outputs, each off by
@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 CASES = [  # (local lens, H, H_kv, cp, rank, dtype, page, heads alone): row tiles of 256 / (heads per workgroup) rows
     ([386], 144, 144, 2, 0, torch.bfloat16, 0, 8),             # 2 x 144: a partial row tile
     ([258], 130, 130, 3, 2, torch.float16, 128, 26),           # 260
-    ([1026], 96, 48, 2, 1, torch.bfloat16, 0, 16),             # two heads per workgroup: 9 x 48
+    ([1026], 96, 48, 2, 1, torch.bfloat16, 0, 16),             # two heads per workgroup: 9 x 48, one per CU
+    ([1026], 128, 64, 2, 1, torch.bfloat16, 0, 16),            # 9 x 64
     ([2048], 32, 8, 8, 3, torch.bfloat16, 0, 4),               # four; 256 row tiles whose keys are shared
     ([2048], 32, 8, 8, 3, torch.float16, 256, 4),
     ([640, 2, 0, 322, 126, 514], 128, 32, 4, 1, torch.bfloat16, 0, 16),  # packed: empty and short sequences

@@ -77,35 +77,45 @@ def test_packed_sweeps_are_not_split_at_a_loss(lens, h, h_kv, cp, rank, dtype, l
     ([256] * 8, 32, 8),                                  # whole tiles: 256 workgroups, none to spare
     ([322] * 8, 32, 8),
     ([1024] * 8, 32, 8),
+    ([4098], 32, 8),
+    ([4096], 32, 8),                                     # 512
     ([2050], 32, 8),
-    ([2048], 32, 8),
+    ([27782], 8, 1),                                     # two head groups: 870, a sweep needs four for each CU
+    ([34000], 8, 1),
     ([1300] * 12, 16, 16),
     ([600] * 9, 6, 3),
+    ([386], 144, 144),                                   # short row tiles: from 256 on
+    ([250], 144, 144),
 ])
 @pytest.mark.parametrize("q_sel", [0, 1])
 def test_two_per_cu_counts_the_workgroups_with_rows(lens, h, h_kv, q_sel):
-    """Two workgroups per CU (head dim 64) only where more than 256 have rows; half a tile per sequence
-    off at most, as the host doesn't know the lengths."""
+    """Two workgroups per CU (head dim 64) only where more than two for each have rows (four in a sweep of few
+    head groups), or one where all row tiles are short (then, per step, those of the grid); half a tile per sequence off at
+    most, as the host doesn't know the lengths."""
     hp = plans.heads_per_wg(h // h_kv)
-
-    def workgroups(ns):
-        return h // hp * sum(-(-n * hp // 256) for n in ns)
-
-    slack = h // hp * len(lens) // 2 if len(lens) > 1 else 0
-    for two, ns in ((plans.attn_two_per_cu(lens, h, h_kv, 64, q_sel), [n if q_sel == 0 else n // 2 for n in lens]),
-                    (plans.sweep_two_per_cu(lens, h, h_kv, 64), lens)):
-        n = workgroups(ns)
-        assert two == (n > 256) or abs(n - 256) <= slack, (two, n)
+    tiles = lambda n: -(-n * hp // 256)  # noqa: E731
+    for step, two, ns in ((True, plans.attn_two_per_cu(lens, h, h_kv, 64, q_sel), [n if q_sel == 0 else n // 2 for n in lens]),
+                          (False, plans.sweep_two_per_cu(lens, h, h_kv, 64), lens)):
+        few = max(ns) <= 512 and tiles(max(ns)) <= 4
+        n = h // hp * (len(ns) * tiles(max(ns)) if step and few else sum(map(tiles, ns)))
+        slack = h // hp * len(lens) // 2 if len(lens) > 1 and not (step and few) else 0
+        most = 256 if few else 512 if step or h // hp >= 4 else 1024
+        assert two == (n > most) or abs(n - most) <= slack, (two, n)
     assert not plans.attn_two_per_cu(lens, h, h_kv, 128, q_sel)
 
 
-def test_two_per_cu_of_packed_sequences():
-    nine = [350, 150, 124, 100, 100, 80, 60, 40, 20]
-    assert not plans.attn_two_per_cu(nine, 32, 8, 64) and not plans.sweep_two_per_cu(nine, 32, 8, 64)
-    assert not plans.attn_two_per_cu([256] * 8, 32, 8, 64) and not plans.sweep_two_per_cu([256] * 8, 32, 8, 64)
-    assert plans.attn_two_per_cu([322] * 8, 32, 8, 64)
-    # short row tiles: by the grid, empty workgroups and all
-    assert plans.attn_two_per_cu([222] + [70] * 8, 32, 8, 64) and not plans.sweep_two_per_cu([222] + [70] * 8, 32, 8, 64)
+def test_two_per_cu_where_measured():
+    step, sweep = plans.attn_two_per_cu, plans.sweep_two_per_cu
+    nine, short = [350, 150, 124, 100, 100, 80, 60, 40, 20], [222] + [70] * 8
+    assert not step(nine, 32, 8, 64) and not sweep(nine, 32, 8, 64)
+    assert not step([256] * 8, 32, 8, 64) and not sweep([256] * 8, 32, 8, 64)
+    assert step(short, 32, 8, 64) and not sweep(short, 32, 8, 64)  # the grid, empty workgroups and all
+    assert sweep([296], 144, 144, 64) and step([296], 144, 144, 64)
+    # all at once on two per CU the longest tiles share CUs while others fall idle (800 us, 1170; 730, 930)
+    for lens, h, h_kv in (([4504], 24, 8), ([16208], 8, 2), ([7096], 16, 2)):
+        assert not sweep(lens, h, h_kv, 64) and not step(lens, h, h_kv, 64)
+    assert not sweep([27782], 8, 1, 64) and step([27782], 8, 1, 64)
+    assert sweep([16384], 32, 8, 64) and step([16384], 32, 8, 64)
 
 
 @pytest.mark.parametrize("h,h_kv,d,cp,rank", [(16, 2, 256, 4, 1), (8, 1, 256, 4, 0), (16, 2, 256, 4, 3), (8, 2, 256, 8, 5),
