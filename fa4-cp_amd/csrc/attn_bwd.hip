@@ -130,6 +130,12 @@ constexpr int kAgent = 16;
 // The share of a tile's n blocks that workgroup i of the launch's ns takes: [lo, hi), of `shares`;
 // false: the tile has fewer shares.
 __device__ __forceinline__ bool take_share(const BwdParams& p, int i, int n, int& lo, int& hi, int& shares) {
+  if (p.ns == 1) {  // (an integer division takes 0.2 us)
+    shares = 1;
+    lo = 0;
+    hi = n;
+    return true;
+  }
   shares = shares_of(p.ns, p.chunk, p.top2, p.chunk2, n);
   lo = n * i / shares;
   hi = n * (i + 1) / shares;
@@ -661,9 +667,12 @@ __global__ __launch_bounds__(512) void bwd_dq_pp_kernel(BwdParams p) {
   int b = blockIdx.x;
   const int hg = b % n_hg;
   b /= n_hg;
-  int share = b % p.ns;
-  b /= p.ns;
-  if (p.nseq > 1) share = turned_share(share, b, p.ns);
+  int share = 0;
+  if (p.ns > 1) {
+    share = b % p.ns;
+    b /= p.ns;
+    if (p.nseq > 1) share = turned_share(share, b, p.ns);
+  }
   const int tile = b * n_hg + hg;
   const int rt = p.n_tiles - 1 - b % p.n_tiles;
   const int seq = b / p.n_tiles;
@@ -921,8 +930,11 @@ __device__ __forceinline__ void dkdv_tile(const BwdParams& p, int b, int ns, int
     }
   }
   const int k = c == 0 ? front : c == 1 ? own : c == 2 ? p.n_tiles : c == 3 ? p.n_tiles - own : p.n_tiles - front;
-  share = b / n;
-  b -= share * n;
+  share = 0;
+  if (ns > 1) {
+    share = b / n;
+    b -= share * n;
+  }
   tile = at + b;
   int r;
   if (c == 1 || c == 3) {
@@ -930,14 +942,15 @@ __device__ __forceinline__ void dkdv_tile(const BwdParams& p, int b, int ns, int
     kt = b / per_kt;
     r = b - kt * per_kt;
   } else {
-    const int s = b / (k * per_kt);
-    b -= s * k * per_kt;
-    r = b / k;
+    const int m = k * per_kt;
+    int s = 0;
+    for (; b >= m && s < p.S; b -= m) ++s;
+    r = k > 1 ? b / k : b;
     kt = b - r * k;
     src = c == 2 ? p.rank + 1 + s : s;
   }
   kt += c == 3 ? own : c == 4 ? front : 0;
-  kvh = r / p.nseq;
+  kvh = p.nseq > 1 ? r / p.nseq : r;
   seq = r - kvh * p.nseq;
 }
 
@@ -1070,7 +1083,9 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
       struct Cursor {
         int lh, lr;
       };
-      Cursor rc{lo / n_rb, lo % n_rb}, tc = rc;
+      Cursor rc{0, 0};
+      if (lo > 0) rc = {lo / n_rb, lo % n_rb};
+      Cursor tc = rc;
       // head dim 256: the half of the block at cursor cu made of regions r0 and r0 + 2 into
       // half-stage st, then the per-row values
       auto load = [&](Cursor& cu, char* st, int r0) {
@@ -1105,7 +1120,7 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
         constexpr bool PW = decltype(role)::value;
         frag pb0, pb1;  // first wavefront: P of the previous block (operands of dV)
         f32x16 dpt;     // second wavefront: dP of the previous block
-        int cr = lo % n_rb;  // row block (within the head) of block i
+        int cr = rc.lr;  // row block (within the head) of block i
         load(rc, rows_of(0), 0);
         __builtin_amdgcn_s_waitcnt(kWaitAll);
         wg_barrier();
@@ -1214,9 +1229,9 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
         // the next block to load (wave-uniform, advanced block by block: the blocks of one query
         // head are consecutive, the next head's start n_pb blocks after the previous one's)
         const char* gnext = reinterpret_cast<const char*>(
-            uniform_ptr(p.pk + ((int64_t)(kvh * p.group + lo / n_rb) * p.n_pb + blk0 + lo % n_rb) * BB));
+            uniform_ptr(p.pk + ((int64_t)(kvh * p.group + rc.lh) * p.n_pb + blk0 + rc.lr) * BB));
         const int64_t head_jump = (int64_t)(p.n_pb - n_rb) * BB;
-        int lr = lo % n_rb;
+        int lr = rc.lr;
         auto load_block = [&](char* st) __attribute__((always_inline)) {
           const __amdgpu_buffer_rsrc_t rs = make_rsrc32(gnext, BB);
           gnext += BB;
@@ -1244,7 +1259,7 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
         constexpr bool PW = decltype(role)::value;
         frag pb0, pb1;  // first wavefront: P of the previous block (operands of dV)
         f32x16 dpt;     // second wavefront: dP of the previous block
-        int cr = lo % n_rb;  // row block (within the head) of block i
+        int cr = rc.lr;  // row block (within the head) of block i
         wg_barrier();
         for (int i = 0; i <= n_blk; ++i) {
           const char* cur = stage_of(i);       // block i: its row regions
