@@ -122,6 +122,19 @@ def test_quantize_many_equals_single_calls(dtype):
             assert ds.shape == ds1.shape
 
 
+def test_quantize_many_by_bytes(monkeypatch):
+    """More bytes than one call takes: several calls, the same bytes and descales."""
+    from fa4_ring import fp8
+
+    say("quantize_e4m3_many by bytes")
+    xs = [_heads_scaled(r, 2, 128, torch.bfloat16, seed=r).to(DEV) for r in (40, 1, 64, 0, 200, 8, 7)]
+    whole = fp8.quantize_e4m3_many(xs, heads_per_scale=[0, 1] * 3 + [1])
+    monkeypatch.setattr(fp8, "QUANT_MAX_BYTES", 512 * 64)  # 64 rows
+    assert fp8._quant_calls(xs) == [range(0, 2), range(2, 4), range(4, 5), range(5, 7)]
+    for (y, ds), (y1, ds1) in zip(fp8.quantize_e4m3_many(xs, heads_per_scale=[0, 1] * 3 + [1]), whole):
+        assert torch.equal(y.view(torch.uint8), y1.view(torch.uint8)) and torch.equal(ds, ds1)
+
+
 def test_quantize_zero_and_empty():
     say("quantize_e4m3 all-zero and empty")
     y, ds = quantize_e4m3(torch.zeros(64, 2, 128, dtype=torch.bfloat16, device=DEV), heads_per_scale=1)

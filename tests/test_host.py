@@ -338,6 +338,21 @@ def test_shared_workspaces_are_bounded():
     assert most["fwd", 256] > 300 << 20 and most["bwd", 256] > 128 << 20
 
 
+def test_quantiser_calls_cover_the_tensors():
+    """Calls of quantize_e4m3_many: every tensor once and in order, at most 33 and 384 MiB of input, a larger
+    tensor by itself."""
+    from fa4_ring.fp8 import _quant_calls
+
+    def calls(*mib):
+        return [list(c) for c in _quant_calls([torch.empty(m << 12, 1, 128, dtype=torch.bfloat16, device="meta") for m in mib])]
+
+    assert calls(64, *[16] * 16) == [list(range(17))]
+    assert calls(503, 252, 252, 252, 252) == [[0], [1], [2], [3], [4]]
+    assert calls(192, 192, 1, 0, 500, 3) == [[0, 1], [2, 3], [4], [5]]
+    assert calls(*[1] * 70) == [list(range(33)), list(range(33, 66)), list(range(66, 70))]
+    assert calls(0) == [[0]]
+
+
 _CHECKED_CODE = """
 import sys, torch
 sys.path.insert(0, sys.argv[1])
