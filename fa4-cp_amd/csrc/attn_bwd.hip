@@ -128,9 +128,12 @@ struct BwdParams {
 constexpr int kAgent = 16;
 
 // The share of a tile's n blocks that workgroup i of the launch's ns takes: [lo, hi), of `shares`;
-// false: the tile has fewer shares.
+// false: the tile has fewer shares.  LONG false: for launches of many short tiles; the divisions of about 0.2 us
+// each are left out where nothing is shared (30 sequences of 270 rows in all, H 16/16, D 64, cp 4: dk / dv 38.9 -> 34.0
+// us).  The branch costs dq and the paired dk / dv 0.3-0.6 % (headline backward 53.06 -> 53.39 ms).
+template <bool LONG = true>
 __device__ __forceinline__ bool take_share(const BwdParams& p, int i, int n, int& lo, int& hi, int& shares) {
-  if (p.ns == 1) {  // (an integer division takes 0.2 us)
+  if (!LONG && p.ns == 1) {
     shares = 1;
     lo = 0;
     hi = n;
@@ -667,12 +670,9 @@ __global__ __launch_bounds__(512) void bwd_dq_pp_kernel(BwdParams p) {
   int b = blockIdx.x;
   const int hg = b % n_hg;
   b /= n_hg;
-  int share = 0;
-  if (p.ns > 1) {
-    share = b % p.ns;
-    b /= p.ns;
-    if (p.nseq > 1) share = turned_share(share, b, p.ns);
-  }
+  int share = b % p.ns;
+  b /= p.ns;
+  if (p.nseq > 1) share = turned_share(share, b, p.ns);
   const int tile = b * n_hg + hg;
   const int rt = p.n_tiles - 1 - b % p.n_tiles;
   const int seq = b / p.n_tiles;
@@ -931,7 +931,7 @@ __device__ __forceinline__ void dkdv_tile(const BwdParams& p, int b, int ns, int
   }
   const int k = c == 0 ? front : c == 1 ? own : c == 2 ? p.n_tiles : c == 3 ? p.n_tiles - own : p.n_tiles - front;
   share = 0;
-  if (ns > 1) {
+  if (PAIR || ns > 1) {
     share = b / n;
     b -= share * n;
   }
@@ -944,13 +944,18 @@ __device__ __forceinline__ void dkdv_tile(const BwdParams& p, int b, int ns, int
   } else {
     const int m = k * per_kt;
     int s = 0;
-    for (; b >= m && s < p.S; b -= m) ++s;
-    r = k > 1 ? b / k : b;
+    if (PAIR) {
+      s = b / m;
+      b -= s * m;
+    } else {
+      for (; b >= m && s < p.S; b -= m) ++s;
+    }
+    r = PAIR || k > 1 ? b / k : b;
     kt = b - r * k;
     src = c == 2 ? p.rank + 1 + s : s;
   }
   kt += c == 3 ? own : c == 4 ? front : 0;
-  kvh = p.nseq > 1 ? r / p.nseq : r;
+  kvh = PAIR || p.nseq > 1 ? r / p.nseq : r;
   seq = r - kvh * p.nseq;
 }
 
@@ -1072,7 +1077,7 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
       // (query head, 32-row block) pairs, head-major: this workgroup's share of them, from `lo` on
       int lo, hi;
       if (kShares) {
-        if (!take_share(p, share, n_rb * p.group, lo, hi, shares)) continue;
+        if (!take_share<PAIR>(p, share, n_rb * p.group, lo, hi, shares)) continue;
       } else {
         lo = 0;
         hi = n_rb * p.group;
@@ -1084,7 +1089,7 @@ __global__ __launch_bounds__(D > 128 ? 512 : 576) void bwd_dkdv_kernel(BwdParams
         int lh, lr;
       };
       Cursor rc{0, 0};
-      if (lo > 0) rc = {lo / n_rb, lo % n_rb};
+      if (PAIR || lo > 0) rc = {lo / n_rb, lo % n_rb};
       Cursor tc = rc;
       // head dim 256: the half of the block at cursor cu made of regions r0 and r0 + 2 into
       // half-stage st, then the per-row values
